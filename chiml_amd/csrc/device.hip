@@ -29,6 +29,7 @@
 // src/PML/parallelPML.hpp:693-765 and src/PML/parallelPML.cpp:12-40.
 #include <hip/hip_runtime.h>
 
+#include "grid_layout.hpp"
 #include "qe_layout.hpp"
 
 #include <algorithm>
@@ -106,8 +107,10 @@ struct StepArgs {
     T* F[6];  // Ex, Ey, Ez, Hx, Hy, Hz
     const T* G[6];  // fused step: the fields before the step (ping-pong); F itself elsewhere
     int nx, ny, nz;
+    int px;  // cells per stored x row: nx, or nx rounded up to whole W-cell groups (the added cells stay zero)
     T inv_d[3];
     int Tp[3];
+    int fma_curl;  // 2D sweeps: curl_of's FMA form
     const uint8_t* mat_e[3];
     const T* ce[3];
     const T* inveps[3];
@@ -199,10 +202,10 @@ __device__ __forceinline__ void update_h_cells(const StepArgs<T>& a) {
     const int x = blockIdx.x * blockDim.x + threadIdx.x;
     const int y = blockIdx.y * blockDim.y + threadIdx.y;
     const int z = blockIdx.z;
-    const int nx = a.nx, ny = a.ny, nz = a.nz;
+    const int nx = a.nx, ny = a.ny, nz = a.nz, px = a.px;
     if (x >= nx || y >= ny) return;
-    const long long i = lidx(x, y, z, nx, ny);
-    const long long sy = nx, sz = static_cast<long long>(nx) * ny;
+    const long long i = lidx(x, y, z, px, ny);
+    const long long sy = px, sz = static_cast<long long>(px) * ny;
     const bool inpml = (x < a.Tp[0]) || (x >= nx - a.Tp[0]) || (y < a.Tp[1]) || (y >= ny - a.Tp[1]) ||
                        (DIM == 3 && ((z < a.Tp[2]) || (z >= nz - a.Tp[2])));
     int step = 0;
@@ -218,10 +221,10 @@ __device__ __forceinline__ void update_h_cells(const StepArgs<T>& a) {
         if (DIM == 3) {
             T dEy = Ey[i + sz] - Ey[i];
             if (!inpml) acc = dEy * a.inv_d[2] - dEz * a.inv_d[1];
-            else acc = pml_term(a.pml[3], 2, z, x, y, z, nx, ny, dEy, dEy * a.inv_d[2]) - pml_term(a.pml[3], 1, y, x, y, z, nx, ny, dEz, dEz * a.inv_d[1]);
+            else acc = pml_term(a.pml[3], 2, z, x, y, z, px, ny, dEy, dEy * a.inv_d[2]) - pml_term(a.pml[3], 1, y, x, y, z, px, ny, dEz, dEz * a.inv_d[1]);
         } else {
             if (!inpml) acc = -(dEz * a.inv_d[1]);
-            else acc = -pml_term(a.pml[3], 1, y, x, y, z, nx, ny, dEz, dEz * a.inv_d[1]);
+            else acc = -pml_term(a.pml[3], 1, y, x, y, z, px, ny, dEz, dEz * a.inv_d[1]);
         }
         T ch = HMAP ? a.ch[0][a.mat_h[0][i]] : a.ch[0][0];
         T h = a.F[3][i] + ch * acc;
@@ -235,10 +238,10 @@ __device__ __forceinline__ void update_h_cells(const StepArgs<T>& a) {
         if (DIM == 3) {
             T dEx = Ex[i + sz] - Ex[i];
             if (!inpml) acc = dEz * a.inv_d[0] - dEx * a.inv_d[2];
-            else acc = pml_term(a.pml[4], 0, x, x, y, z, nx, ny, dEz, dEz * a.inv_d[0]) - pml_term(a.pml[4], 2, z, x, y, z, nx, ny, dEx, dEx * a.inv_d[2]);
+            else acc = pml_term(a.pml[4], 0, x, x, y, z, px, ny, dEz, dEz * a.inv_d[0]) - pml_term(a.pml[4], 2, z, x, y, z, px, ny, dEx, dEx * a.inv_d[2]);
         } else {
             if (!inpml) acc = dEz * a.inv_d[0];
-            else acc = pml_term(a.pml[4], 0, x, x, y, z, nx, ny, dEz, dEz * a.inv_d[0]);
+            else acc = pml_term(a.pml[4], 0, x, x, y, z, px, ny, dEz, dEz * a.inv_d[0]);
         }
         T ch = HMAP ? a.ch[1][a.mat_h[1][i]] : a.ch[1][0];
         T h = a.F[4][i] + ch * acc;
@@ -251,7 +254,7 @@ __device__ __forceinline__ void update_h_cells(const StepArgs<T>& a) {
         T dEy = Ey[i + 1] - Ey[i];
         T acc;
         if (!inpml) acc = dEx * a.inv_d[1] - dEy * a.inv_d[0];
-        else acc = pml_term(a.pml[5], 1, y, x, y, z, nx, ny, dEx, dEx * a.inv_d[1]) - pml_term(a.pml[5], 0, x, x, y, z, nx, ny, dEy, dEy * a.inv_d[0]);
+        else acc = pml_term(a.pml[5], 1, y, x, y, z, px, ny, dEx, dEx * a.inv_d[1]) - pml_term(a.pml[5], 0, x, x, y, z, px, ny, dEy, dEy * a.inv_d[0]);
         T ch = HMAP ? a.ch[2][a.mat_h[2][i]] : a.ch[2][0];
         T h = a.F[5][i] + ch * acc;
         if (SRC) h += src_value(a, 5, x, y, z, step);
@@ -305,10 +308,10 @@ __global__ void __launch_bounds__(256) k_update_e(StepArgs<T> a) {
     const int x = blockIdx.x * blockDim.x + threadIdx.x;
     const int y = blockIdx.y * blockDim.y + threadIdx.y;
     const int z = blockIdx.z;
-    const int nx = a.nx, ny = a.ny, nz = a.nz;
+    const int nx = a.nx, ny = a.ny, nz = a.nz, px = a.px;
     if (x >= nx || y >= ny) return;
-    const long long i = lidx(x, y, z, nx, ny);
-    const long long sy = nx, sz = static_cast<long long>(nx) * ny;
+    const long long i = lidx(x, y, z, px, ny);
+    const long long sy = px, sz = static_cast<long long>(px) * ny;
     const bool inpml = (x < a.Tp[0]) || (x >= nx - a.Tp[0]) || (y < a.Tp[1]) || (y >= ny - a.Tp[1]) ||
                        (DIM == 3 && ((z < a.Tp[2]) || (z >= nz - a.Tp[2])));
     int step = 0;
@@ -322,7 +325,7 @@ __global__ void __launch_bounds__(256) k_update_e(StepArgs<T> a) {
             T dHy = Hy[i] - (z > 0 ? Hy[i - sz] : T(0));
             T acc;
             if (!inpml) acc = dHz * a.inv_d[1] - dHy * a.inv_d[2];
-            else acc = pml_term(a.pml[0], 1, y, x, y, z, nx, ny, dHz, dHz * a.inv_d[1]) - pml_term(a.pml[0], 2, z, x, y, z, nx, ny, dHy, dHy * a.inv_d[2]);
+            else acc = pml_term(a.pml[0], 1, y, x, y, z, px, ny, dHz, dHz * a.inv_d[1]) - pml_term(a.pml[0], 2, z, x, y, z, px, ny, dHy, dHy * a.inv_d[2]);
             e_finish<T, SRC>(a, 0, i, x, y, z, acc, step);
         }
         if (y < ny - 1) {  // Ey
@@ -330,7 +333,7 @@ __global__ void __launch_bounds__(256) k_update_e(StepArgs<T> a) {
             T dHz = Hz[i] - (x > 0 ? Hz[i - 1] : T(0));
             T acc;
             if (!inpml) acc = dHx * a.inv_d[2] - dHz * a.inv_d[0];
-            else acc = pml_term(a.pml[1], 2, z, x, y, z, nx, ny, dHx, dHx * a.inv_d[2]) - pml_term(a.pml[1], 0, x, x, y, z, nx, ny, dHz, dHz * a.inv_d[0]);
+            else acc = pml_term(a.pml[1], 2, z, x, y, z, px, ny, dHx, dHx * a.inv_d[2]) - pml_term(a.pml[1], 0, x, x, y, z, px, ny, dHz, dHz * a.inv_d[0]);
             e_finish<T, SRC>(a, 1, i, x, y, z, acc, step);
         }
         if (z < nz - 1) {  // Ez
@@ -338,7 +341,7 @@ __global__ void __launch_bounds__(256) k_update_e(StepArgs<T> a) {
             T dHx = Hx[i] - (y > 0 ? Hx[i - sy] : T(0));
             T acc;
             if (!inpml) acc = dHy * a.inv_d[0] - dHx * a.inv_d[1];
-            else acc = pml_term(a.pml[2], 0, x, x, y, z, nx, ny, dHy, dHy * a.inv_d[0]) - pml_term(a.pml[2], 1, y, x, y, z, nx, ny, dHx, dHx * a.inv_d[1]);
+            else acc = pml_term(a.pml[2], 0, x, x, y, z, px, ny, dHy, dHy * a.inv_d[0]) - pml_term(a.pml[2], 1, y, x, y, z, px, ny, dHx, dHx * a.inv_d[1]);
             e_finish<T, SRC>(a, 2, i, x, y, z, acc, step);
         }
     } else {
@@ -346,23 +349,29 @@ __global__ void __launch_bounds__(256) k_update_e(StepArgs<T> a) {
         T dHx = Hx[i] - (y > 0 ? Hx[i - sy] : T(0));
         T acc;
         if (!inpml) acc = dHy * a.inv_d[0] - dHx * a.inv_d[1];
-        else acc = pml_term(a.pml[2], 0, x, x, y, z, nx, ny, dHy, dHy * a.inv_d[0]) - pml_term(a.pml[2], 1, y, x, y, z, nx, ny, dHx, dHx * a.inv_d[1]);
+        else acc = pml_term(a.pml[2], 0, x, x, y, z, px, ny, dHy, dHy * a.inv_d[0]) - pml_term(a.pml[2], 1, y, x, y, z, px, ny, dHx, dHx * a.inv_d[1]);
         e_finish<T, SRC>(a, 2, i, x, y, z, acc, step);
     }
 }
 
 // ------------------------------------------------ 3D split kernels ---------
 // The 3D field update is split by region: an interior box (whole x rows of
-// the y/z interior in FP32, with CPML terms only where a row enters an x
-// slab; the x/y/z interior in FP64) and the CPML slabs around it.  FP32 runs
-// both regions of a field as one launch (k_h3_all / k_e3_all), FP64 as two
-// (k_h3_int + k_h3_slab, k_e3_int + k_e3_slab).  Every thread takes W consecutive x cells so that every
-// field, psi and material access of a lane is one 16-byte load or store
-// (W = 4 in FP32, 2 in FP64): on MI355X a plain copy reaches ~3.8 TB/s with
-// 4-byte lanes and ~6.3 TB/s with 16-byte lanes.  The caller guarantees
-// nx % W == 0 and Tx % W == 0, and the psi regions are widened to whole
-// slabs [0, T) and [n - T, n) (identity coefficients on the added positions),
-// so that the W cells of a group share their CPML membership on every axis.
+// the y/z interior, with CPML terms only where a row enters an x slab; in FP64
+// on aligned grids the x/y/z interior) and the CPML slabs around it.  The
+// whole-row form runs both regions of a field as one launch (k_h3_all /
+// k_e3_all), the other as two (k_h3_int + k_h3_slab, k_e3_int + k_e3_slab).
+// Every thread takes W consecutive x cells so that every field, psi and
+// material access of a lane is one 16-byte load or store (W = 4 in FP32, 2 in
+// FP64): on MI355X a plain copy reaches ~3.8 TB/s with 4-byte lanes and
+// ~6.3 TB/s with 16-byte lanes.  Rows are stored in whole groups and the psi
+// regions widened to whole groups (grid_layout.hpp; identity coefficients on
+// the added positions), so that the W cells of a group share their CPML
+// membership on every axis.  101x93x87 FP32 with a 10-cell CPML: one thread
+// per cell 65 us a step, groups 49.
+// The interior walk leaves out the y and z CPML terms at compile time, and
+// blocks and groups are numbered in 32 bits: 256^3 FP32 with a 16-cell CPML
+// 0.302 -> 0.284 ms a step (the 64-bit divisions of the numbering and the
+// slab tests of every group cost the latency that the loads then wait for).
 template <typename T>
 struct MatLds {
     T ce, inveps;
@@ -414,9 +423,18 @@ __device__ __forceinline__ Pk<T, W> zpk() {
 // Blocks are dealt to the 8 XCDs round robin in dispatch order; renumber
 // them so that each XCD walks one contiguous eighth of the domain and the
 // y/z neighbour rows a block reads were loaded into the same L2.
-__device__ __forceinline__ long long xcd_block(long long b, long long nb) {
-    const long long q = nb / 8, r = nb % 8, x = b % 8, k = b / 8;
+__device__ __forceinline__ int xcd_block(int b, int nb) {
+    const int q = nb / 8, r = nb % 8, x = b % 8, k = b / 8;
     return (x < r ? x * (q + 1) : r * (q + 1) + (x - r) * q) + k;
+}
+
+// The cells of the group at x0 with x < nx - 1, as a bit mask (the components
+// staggered along x have no point at nx - 1, nor in the row's padding).
+template <int W>
+__device__ __forceinline__ unsigned cells_below_last(int x0, int nx) {
+    constexpr unsigned all = (1u << W) - 1;
+    const int n = nx - 1 - x0;
+    return n >= W ? all : (n > 0 ? (1u << n) - 1 : 0u);
 }
 
 // Does the group [x0, x0 + W) x {y} x {z} touch any source box?
@@ -502,107 +520,165 @@ __device__ __forceinline__ void pml_group(const PmlDev<T>& p, int ax, int pos0, 
     stv_nt<T, W>(p.psi[ax] + pi, ps);
 }
 
+// One CPML term of a group along derivative axis AX (pml_group's arithmetic):
+// load() fetches psi and the profiles with the component's other loads, apply()
+// forms the term and stores psi.  ON = false: a region without this term.
+template <typename T, int W, int AX, bool ON>
+struct PsiTerm {
+    int s;
+    T* at;
+    Pk<T, W> ps;
+    T b[AX == 0 ? W : 1], cd[AX == 0 ? W : 1], ki[AX == 0 ? W : 1];
+    __device__ __forceinline__ void load(const PmlDev<T>& p, int pos, int x0, int y, int z, int px, int ny) {
+        s = -1;
+        if (!ON) return;
+        if (pos < p.lo[AX]) s = pos;
+        else if (pos >= p.hi0[AX] && pos < p.hi1[AX]) s = p.lo[AX] + pos - p.hi0[AX];
+        if (s < 0) return;
+        long long pi;
+        if (AX == 0) pi = s + static_cast<long long>(p.S[0]) * (y + static_cast<long long>(ny) * z);
+        else if (AX == 1) pi = x0 + static_cast<long long>(px) * (s + static_cast<long long>(p.S[1]) * z);
+        else pi = x0 + static_cast<long long>(px) * (y + static_cast<long long>(ny) * s);
+        at = p.psi[AX] + pi;
+        ps = ldv_nt<T, W>(at);
+        if (AX == 0) {
+            const Pk<T, W> vb = ldv<T, W>(p.b[0] + pos), vc = ldv<T, W>(p.cd[0] + pos), vk = ldv<T, W>(p.kinv[0] + pos);
+#pragma unroll
+            for (int w = 0; w < (AX == 0 ? W : 1); ++w) {
+                b[w] = vb.v[w];
+                cd[w] = vc.v[w];
+                ki[w] = vk.v[w];
+            }
+        } else {
+            b[0] = p.b[AX][pos];
+            cd[0] = p.cd[AX][pos];
+            ki[0] = p.kinv[AX][pos];
+        }
+    }
+    // term = dV/d, or dV/(kappa d) + psi' on psi positions; cells outside
+    // `valid` keep their psi
+    __device__ __forceinline__ void apply(const T (&dV)[W], T invd, unsigned valid, T (&term)[W]) {
+#pragma unroll
+        for (int w = 0; w < W; ++w) term[w] = dV[w] * invd;
+        if (!ON || s < 0) return;
+#pragma unroll
+        for (int w = 0; w < W; ++w) {
+            const int k = AX == 0 ? w : 0;
+            const T psi = fma(b[k], ps.v[w], cd[k] * dV[w]);
+            if (valid & (1u << w)) ps.v[w] = psi;
+            term[w] = fma(ki[k], term[w], psi);
+        }
+        stv_nt<T, W>(at, ps);
+    }
+};
+
+// t1 - t2 of a curl.  FMA (grids whose rows or x CPML are no whole groups):
+// cells outside the CPML keep the second product unrounded, as the per-cell
+// kernels that swept such grids form it; FP32 metals amplify a change of
+// rounding.  plain: the group's cells outside the CPML.
+template <typename T, int W, bool FMA>
+__device__ __forceinline__ void curl_of(const T (&t1)[W], const T (&t2)[W], const T (&d2)[W], T inv2, unsigned plain, T (&acc)[W]) {
+// (a product that feeds the difference is rounded first, whatever the path)
+#pragma clang fp contract(off)
+#pragma unroll
+    for (int w = 0; w < W; ++w) {
+        acc[w] = t1[w] - t2[w];
+        if (FMA && (plain & (1u << w))) acc[w] = fma(-inv2, d2[w], t1[w]);
+    }
+}
+
+// The cells of the group with Tx <= x < nx - Tx, as a bit mask.
+template <int W>
+__device__ __forceinline__ unsigned cells_inside(int x0, int nx, int Tx) {
+    unsigned m = 0;
+#pragma unroll
+    for (int w = 0; w < W; ++w)
+        if (x0 + w >= Tx && x0 + w < nx - Tx) m |= 1u << w;
+    return m;
+}
+
 // H update of the group (x0..x0+W-1, y, z): H += ch (curl E) (+ sources).
+// PX / PYZ: the group may lie in an x / in a y or z CPML slab.
 // nb: the next lane of the wave holds the next group of the same row, so the
-// first value of that group comes by a lane shuffle instead of a load
-template <typename T, int W, bool PML, bool SRC>
+// first value of that group comes by a lane shuffle instead of a load.
+template <typename T, int W, bool PX, bool PYZ, bool SRC, bool FMA>
 __device__ __forceinline__ void h_group(const StepArgs<T>& a, int x0, int y, int z, bool nb = false) {
-    const int nx = a.nx, ny = a.ny, nz = a.nz;
-    const long long sy = nx, sz = static_cast<long long>(nx) * ny;
-    const long long i = lidx(x0, y, z, nx, ny);
+    const int nx = a.nx, ny = a.ny, nz = a.nz, px = a.px;
+    const long long sy = px, sz = static_cast<long long>(px) * ny;
+    const long long i = lidx(x0, y, z, px, ny);
     const T idx = a.inv_d[0], idy = a.inv_d[1], idz = a.inv_d[2];
     const T *Ex = a.F[0], *Ey = a.F[1], *Ez = a.F[2];
     const Pk<T, W> ex = ldv<T, W>(Ex + i), ey = ldv<T, W>(Ey + i), ez = ldv<T, W>(Ez + i);
+    const bool last = x0 + W >= nx, yin = y < ny - 1, zin = z < nz - 1;
+    const unsigned all = (1u << W) - 1, vx = cells_below_last<W>(x0, nx);  // vx: cells with x < nx - 1
+    const unsigned plain = FMA && !PYZ ? cells_inside<W>(x0, nx, a.Tp[0]) : 0u;
     const T ez_nb = __shfl_down(ez.v[0], 1), ey_nb = __shfl_down(ey.v[0], 1);
-    const bool last = x0 + W >= nx;
-    const unsigned all = (1u << W) - 1, vx = last ? (all >> 1) : all;  // cells with x < nx - 1
     const bool src = SRC && group_has_src<T, W>(a, x0, y, z);
     const int step = src ? step_now(a.step, a.stepv) : 0;
-    T d1[W], d2[W], t1[W], t2[W];
-    if (y < ny - 1 && z < nz - 1) {  // Hx += ch [dEy/dz - dEz/dy]
+    T d1[W], d2[W], t1[W], t2[W], acc[W];
+    auto finish = [&](int c, Pk<T, W>& h, unsigned valid) {
+        const T ch = a.ch[c][0];
+#pragma unroll
+        for (int w = 0; w < W; ++w) {
+            if (!(valid & (1u << w))) continue;
+            T hv = fma(ch, acc[w], h.v[w]);
+            if (src) hv += src_value(a, 3 + c, x0 + w, y, z, step);
+            h.v[w] = hv;
+        }
+        stv_nt<T, W>(a.F[3 + c] + i, h);
+    };
+    if (yin && zin) {  // Hx += ch [dEy/dz - dEz/dy]
         const Pk<T, W> eyz = ldv<T, W>(Ey + i + sz), ezy = ldv<T, W>(Ez + i + sy);
         Pk<T, W> h = ldv_nt<T, W>(a.F[3] + i);
+        PsiTerm<T, W, 2, PYZ> q1;
+        PsiTerm<T, W, 1, PYZ> q2;
+        q1.load(a.pml[3], z, x0, y, z, px, ny);
+        q2.load(a.pml[3], y, x0, y, z, px, ny);
 #pragma unroll
         for (int w = 0; w < W; ++w) {
             d1[w] = eyz.v[w] - ey.v[w];
             d2[w] = ezy.v[w] - ez.v[w];
         }
-        if (PML) {
-            pml_group<T, W>(a.pml[3], 2, z, x0, y, z, nx, ny, d1, idz, all, t1);
-            pml_group<T, W>(a.pml[3], 1, y, x0, y, z, nx, ny, d2, idy, all, t2);
-        } else {
-#pragma unroll
-            for (int w = 0; w < W; ++w) {
-                t1[w] = d1[w] * idz;
-                t2[w] = d2[w] * idy;
-            }
-        }
-        const T ch = a.ch[0][0];
-#pragma unroll
-        for (int w = 0; w < W; ++w) {
-            T hv = h.v[w] + ch * (t1[w] - t2[w]);
-            if (src) hv += src_value(a, 3, x0 + w, y, z, step);
-            h.v[w] = hv;
-        }
-        stv_nt<T, W>(a.F[3] + i, h);
+        q1.apply(d1, idz, all, t1);
+        q2.apply(d2, idy, all, t2);
+        curl_of<T, W, FMA>(t1, t2, d2, idy, plain, acc);
+        finish(0, h, all);
     }
-    if (z < nz - 1) {  // Hy += ch [dEz/dx - dEx/dz], x < nx - 1
+    if (zin) {  // Hy += ch [dEz/dx - dEx/dz], x < nx - 1
         const Pk<T, W> exz = ldv<T, W>(Ex + i + sz);
         const T ezn = last ? T(0) : (nb ? ez_nb : Ez[i + W]);
         Pk<T, W> h = ldv_nt<T, W>(a.F[4] + i);
+        PsiTerm<T, W, 0, PX> q1;
+        PsiTerm<T, W, 2, PYZ> q2;
+        q1.load(a.pml[4], x0, x0, y, z, px, ny);
+        q2.load(a.pml[4], z, x0, y, z, px, ny);
 #pragma unroll
         for (int w = 0; w < W; ++w) {
-            d1[w] = (w + 1 < W ? ez.v[w + 1] : ezn) - ez.v[w];
+            d1[w] = (w + 1 < W ? ez.v[w + 1 < W ? w + 1 : w] : ezn) - ez.v[w];
             d2[w] = exz.v[w] - ex.v[w];
         }
-        if (PML) {
-            pml_group<T, W>(a.pml[4], 0, x0, x0, y, z, nx, ny, d1, idx, vx, t1);
-            pml_group<T, W>(a.pml[4], 2, z, x0, y, z, nx, ny, d2, idz, vx, t2);
-        } else {
-#pragma unroll
-            for (int w = 0; w < W; ++w) {
-                t1[w] = d1[w] * idx;
-                t2[w] = d2[w] * idz;
-            }
-        }
-        const T ch = a.ch[1][0];
-#pragma unroll
-        for (int w = 0; w < W; ++w) {
-            if (!(vx & (1u << w))) continue;
-            T hv = h.v[w] + ch * (t1[w] - t2[w]);
-            if (src) hv += src_value(a, 4, x0 + w, y, z, step);
-            h.v[w] = hv;
-        }
-        stv_nt<T, W>(a.F[4] + i, h);
+        q1.apply(d1, idx, vx, t1);
+        q2.apply(d2, idz, vx, t2);
+        curl_of<T, W, FMA>(t1, t2, d2, idz, plain, acc);
+        finish(1, h, vx);
     }
-    if (y < ny - 1) {  // Hz += ch [dEx/dy - dEy/dx], x < nx - 1
+    if (yin) {  // Hz += ch [dEx/dy - dEy/dx], x < nx - 1
         const Pk<T, W> exy = ldv<T, W>(Ex + i + sy);
         const T eyn = last ? T(0) : (nb ? ey_nb : Ey[i + W]);
         Pk<T, W> h = ldv_nt<T, W>(a.F[5] + i);
+        PsiTerm<T, W, 1, PYZ> q1;
+        PsiTerm<T, W, 0, PX> q2;
+        q1.load(a.pml[5], y, x0, y, z, px, ny);
+        q2.load(a.pml[5], x0, x0, y, z, px, ny);
 #pragma unroll
         for (int w = 0; w < W; ++w) {
             d1[w] = exy.v[w] - ex.v[w];
-            d2[w] = (w + 1 < W ? ey.v[w + 1] : eyn) - ey.v[w];
+            d2[w] = (w + 1 < W ? ey.v[w + 1 < W ? w + 1 : w] : eyn) - ey.v[w];
         }
-        if (PML) {
-            pml_group<T, W>(a.pml[5], 1, y, x0, y, z, nx, ny, d1, idy, vx, t1);
-            pml_group<T, W>(a.pml[5], 0, x0, x0, y, z, nx, ny, d2, idx, vx, t2);
-        } else {
-#pragma unroll
-            for (int w = 0; w < W; ++w) {
-                t1[w] = d1[w] * idy;
-                t2[w] = d2[w] * idx;
-            }
-        }
-        const T ch = a.ch[2][0];
-#pragma unroll
-        for (int w = 0; w < W; ++w) {
-            if (!(vx & (1u << w))) continue;
-            T hv = h.v[w] + ch * (t1[w] - t2[w]);
-            if (src) hv += src_value(a, 5, x0 + w, y, z, step);
-            h.v[w] = hv;
-        }
-        stv_nt<T, W>(a.F[5] + i, h);
+        q1.apply(d1, idy, vx, t1);
+        q2.apply(d2, idx, vx, t2);
+        curl_of<T, W, FMA>(t1, t2, d2, idx, plain, acc);
+        finish(2, h, vx);
     }
 }
 
@@ -617,13 +693,13 @@ __device__ __forceinline__ Pk<uint8_t, W> load_ids(const uint8_t* m, long long i
     return ldv_nt<uint8_t, W>(m + i);
 }
 
-// E of the W cells of a group from their curl terms t1 - t2, materials,
+// E of the W cells of a group from their curl acc, materials,
 // sources and poles: e_new for a group, with each pole's P and J of the
 // group read and written as one aligned 16-byte access (the pole-state box
 // is 4-aligned in x); cells without poles keep their stored values.
-template <typename T, int W, bool PRE = false>
+template <typename T, int W>
 __device__ __forceinline__ Pk<T, W> e_finish_group(const StepArgs<T>& a, const MatLds<T> (*mt)[CHIML_MAX_MAT], int c, long long i, int x0,
-                                               int y, int z, unsigned valid, const T (&t1)[W], const T (&t2)[W], bool src, int step) {
+                                               int y, int z, unsigned valid, const T (&acc)[W], bool src, int step) {
     const Pk<uint8_t, W> id = load_ids<W>(a.mat_e[c], i);
     Pk<T, W> e = ldv_nt<T, W>(a.F[c] + i);
     T jsum[W];
@@ -633,14 +709,7 @@ __device__ __forceinline__ Pk<T, W> e_finish_group(const StepArgs<T>& a, const M
         jsum[w] = T(0);
         anyp |= (mt[c][id.v[w]].poleset >= 0) && (valid & (1u << w));
     }
-    if (PRE && anyp) {  // the pole currents were advanced by ade_block this step
-        const int* bx = a.box[c];
-        const long long bi = (x0 - bx[0]) + static_cast<long long>(bx[1] - bx[0]) * ((y - bx[2]) + static_cast<long long>(bx[3] - bx[2]) * (z - bx[4]));
-        const Pk<T, W> js = ldv<T, W>(a.jsum[c] + bi);
-#pragma unroll
-        for (int w = 0; w < W; ++w)
-            if (mt[c][id.v[w]].poleset >= 0 && (valid & (1u << w))) jsum[w] = js.v[w];
-    } else if (anyp) {  // rare: groups that touch a dispersive object
+    if (anyp) {  // rare: groups that touch a dispersive object
         const int* bx = a.box[c];
         const long long bi = (x0 - bx[0]) + static_cast<long long>(bx[1] - bx[0]) * ((y - bx[2]) + static_cast<long long>(bx[3] - bx[2]) * (z - bx[4]));
         int np[W], npmax = 0;
@@ -675,88 +744,105 @@ __device__ __forceinline__ Pk<T, W> e_finish_group(const StepArgs<T>& a, const M
         const MatLds<T> m = mt[c][id.v[w]];
         const T sv = src ? src_value(a, c, x0 + w, y, z, step) : T(0);
         const T e_base = (m.flags & CHIML_MAT_DCELL) ? e.v[w] : e.v[w] + sv;
-        e.v[w] = e_base + m.ce * (t1[w] - t2[w]) - m.inveps * jsum[w];
+        e.v[w] = fma(-m.inveps, jsum[w], fma(m.ce, acc[w], e_base));
     }
     stv_nt<T, W>(a.F[c] + i, e);
     return e;
 }
 
-// E update of the group: the E-form of updateE/updateD + ADE + D2E per cell.// E update of the group: the E-form of updateE/updateD + ADE + D2E per cell.
+// E update of the group: the E-form of updateE/updateD + ADE + D2E per cell,
+// the pole currents already advanced by ade_block.  PX, PYZ, FMA as in
+// h_group; mt: the material tables in LDS.
 // nb: the previous lane of the wave holds the previous group of the same row
-template <typename T, int W, bool PML, bool SRC, bool PRE>
+template <typename T, int W, bool PX, bool PYZ, bool SRC, bool FMA>
 __device__ __forceinline__ void e_group(const StepArgs<T>& a, const MatLds<T> (*mt)[CHIML_MAX_MAT], int x0, int y, int z,
                                         bool nb = false) {
-    const int nx = a.nx, ny = a.ny, nz = a.nz;
-    const long long sy = nx, sz = static_cast<long long>(nx) * ny;
-    const long long i = lidx(x0, y, z, nx, ny);
+    const int nx = a.nx, ny = a.ny, nz = a.nz, px = a.px;
+    const long long sy = px, sz = static_cast<long long>(px) * ny;
+    const long long i = lidx(x0, y, z, px, ny);
     const T idx = a.inv_d[0], idy = a.inv_d[1], idz = a.inv_d[2];
     const T *Hx = a.F[3], *Hy = a.F[4], *Hz = a.F[5];
     const Pk<T, W> hx = ldv<T, W>(Hx + i), hy = ldv<T, W>(Hy + i), hz = ldv<T, W>(Hz + i);
+    const bool yin = y < ny - 1, zin = z < nz - 1;
+    const unsigned all = (1u << W) - 1, vx = cells_below_last<W>(x0, nx);
+    const unsigned plain = FMA && !PYZ ? cells_inside<W>(x0, nx, a.Tp[0]) : 0u;
     const T hz_nb = __shfl_up(hz.v[W - 1], 1), hy_nb = __shfl_up(hy.v[W - 1], 1);
-    const bool last = x0 + W >= nx;
-    const unsigned all = (1u << W) - 1, vx = last ? (all >> 1) : all;
     const bool src = SRC && group_has_src<T, W>(a, x0, y, z);
     const int step = src ? step_now(a.step, a.stepv) : 0;
-    T d1[W], d2[W], t1[W], t2[W];
+    T d1[W], d2[W], t1[W], t2[W], acc[W];
+    auto finish = [&](int c, unsigned valid) {
+        const Pk<uint8_t, W> id = load_ids<W>(a.mat_e[c], i);
+        Pk<T, W> e = ldv_nt<T, W>(a.F[c] + i);
+        bool anyp = false;
+#pragma unroll
+        for (int w = 0; w < W; ++w) anyp |= (mt[c][id.v[w]].poleset >= 0) && (valid & (1u << w));
+        Pk<T, W> js = zpk<T, W>();
+        if (anyp) {  // rare: groups that touch a dispersive object
+            const int* bx = a.box[c];
+            const long long bi = (x0 - bx[0]) + static_cast<long long>(bx[1] - bx[0]) * ((y - bx[2]) + static_cast<long long>(bx[3] - bx[2]) * (z - bx[4]));
+            js = ldv<T, W>(a.jsum[c] + bi);
+        }
+#pragma unroll
+        for (int w = 0; w < W; ++w) {
+            if (!(valid & (1u << w))) continue;
+            const MatLds<T> m = mt[c][id.v[w]];
+            const T sv = src ? src_value(a, c, x0 + w, y, z, step) : T(0);
+            const T e_base = (m.flags & CHIML_MAT_DCELL) ? e.v[w] : e.v[w] + sv;
+            const T jsum = m.poleset >= 0 ? js.v[w] : T(0);
+            e.v[w] = fma(-m.inveps, jsum, fma(m.ce, acc[w], e_base));
+        }
+        stv_nt<T, W>(a.F[c] + i, e);
+    };
     {  // Ex += ce [dHz/dy - dHy/dz], x < nx - 1
         const Pk<T, W> hzy = y > 0 ? ldv<T, W>(Hz + i - sy) : zpk<T, W>();
         const Pk<T, W> hyz = z > 0 ? ldv<T, W>(Hy + i - sz) : zpk<T, W>();
+        PsiTerm<T, W, 1, PYZ> q1;
+        PsiTerm<T, W, 2, PYZ> q2;
+        q1.load(a.pml[0], y, x0, y, z, px, ny);
+        q2.load(a.pml[0], z, x0, y, z, px, ny);
 #pragma unroll
         for (int w = 0; w < W; ++w) {
             d1[w] = hz.v[w] - hzy.v[w];
             d2[w] = hy.v[w] - hyz.v[w];
         }
-        if (PML) {
-            pml_group<T, W>(a.pml[0], 1, y, x0, y, z, nx, ny, d1, idy, vx, t1);
-            pml_group<T, W>(a.pml[0], 2, z, x0, y, z, nx, ny, d2, idz, vx, t2);
-        } else {
-#pragma unroll
-            for (int w = 0; w < W; ++w) {
-                t1[w] = d1[w] * idy;
-                t2[w] = d2[w] * idz;
-            }
-        }
-        e_finish_group<T, W, PRE>(a, mt, 0, i, x0, y, z, vx, t1, t2, src, step);
+        q1.apply(d1, idy, vx, t1);
+        q2.apply(d2, idz, vx, t2);
+        curl_of<T, W, FMA>(t1, t2, d2, idz, plain, acc);
+        finish(0, vx);
     }
-    if (y < ny - 1) {  // Ey += ce [dHx/dz - dHz/dx]
+    if (yin) {  // Ey += ce [dHx/dz - dHz/dx]
         const Pk<T, W> hxz = z > 0 ? ldv<T, W>(Hx + i - sz) : zpk<T, W>();
         const T hzm = x0 > 0 ? (nb ? hz_nb : Hz[i - 1]) : T(0);
+        PsiTerm<T, W, 2, PYZ> q1;
+        PsiTerm<T, W, 0, PX> q2;
+        q1.load(a.pml[1], z, x0, y, z, px, ny);
+        q2.load(a.pml[1], x0, x0, y, z, px, ny);
 #pragma unroll
         for (int w = 0; w < W; ++w) {
             d1[w] = hx.v[w] - hxz.v[w];
-            d2[w] = hz.v[w] - (w > 0 ? hz.v[w - 1] : hzm);
+            d2[w] = hz.v[w] - (w > 0 ? hz.v[w > 0 ? w - 1 : 0] : hzm);
         }
-        if (PML) {
-            pml_group<T, W>(a.pml[1], 2, z, x0, y, z, nx, ny, d1, idz, all, t1);
-            pml_group<T, W>(a.pml[1], 0, x0, x0, y, z, nx, ny, d2, idx, all, t2);
-        } else {
-#pragma unroll
-            for (int w = 0; w < W; ++w) {
-                t1[w] = d1[w] * idz;
-                t2[w] = d2[w] * idx;
-            }
-        }
-        e_finish_group<T, W, PRE>(a, mt, 1, i, x0, y, z, all, t1, t2, src, step);
+        q1.apply(d1, idz, all, t1);
+        q2.apply(d2, idx, all, t2);
+        curl_of<T, W, FMA>(t1, t2, d2, idx, plain, acc);
+        finish(1, all);
     }
-    if (z < nz - 1) {  // Ez += ce [dHy/dx - dHx/dy]
+    if (zin) {  // Ez += ce [dHy/dx - dHx/dy]
         const Pk<T, W> hxy = y > 0 ? ldv<T, W>(Hx + i - sy) : zpk<T, W>();
         const T hym = x0 > 0 ? (nb ? hy_nb : Hy[i - 1]) : T(0);
+        PsiTerm<T, W, 0, PX> q1;
+        PsiTerm<T, W, 1, PYZ> q2;
+        q1.load(a.pml[2], x0, x0, y, z, px, ny);
+        q2.load(a.pml[2], y, x0, y, z, px, ny);
 #pragma unroll
         for (int w = 0; w < W; ++w) {
-            d1[w] = hy.v[w] - (w > 0 ? hy.v[w - 1] : hym);
+            d1[w] = hy.v[w] - (w > 0 ? hy.v[w > 0 ? w - 1 : 0] : hym);
             d2[w] = hx.v[w] - hxy.v[w];
         }
-        if (PML) {
-            pml_group<T, W>(a.pml[2], 0, x0, x0, y, z, nx, ny, d1, idx, all, t1);
-            pml_group<T, W>(a.pml[2], 1, y, x0, y, z, nx, ny, d2, idy, all, t2);
-        } else {
-#pragma unroll
-            for (int w = 0; w < W; ++w) {
-                t1[w] = d1[w] * idx;
-                t2[w] = d2[w] * idy;
-            }
-        }
-        e_finish_group<T, W, PRE>(a, mt, 2, i, x0, y, z, all, t1, t2, src, step);
+        q1.apply(d1, idx, all, t1);
+        q2.apply(d2, idy, all, t2);
+        curl_of<T, W, FMA>(t1, t2, d2, idy, plain, acc);
+        finish(2, all);
     }
 }
 
@@ -778,11 +864,11 @@ __device__ __forceinline__ void ade_block(const StepArgs<T>& a, int c, long long
     const int x0 = bx[0] + static_cast<int>(t - r * gw) * W;
     const int y = bx[2] + static_cast<int>(r % ny), z = bx[4] + static_cast<int>(r / ny);
     const long long bi = t * W;  // (x0 - bx0) + width * ((y - by0) + height * (z - bz0))
-    const long long i = lidx(x0, y, z, a.nx, a.ny);
+    const long long i = lidx(x0, y, z, a.px, a.ny);
     const Pk<uint8_t, W> id = load_ids<W>(a.mat_e[c], i);
     // the cells the E kernels update: Ex x < nx - 1, Ey y < ny - 1, Ez z < nz - 1
     unsigned valid = (1u << W) - 1;
-    if (c == 0 && x0 + W >= a.nx) valid >>= 1;
+    if (c == 0) valid = cells_below_last<W>(x0, a.nx);
     if ((c == 1 && y >= a.ny - 1) || (c == 2 && z >= a.nz - 1)) valid = 0;
     int ps[W], np[W], npmax = 0;
 #pragma unroll
@@ -825,25 +911,17 @@ __device__ __forceinline__ void ade_block(const StepArgs<T>& a, int c, long long
 // planes a group reads are still in that XCD's L2 (a whole plane of six
 // fields is larger than an L2).
 template <typename T, int W>
-__device__ __forceinline__ long long int_groups(const Box3& b) {
-    const int gw = (b.x1 - b.x0) / W, ny = b.y1 - b.y0, nz = b.z1 - b.z0;
-    const int by = b.by > 0 ? b.by : ny, nb = (ny + by - 1) / by;
-    return static_cast<long long>(gw) * by * nz * nb;
-}
-
-template <typename T, int W>
-__device__ __forceinline__ bool int_group(const Box3& b, long long t, int& x0, int& y, int& z, int& col) {
-    const int gw = (b.x1 - b.x0) / W, ny = b.y1 - b.y0, nz = b.z1 - b.z0;
-    const int by = b.by > 0 ? b.by : ny;
-    if (t >= int_groups<T, W>(b)) return false;
-    long long r = t / gw;
+__device__ __forceinline__ bool int_group(const Box3& b, int blk, int& x0, int& y, int& z, int& col) {
+    const unsigned gw = (b.x1 - b.x0) / W, ny = b.y1 - b.y0, nz = b.z1 - b.z0;
+    const unsigned by = b.by > 0 ? b.by : ny, nb = (ny + by - 1) / by;
+    const unsigned t = static_cast<unsigned>(blk) * blockDim.x + threadIdx.x;
+    unsigned r = t / gw;
+    if (r >= by * nz * nb) return false;
     col = static_cast<int>(t - r * gw);
     x0 = b.x0 + col * W;
-    const int yy = static_cast<int>(r % by);
-    r /= by;
-    z = b.z0 + static_cast<int>(r % nz);
-    const int band = static_cast<int>(r / nz);
-    y = b.y0 + band * by + yy;
+    const unsigned p = r / by, band = p / nz;
+    z = b.z0 + static_cast<int>(p - band * nz);
+    y = b.y0 + static_cast<int>(band * by + (r - p * by));
     return y < b.y1;  // the last band may be short
 }
 
@@ -863,13 +941,11 @@ __device__ __forceinline__ void h3_int_sweep(const StepArgs<T>& a, const Box3& b
         if (c < 3) ade_block<T, W, SRC>(a, c, bx - c * ade_bpc);
         return;
     }
-    const long long blk = xcd_block(bx - nade, nib);
     int x0, y, z, col;
-    const bool in = int_group<T, W>(b, blk * blockDim.x + threadIdx.x, x0, y, z, col);
-    if (!in) return;
+    if (!int_group<T, W>(b, xcd_block(bx - nade, nib), x0, y, z, col)) return;
     // consecutive threads walk a row: lane + 1 holds the next group unless this one ends the row
     const int lane = threadIdx.x & 63, gw = (b.x1 - b.x0) / W;
-    h_group<T, W, false, SRC>(a, x0, y, z, lane < 63 && col + 1 < gw);
+    h_group<T, W, false, false, SRC, false>(a, x0, y, z, lane < 63 && col + 1 < gw);
 }
 
 template <typename T, int W, bool SRC, bool ADV>
@@ -880,11 +956,10 @@ __global__ void __launch_bounds__(256) k_h3_int(StepArgs<T> a, Box3 b, int nib, 
 
 template <typename T, int W, bool SRC>
 __device__ __forceinline__ void e3_int_sweep(const StepArgs<T>& a, const MatLds<T> (*mt)[CHIML_MAX_MAT], const Box3& b, int bx, int nb) {
-    const long long blk = xcd_block(bx, nb);
     int x0, y, z, col;
-    if (!int_group<T, W>(b, blk * blockDim.x + threadIdx.x, x0, y, z, col)) return;
+    if (!int_group<T, W>(b, xcd_block(bx, nb), x0, y, z, col)) return;
     const int lane = threadIdx.x & 63;
-    e_group<T, W, false, SRC, true>(a, mt, x0, y, z, lane > 0 && col > 0);
+    e_group<T, W, false, false, SRC, false>(a, mt, x0, y, z, lane > 0 && col > 0);
 }
 
 template <typename T, int W, bool SRC>
@@ -895,68 +970,57 @@ __global__ void __launch_bounds__(256) k_e3_int(StepArgs<T> a, Box3 b, int nm0, 
     e3_int_sweep<T, W, SRC>(a, mt, b, blockIdx.x, gridDim.x);
 }
 
-
 // CPML slab groups: the union of the z slabs, the y slabs inside the z range
 // and the x slabs inside the y and z ranges, enumerated x fastest, in units
 // of W-cell groups (gx = nx / W groups per row, gT = Tx / W per x slab).
 struct SlabMap {
-    int nx, ny, nz, Tx, Ty, Tz, W;
-    long long nA, nB, nC;  // group counts of the three regions
+    int nx, ny, nz, Tx, Ty, Tz, W;  // nx: cells per stored row
+    unsigned nA, nB, nC;  // group counts of the three regions
 };
 
 // col / rowlen: the group's place in a run of consecutive groups of one x
 // row (rowlen 0 where rows are not walked whole: the x slabs)
-__device__ __forceinline__ void slab_group(const SlabMap& m, long long t, int& x0, int& y, int& z, int& col, int& rowlen) {
-    const int gx = m.nx / m.W;
+__device__ __forceinline__ bool slab_group(const SlabMap& m, unsigned t, int& x0, int& y, int& z, int& col, int& rowlen) {
+    if (t >= m.nA + m.nB + m.nC) return false;
+    const unsigned gx = m.nx / m.W;
     rowlen = gx;
     if (t < m.nA) {  // z slabs: z in [0,Tz) U [nz-Tz,nz), all x, y
-        const long long plane = static_cast<long long>(gx) * m.ny;
-        const int k = static_cast<int>(t / plane);
-        const long long r = t - k * plane;
-        z = k < m.Tz ? k : m.nz - 2 * m.Tz + k;
-        y = static_cast<int>(r / gx);
-        col = static_cast<int>(r - static_cast<long long>(y) * gx);
+        const unsigned row = t / gx, k = row / m.ny;
+        z = static_cast<int>(k) < m.Tz ? k : m.nz - 2 * m.Tz + k;
+        y = row - k * m.ny;
+        col = t - row * gx;
         x0 = col * m.W;
-        return;
+        return true;
     }
     t -= m.nA;
     if (t < m.nB) {  // y slabs inside the z interior
-        const long long plane = static_cast<long long>(gx) * 2 * m.Ty;
-        const int k = static_cast<int>(t / plane);
-        const long long r = t - k * plane;
+        const unsigned row = t / gx, w = 2 * m.Ty, k = row / w;
         z = m.Tz + k;
-        const int yy = static_cast<int>(r / gx);
-        col = static_cast<int>(r - static_cast<long long>(yy) * gx);
+        const int yy = row - k * w;
+        col = t - row * gx;
         x0 = col * m.W;
         y = yy < m.Ty ? yy : m.ny - 2 * m.Ty + yy;
-        return;
+        return true;
     }
     t -= m.nB;
     col = 0;
     rowlen = 0;
-    {  // x slabs inside the y and z interiors
-        const int gT = 2 * (m.Tx / m.W);
-        const int nyi = m.ny - 2 * m.Ty;
-        const long long plane = static_cast<long long>(gT) * nyi;
-        const int k = static_cast<int>(t / plane);
-        const long long r = t - k * plane;
-        z = m.Tz + k;
-        const int yy = static_cast<int>(r / gT);
-        const int xx = static_cast<int>(r - static_cast<long long>(yy) * gT) * m.W;
-        y = m.Ty + yy;
-        x0 = xx < m.Tx ? xx : m.nx - 2 * m.Tx + xx;
-    }
+    // x slabs inside the y and z interiors
+    const unsigned gT = 2 * (m.Tx / m.W), row = t / gT, nyi = m.ny - 2 * m.Ty, k = row / nyi;
+    z = m.Tz + k;
+    const int xx = static_cast<int>(t - row * gT) * m.W;
+    y = m.Ty + static_cast<int>(row - k * nyi);
+    x0 = xx < m.Tx ? xx : m.nx - 2 * m.Tx + xx;
+    return true;
 }
 
 template <typename T, int W, bool SRC>
 __device__ __forceinline__ void h3_slab_sweep(const StepArgs<T>& a, const SlabMap& m, int bx, int nb) {
-    const long long t = xcd_block(bx, nb) * blockDim.x + threadIdx.x;
-    if (t >= m.nA + m.nB + m.nC) return;
     int x0, y, z, col, rowlen;
-    slab_group(m, t, x0, y, z, col, rowlen);
+    if (!slab_group(m, static_cast<unsigned>(xcd_block(bx, nb)) * blockDim.x + threadIdx.x, x0, y, z, col, rowlen)) return;
     // the z- and y-slab regions start on row boundaries (nA is whole rows), so
     // lane + 1 holds the next group of the row unless this one ends it
-    h_group<T, W, true, SRC>(a, x0, y, z, (threadIdx.x & 63) < 63 && col + 1 < rowlen);
+    h_group<T, W, true, true, SRC, false>(a, x0, y, z, (threadIdx.x & 63) < 63 && col + 1 < rowlen);
 }
 
 template <typename T, int W, bool SRC>
@@ -966,11 +1030,9 @@ __global__ void __launch_bounds__(256) k_h3_slab(StepArgs<T> a, SlabMap m) {
 
 template <typename T, int W, bool SRC>
 __device__ __forceinline__ void e3_slab_sweep(const StepArgs<T>& a, const MatLds<T> (*mt)[CHIML_MAX_MAT], const SlabMap& m, int bx, int nb) {
-    const long long t = xcd_block(bx, nb) * blockDim.x + threadIdx.x;
-    if (t >= m.nA + m.nB + m.nC) return;
     int x0, y, z, col, rowlen;
-    slab_group(m, t, x0, y, z, col, rowlen);
-    e_group<T, W, true, SRC, true>(a, mt, x0, y, z);  // (the lane shuffle measured slower here)
+    if (!slab_group(m, static_cast<unsigned>(xcd_block(bx, nb)) * blockDim.x + threadIdx.x, x0, y, z, col, rowlen)) return;
+    e_group<T, W, true, true, SRC, false>(a, mt, x0, y, z);  // (the lane shuffle measured slower here)
 }
 
 template <typename T, int W, bool SRC>
@@ -981,15 +1043,15 @@ __global__ void __launch_bounds__(256) k_e3_slab(StepArgs<T> a, SlabMap m, int n
     e3_slab_sweep<T, W, SRC>(a, mt, m, blockIdx.x, gridDim.x);
 }
 
-// FP32: the whole 3D sweep of a field in one launch, [pole update | CPML
-// slabs | interior] for H and [CPML slabs | interior] for E, each region
-// starting on a multiple of 8 blocks so that every region keeps its XCD
-// numbering.  The less efficient slab and pole blocks run first and overlap
-// the interior stream, and two launch ramps and tails per step go away
-// (5% on the 256^3 step).  FP64 keeps separate launches: there the interior
-// kernel carries no CPML code and runs at a higher occupancy than a merged
-// kernel would.
-template <typename T, int W, bool SRC>
+// Whole-row layout (GridLayout::rows): the whole 3D sweep of a field in one
+// launch, [pole update | CPML slabs | interior] for H and [CPML slabs |
+// interior] for E, each region starting on a multiple of 8 blocks so that
+// every region keeps its XCD numbering.  The less efficient slab and pole
+// blocks run first and overlap the interior stream, and two launch ramps and
+// tails per step go away (5% on the 256^3 FP32 step).  Aligned FP64 grids keep
+// separate launches: there the interior kernel carries no CPML code and runs
+// at a higher occupancy than a merged kernel would.
+template <typename T, int W, bool SRC, bool FMA>
 __device__ __forceinline__ void h3_all_sweep(const StepArgs<T>& a, const Box3& b, const SlabMap& m, int nib, int nsbp,
                                              int ade_bpc, int bx) {
     const int nade = ade_blocks(ade_bpc);
@@ -1000,52 +1062,46 @@ __device__ __forceinline__ void h3_all_sweep(const StepArgs<T>& a, const Box3& b
     }
     bx -= nade;
     if (bx < nsbp) {
-        const long long t = xcd_block(bx, nsbp) * blockDim.x + threadIdx.x;
-        if (t >= m.nA + m.nB + m.nC) return;
         int x0, y, z, col, rowlen;
-        slab_group(m, t, x0, y, z, col, rowlen);
-        h_group<T, W, true, SRC>(a, x0, y, z, (threadIdx.x & 63) < 63 && col + 1 < rowlen);
+        if (!slab_group(m, static_cast<unsigned>(xcd_block(bx, nsbp)) * blockDim.x + threadIdx.x, x0, y, z, col, rowlen)) return;
+        h_group<T, W, true, true, SRC, FMA>(a, x0, y, z, (threadIdx.x & 63) < 63 && col + 1 < rowlen);
         return;
     }
     bx -= nsbp;
-    const long long blk = xcd_block(bx, nib);
     int x0, y, z, col;
-    if (!int_group<T, W>(b, blk * blockDim.x + threadIdx.x, x0, y, z, col)) return;
+    if (!int_group<T, W>(b, xcd_block(bx, nib), x0, y, z, col)) return;
     const int lane = threadIdx.x & 63, gw = (b.x1 - b.x0) / W;
-    h_group<T, W, true, SRC>(a, x0, y, z, lane < 63 && col + 1 < gw);
+    h_group<T, W, true, false, SRC, FMA>(a, x0, y, z, lane < 63 && col + 1 < gw);
 }
 
-template <typename T, int W, bool SRC, bool ADV>
+template <typename T, int W, bool SRC, bool ADV, bool FMA>
 __global__ void __launch_bounds__(256) k_h3_all(StepArgs<T> a, Box3 b, SlabMap m, int nib, int nsbp, int ade_bpc) {
-    h3_all_sweep<T, W, SRC>(a, b, m, nib, nsbp, ade_bpc, blockIdx.x);
+    h3_all_sweep<T, W, SRC, FMA>(a, b, m, nib, nsbp, ade_bpc, blockIdx.x);
     if (ADV) advance_counter(a);
 }
 
-template <typename T, int W, bool SRC>
+template <typename T, int W, bool SRC, bool FMA>
 __device__ __forceinline__ void e3_all_sweep(const StepArgs<T>& a, const MatLds<T> (*mt)[CHIML_MAX_MAT], const Box3& b, const SlabMap& m,
                                              int nib, int nsbp, int bx) {
     if (bx < nsbp) {
-        const long long t = xcd_block(bx, nsbp) * blockDim.x + threadIdx.x;
-        if (t >= m.nA + m.nB + m.nC) return;
         int x0, y, z, col, rowlen;
-        slab_group(m, t, x0, y, z, col, rowlen);
-        e_group<T, W, true, SRC, true>(a, mt, x0, y, z);
+        if (!slab_group(m, static_cast<unsigned>(xcd_block(bx, nsbp)) * blockDim.x + threadIdx.x, x0, y, z, col, rowlen)) return;
+        e_group<T, W, true, true, SRC, FMA>(a, mt, x0, y, z);
         return;
     }
     bx -= nsbp;
-    const long long blk = xcd_block(bx, nib);
     int x0, y, z, col;
-    if (!int_group<T, W>(b, blk * blockDim.x + threadIdx.x, x0, y, z, col)) return;
+    if (!int_group<T, W>(b, xcd_block(bx, nib), x0, y, z, col)) return;
     const int lane = threadIdx.x & 63;
-    e_group<T, W, true, SRC, true>(a, mt, x0, y, z, lane > 0 && col > 0);
+    e_group<T, W, true, false, SRC, FMA>(a, mt, x0, y, z, lane > 0 && col > 0);
 }
 
-template <typename T, int W, bool SRC>
+template <typename T, int W, bool SRC, bool FMA>
 __global__ void __launch_bounds__(256) k_e3_all(StepArgs<T> a, Box3 b, SlabMap m, int nib, int nsbp, int nm0, int nm1, int nm2) {
     __shared__ MatLds<T> mt[3][CHIML_MAX_MAT];
     const int nm[3] = {nm0, nm1, nm2};
     load_mat(a, mt, nm);
-    e3_all_sweep<T, W, SRC>(a, mt, b, m, nib, nsbp, blockIdx.x);
+    e3_all_sweep<T, W, SRC, FMA>(a, mt, b, m, nib, nsbp, blockIdx.x);
 }
 
 // ------------------------------------------------------- fused 3D step ----
@@ -1567,7 +1623,7 @@ __global__ void __launch_bounds__(kFusedMaxThreads) k_fused3(StepArgs<T> a, Fuse
     load_mat(a, mt, nm);  // (its barrier also publishes the source and profile tables)
     const T chv[3] = {a.ch[0][0], a.ch[1][0], a.ch[2][0]};
     const int nx = a.nx, ny = a.ny, nz = a.nz;
-    const int item = static_cast<int>(xcd_block(blockIdx.x, gridDim.x));
+    const int item = xcd_block(blockIdx.x, gridDim.x);
     const int tile = item / m.nseg, seg = item - tile * m.nseg;
     const int z0 = seg * m.lz, z1 = min(z0 + m.lz, nz);
     const int tid = threadIdx.x;
@@ -1666,24 +1722,24 @@ __device__ __forceinline__ void store_point(const SampleArgs<T>& a, int t, doubl
 // x-slab membership is uniform within a group as in 3D).
 template <typename T, int W, bool SRC>
 __device__ __forceinline__ void h2v_sweep(const StepArgs<T>& a, int bx, int nb) {
-    const int nx = a.nx, ny = a.ny, gx = nx / W;
-    const long long t = xcd_block(bx, nb) * blockDim.x + threadIdx.x;
-    if (t >= static_cast<long long>(gx) * ny) return;
-    const int y = static_cast<int>(t / gx), x0 = static_cast<int>(t - static_cast<long long>(y) * gx) * W;
-    const long long i = x0 + static_cast<long long>(nx) * y;
+    const int nx = a.nx, ny = a.ny, px = a.px, gx = px / W;
+    const unsigned t = static_cast<unsigned>(xcd_block(bx, nb)) * blockDim.x + threadIdx.x;
+    const int y = static_cast<int>(t / static_cast<unsigned>(gx)), x0 = static_cast<int>(t - static_cast<unsigned>(y) * gx) * W;
+    if (y >= ny) return;
+    const long long i = x0 + static_cast<long long>(px) * y;
     const T* Ez = a.F[2];
     const Pk<T, W> ez = ldv<T, W>(Ez + i);
     const bool last = x0 + W >= nx;
-    const unsigned all = (1u << W) - 1, vx = last ? (all >> 1) : all;
+    const unsigned all = (1u << W) - 1, vx = cells_below_last<W>(x0, nx);
     const bool src = SRC && group_has_src<T, W>(a, x0, y, 0);
     const int step = src ? step_now(a.step, a.stepv) : 0;
     T d[W], term[W];
     if (y < ny - 1) {  // Hx += ch [-dEz/dy]
-        const Pk<T, W> ezy = ldv<T, W>(Ez + i + nx);
+        const Pk<T, W> ezy = ldv<T, W>(Ez + i + px);
         Pk<T, W> h = ldv<T, W>(a.F[3] + i);
 #pragma unroll
         for (int w = 0; w < W; ++w) d[w] = ezy.v[w] - ez.v[w];
-        pml_group<T, W>(a.pml[3], 1, y, x0, y, 0, nx, ny, d, a.inv_d[1], all, term);
+        pml_group<T, W>(a.pml[3], 1, y, x0, y, 0, px, ny, d, a.inv_d[1], all, term);
         const T ch = a.ch[0][0];
 #pragma unroll
         for (int w = 0; w < W; ++w) {
@@ -1698,7 +1754,7 @@ __device__ __forceinline__ void h2v_sweep(const StepArgs<T>& a, int bx, int nb) 
         Pk<T, W> h = ldv<T, W>(a.F[4] + i);
 #pragma unroll
         for (int w = 0; w < W; ++w) d[w] = (w + 1 < W ? ez.v[w + 1] : ezn) - ez.v[w];
-        pml_group<T, W>(a.pml[4], 0, x0, x0, y, 0, nx, ny, d, a.inv_d[0], vx, term);
+        pml_group<T, W>(a.pml[4], 0, x0, x0, y, 0, px, ny, d, a.inv_d[0], vx, term);
         const T ch = a.ch[1][0];
 #pragma unroll
         for (int w = 0; w < W; ++w) {
@@ -1722,14 +1778,14 @@ __global__ void __launch_bounds__(256) k_h2v(StepArgs<T> a) {
 // no separate sample launch (2D decks without flux boxes and with few points).
 template <typename T, int W, bool SRC, bool DET>
 __device__ __forceinline__ void e2v_sweep(const StepArgs<T>& a, const SampleArgs<T>& sa, const MatLds<T> (*mt)[CHIML_MAX_MAT], int bx, int nb) {
-    const int nx = a.nx, ny = a.ny, gx = nx / W;
-    const long long t = xcd_block(bx, nb) * blockDim.x + threadIdx.x;
-    if (t >= static_cast<long long>(gx) * ny) return;
-    const int y = static_cast<int>(t / gx), x0 = static_cast<int>(t - static_cast<long long>(y) * gx) * W;
-    const long long i = x0 + static_cast<long long>(nx) * y;
+    const int ny = a.ny, px = a.px, gx = px / W;
+    const unsigned t = static_cast<unsigned>(xcd_block(bx, nb)) * blockDim.x + threadIdx.x;
+    const int y = static_cast<int>(t / static_cast<unsigned>(gx)), x0 = static_cast<int>(t - static_cast<unsigned>(y) * gx) * W;
+    if (y >= ny) return;
+    const long long i = x0 + static_cast<long long>(px) * y;
     const T *Hx = a.F[3], *Hy = a.F[4];
     const Pk<T, W> hx = ldv<T, W>(Hx + i), hy = ldv<T, W>(Hy + i);
-    const Pk<T, W> hxy = y > 0 ? ldv<T, W>(Hx + i - nx) : zpk<T, W>();
+    const Pk<T, W> hxy = y > 0 ? ldv<T, W>(Hx + i - px) : zpk<T, W>();
     const T hym = x0 > 0 ? Hy[i - 1] : T(0);
     const unsigned all = (1u << W) - 1;
     const bool src = SRC && group_has_src<T, W>(a, x0, y, 0);
@@ -1740,9 +1796,12 @@ __device__ __forceinline__ void e2v_sweep(const StepArgs<T>& a, const SampleArgs
         d1[w] = hy.v[w] - (w > 0 ? hy.v[w - 1] : hym);
         d2[w] = hx.v[w] - hxy.v[w];
     }
-    pml_group<T, W>(a.pml[2], 0, x0, x0, y, 0, nx, ny, d1, a.inv_d[0], all, t1);
-    pml_group<T, W>(a.pml[2], 1, y, x0, y, 0, nx, ny, d2, a.inv_d[1], all, t2);
-    const Pk<T, W> ez = e_finish_group<T, W>(a, mt, 2, i, x0, y, 0, all, t1, t2, src, step);
+    pml_group<T, W>(a.pml[2], 0, x0, x0, y, 0, px, ny, d1, a.inv_d[0], all, t1);
+    pml_group<T, W>(a.pml[2], 1, y, x0, y, 0, px, ny, d2, a.inv_d[1], all, t2);
+    T acc[W];
+    const unsigned plain = a.fma_curl && y >= a.Tp[1] && y < ny - a.Tp[1] ? cells_inside<W>(x0, a.nx, a.Tp[0]) : 0u;
+    curl_of<T, W, true>(t1, t2, d2, a.inv_d[1], plain, acc);
+    const Pk<T, W> ez = e_finish_group<T, W>(a, mt, 2, i, x0, y, 0, all, acc, src, step);
     if (DET) {
         const int st = step_now(a.step, a.stepv) + 1;
         for (int p = 0; p < sa.totpts; ++p) {
@@ -2515,7 +2574,7 @@ struct BatchSlot {
     SampleArgs<T> s;
     Box3 b;
     SlabMap m;
-    int nib, nsbp, ade_bpc;
+    int nib, nsbp, ade_bpc, fma;
     int nm[3];
     int nblk[5];  // blocks of each phase launch (unpadded)
 };
@@ -2560,7 +2619,8 @@ __global__ void __launch_bounds__(256) k_bh3_all(const BatchSlot<T>* __restrict_
     const int bx = blockIdx.x - begin[k];
     const BatchSlot<T>& q = sl[k];
     if (bx >= q.nblk[kPhH]) return;
-    h3_all_sweep<T, W, true>(q.a, q.b, q.m, q.nib, q.nsbp, q.ade_bpc, bx);
+    if (q.fma) h3_all_sweep<T, W, true, true>(q.a, q.b, q.m, q.nib, q.nsbp, q.ade_bpc, bx);
+    else h3_all_sweep<T, W, true, false>(q.a, q.b, q.m, q.nib, q.nsbp, q.ade_bpc, bx);
     advance_counter_at(q.a, bx);
 }
 
@@ -2572,7 +2632,8 @@ __global__ void __launch_bounds__(256) k_be3_all(const BatchSlot<T>* __restrict_
     const BatchSlot<T>& q = sl[k];
     if (bx >= q.nblk[kPhE]) return;
     load_mat(q.a, mt, q.nm);
-    e3_all_sweep<T, W, true>(q.a, mt, q.b, q.m, q.nib, q.nsbp, bx);
+    if (q.fma) e3_all_sweep<T, W, true, true>(q.a, mt, q.b, q.m, q.nib, q.nsbp, bx);
+    else e3_all_sweep<T, W, true, false>(q.a, mt, q.b, q.m, q.nib, q.nsbp, bx);
 }
 
 template <typename T, int W>
@@ -2651,6 +2712,8 @@ struct chiml_dev {
     int device = 0;
     int prec = 64;
     int nx = 0, ny = 0, nz = 0, dim = 3;
+    int px = 0;         // cells per stored x row (StepArgs::px)
+    bool vec = false;   // rows hold whole W-cell groups and the x psi regions are whole groups: the W-cell kernels apply
     int nsteps = 0, steps_done = 0;
     std::vector<std::unique_ptr<DevBuf>> bufs;
     DevBuf step_ctr;
@@ -2668,6 +2731,9 @@ struct chiml_dev {
     bool device_flush = false;  // launch the DFT flush every step; it decides on the device
     hipGraphExec_t gexec = nullptr;
     bool split = false;  // 3D interior + CPML-slab kernels
+    bool rows = false;   // split: whole-row interior, one launch per field
+    bool cellwise = false;  // split, but stepped alone with one thread per cell (GridLayout::cellwise)
+    bool fma_curl = false;  // rows or x CPML no whole groups: curls as the per-cell kernels round them (curl_of)
     bool fused = false;  // 3D: one fused H + E launch per step on ping-pong buffers
     FuseMap fmap{};
     size_t fused_lds = 0;  // dynamic LDS of the fused launch (bytes)
@@ -2780,13 +2846,13 @@ void build_cells(chiml_dev* c, const chiml_problem_t* p) {
     if (n == 0) return;
     const bool is3 = p->nz > 1;
     std::vector<std::pair<long long, int>> key(n);  // (component * points + point, position in the list)
-    const long long npt = static_cast<long long>(p->nx) * p->ny * p->nz;
+    const long long npt = static_cast<long long>(c->px) * p->ny * p->nz;
     for (int k = 0; k < n; ++k) {
         const int cc = p->cell_comp[k], x = p->cell_xyz[3 * k], y = p->cell_xyz[3 * k + 1], z = p->cell_xyz[3 * k + 2];
         if (cc < 0 || cc > 5 || (!is3 && cc != 2 && cc != 3 && cc != 4)) throw std::runtime_error("per-cell source on a missing component");
         if (x < 0 || x >= p->nx || y < 0 || y >= p->ny || z < 0 || z >= p->nz) throw std::runtime_error("per-cell source outside the grid");
         if (p->cell_col[k] < 0 || p->cell_col[k] >= p->ncell_col) throw std::runtime_error("per-cell source column out of range");
-        key[k] = {cc * npt + x + static_cast<long long>(p->nx) * (y + static_cast<long long>(p->ny) * z), k};
+        key[k] = {cc * npt + x + static_cast<long long>(c->px) * (y + static_cast<long long>(p->ny) * z), k};
     }
     std::stable_sort(key.begin(), key.end(), [](const auto& a, const auto& b) { return a.first < b.first; });
     std::vector<int> comp(n), col(n);
@@ -2937,16 +3003,53 @@ void build_tfsf(chiml_dev* c, const chiml_problem_t* p, const StepArgs<T>& a) {
 template <typename T>
 void build(chiml_dev* c, const chiml_problem_t* p, StepArgs<T>& a, SampleArgs<T>& s) {
     const int nx = p->nx, ny = p->ny, nz = p->nz;
-    const size_t N = static_cast<size_t>(nx) * ny * nz;
     a.nx = nx;
     a.ny = ny;
     a.nz = nz;
+    {
+        int lo = p->pml_T[0], hi = nx - p->pml_T[0];
+        bool hmap = false;
+        for (int comp = 0; comp < 6; ++comp) {
+            if (p->pml_b[comp][0]) {
+                lo = std::max(lo, p->psi_lo[comp][0]);
+                hi = std::min(hi, p->psi_hi0[comp][0]);
+            }
+            if (comp < 3 && (nz > 1 || comp < 2) && p->mat_h[comp]) hmap = true;
+        }
+        const GridLayout gl = grid_layout(nx, ny, nz, p->pml_T, lo, hi, sizeof(T) == 4, hmap);
+        c->vec = gl.vec;
+        c->px = gl.px;
+        c->split = gl.split;
+        c->rows = gl.rows;
+        c->cellwise = gl.cellwise;
+        c->fma_curl = nx % gl.W != 0 || p->pml_T[0] % gl.W != 0;
+        a.fma_curl = c->fma_curl ? 1 : 0;
+    }
+    const int px = c->px, rw = c->vec ? static_cast<int>(16 / sizeof(T)) : 1;
+    a.px = px;
+    const size_t N = static_cast<size_t>(px) * ny * nz;
+    // a grid point's place in the padded rows (-1, the zero ghost, stays)
+    auto padded = [&](long long i) { return i < 0 ? i : i / nx * px + i % nx; };
+    auto padded_cells = [&](const long long* src, size_t n) {
+        std::vector<long long> r(n);
+        for (size_t i = 0; i < n; ++i) r[i] = padded(src[i]);
+        return r;
+    };
+    // uploads a per-point array into padded rows
+    auto upload_rows = [&](auto* src, auto fill) {
+        using V = std::remove_const_t<std::remove_pointer_t<decltype(src)>>;
+        if (px == nx) return c->upload<V>(src, N);
+        std::vector<V> r(N, static_cast<V>(fill));
+        const size_t nr = static_cast<size_t>(ny) * nz;
+        for (size_t y = 0; y < nr; ++y) std::copy(src + y * nx, src + (y + 1) * nx, r.begin() + y * px);
+        return c->upload<V>(r.data(), N);
+    };
     for (int k = 0; k < 3; ++k) {
         a.inv_d[k] = static_cast<T>(1.0 / p->d[k]);
         a.Tp[k] = p->pml_T[k];
     }
     const bool is3 = nz > 1;
-    {  // the present components in one allocation, x + nx (y + ny z) each, in component order
+    {  // the present components in one allocation, x + px (y + ny z) each, in component order
         int nf = 0;
         for (int k = 0; k < 6; ++k) nf += (is3 || k == 2 || k == 3 || k == 4) ? 1 : 0;
         T* base = c->zeros<T>(N * nf);
@@ -2958,7 +3061,7 @@ void build(chiml_dev* c, const chiml_problem_t* p, StepArgs<T>& a, SampleArgs<T>
     }
     for (int k = 0; k < 3; ++k) {
         bool present = is3 || k == 2;
-        a.mat_e[k] = (present && p->mat_e[k]) ? c->upload<uint8_t>(p->mat_e[k], N) : nullptr;
+        a.mat_e[k] = (present && p->mat_e[k]) ? upload_rows(p->mat_e[k], 0) : nullptr;
         int nm = present ? p->nmat_e[k] : 1;
         if (present && (nm <= 0 || nm > CHIML_MAX_MAT)) throw std::runtime_error("material table size out of range");
         if (present) {
@@ -2969,7 +3072,7 @@ void build(chiml_dev* c, const chiml_problem_t* p, StepArgs<T>& a, SampleArgs<T>
             c->nmat[k] = nm;
         }
         bool hpresent = is3 || k < 2;
-        a.mat_h[k] = (hpresent && p->mat_h[k]) ? c->upload<uint8_t>(p->mat_h[k], N) : nullptr;
+        a.mat_h[k] = (hpresent && p->mat_h[k]) ? upload_rows(p->mat_h[k], 0) : nullptr;
         if (hpresent) {
             int nh = p->nmat_h[k] > 0 ? p->nmat_h[k] : 1;
             a.ch[k] = upload_cast<T>(c, p->mat_h_ch[k], nh);
@@ -2995,7 +3098,7 @@ void build(chiml_dev* c, const chiml_problem_t* p, StepArgs<T>& a, SampleArgs<T>
         // storage belongs to cells without poles and is never changed)
         if (a.box[k][1] > a.box[k][0]) {
             a.box[k][0] = a.box[k][0] / 4 * 4;
-            a.box[k][1] = std::min((a.box[k][1] + 3) / 4 * 4, nx);
+            a.box[k][1] = std::min((a.box[k][1] + 3) / 4 * 4, px);
         }
         long long bn = 0;  // cells of the (aligned) pole-state box
         if (a.box[k][1] > a.box[k][0] && a.box[k][3] > a.box[k][2] && a.box[k][5] > a.box[k][4])
@@ -3020,16 +3123,20 @@ void build(chiml_dev* c, const chiml_problem_t* p, StepArgs<T>& a, SampleArgs<T>
             // Widen the psi region to whole slabs [0, T) and [n - T, n): the
             // added positions carry b = 0, c/d = 0, 1/kappa = 1, for which the
             // CPML term equals the plain dV/d bit for bit and psi stays 0.
-            const int n = nn[ax], T0 = p->pml_T[ax];
+            // Along x also to whole W-cell groups and over the row padding.
+            const int n = nn[ax], T0 = p->pml_T[ax], ns = ax == 0 ? px : n, w = ax == 0 ? rw : 1;
             const int lo = p->psi_lo[comp][ax], hi0 = p->psi_hi0[comp][ax], hi1 = p->psi_hi1[comp][ax];
-            pm.lo[ax] = std::max(lo, T0);
-            pm.hi0[ax] = std::min(hi0, n - T0);
-            pm.hi1[ax] = std::max(hi1, n);
+            pm.lo[ax] = round_up(std::max(lo, T0), w);
+            pm.hi0[ax] = round_down(std::min(hi0, n - T0), w);
+            pm.hi1[ax] = std::max(hi1, ns);
             pm.S[ax] = pm.lo[ax] + (pm.hi1[ax] - pm.hi0[ax]);
             std::vector<double> bb(p->pml_b[comp][ax], p->pml_b[comp][ax] + n), cc(p->pml_cd[comp][ax], p->pml_cd[comp][ax] + n),
                 kk(p->pml_kinv[comp][ax], p->pml_kinv[comp][ax] + n);
+            bb.resize(ns, 0.0);
+            cc.resize(ns, 0.0);
+            kk.resize(ns, 1.0);
             auto ident = [&](int q0, int q1) {
-                for (int q = std::max(q0, 0); q < std::min(q1, n); ++q) {
+                for (int q = std::max(q0, 0); q < std::min(q1, ns); ++q) {
                     bb[q] = 0.0;
                     cc[q] = 0.0;
                     kk[q] = 1.0;
@@ -3038,12 +3145,12 @@ void build(chiml_dev* c, const chiml_problem_t* p, StepArgs<T>& a, SampleArgs<T>
             ident(lo, pm.lo[ax]);
             ident(pm.hi0[ax], hi0);
             ident(hi1, pm.hi1[ax]);
-            pm.b[ax] = upload_cast<T>(c, bb.data(), n);
-            pm.cd[ax] = upload_cast<T>(c, cc.data(), n);
-            pm.kinv[ax] = upload_cast<T>(c, kk.data(), n);
+            pm.b[ax] = upload_cast<T>(c, bb.data(), ns);
+            pm.cd[ax] = upload_cast<T>(c, cc.data(), ns);
+            pm.kinv[ax] = upload_cast<T>(c, kk.data(), ns);
             size_t ps = static_cast<size_t>(pm.S[ax]);
             for (int o = 0; o < 3; ++o)
-                if (o != ax) ps *= nn[o];
+                if (o != ax) ps *= o == 0 ? px : nn[o];
             pm.psi[ax] = ps ? c->zeros<T>(ps) : nullptr;
         }
     }
@@ -3090,7 +3197,7 @@ void build(chiml_dev* c, const chiml_problem_t* p, StepArgs<T>& a, SampleArgs<T>
         s.det_npts = c->upload<int>(p->det_npts, p->ndet);
         s.det_off = c->upload<int>(off.data(), p->ndet + 1);
         s.det_comp = c->upload<int>(p->det_comp, 2 * static_cast<size_t>(eoff[p->ndet]));
-        s.det_cell = c->upload<long long>(p->det_cell, 2 * static_cast<size_t>(eoff[p->ndet]));
+        s.det_cell = c->upload<long long>(padded_cells(p->det_cell, 2 * static_cast<size_t>(eoff[p->ndet])).data(), 2 * static_cast<size_t>(eoff[p->ndet]));
         s.det_nf = c->upload<int>(nf.data(), p->ndet);
         s.det_eoff = c->upload<long long>(eoff.data(), p->ndet + 1);
         c->det_single_field = std::all_of(nf.begin(), nf.end(), [](int v) { return v == 1; });
@@ -3128,7 +3235,7 @@ void build(chiml_dev* c, const chiml_problem_t* p, StepArgs<T>& a, SampleArgs<T>
         ds.stage = nullptr;
         if (n > 0) {
             ds.comp = c->upload<int>(comp, n);
-            ds.cell = c->upload<long long>(cell, n);
+            ds.cell = c->upload<long long>(padded_cells(cell, n).data(), n);
             T* st = c->zeros<T>(static_cast<size_t>(kDftBlock) * n);
             ds.stage = st;
             d.stage = st;
@@ -3143,7 +3250,7 @@ void build(chiml_dev* c, const chiml_problem_t* p, StepArgs<T>& a, SampleArgs<T>
     s.ndft = c->ndft;
     // emitters
     const double* epsn = nullptr;
-    if (p->nqe > 0) epsn = c->upload<double>(p->eps_node, N);
+    if (p->nqe > 0) epsn = upload_rows(p->eps_node, 1.0);
     for (int g = 0; g < p->nqe; ++g) {
         const chiml_qe_t& qi = p->qe[g];
         QeHost qh;
@@ -3321,7 +3428,7 @@ void launch_tfsf(chiml_dev* c, StepArgs<T>& a) {
         const TfsfLineArgs& t = h.line;
         if (h.toth > 0)
             hipLaunchKernelGGL(k_tfsf_add<T>, dim3(static_cast<unsigned>((h.toth + 255) / 256)), dim3(256), 0, c->stream, h.surf, h.nsh,
-                               h.toth, a.F[0], a.F[1], a.F[2], a.F[3], a.F[4], a.F[5], t.line[0], t.len[0], c->nx, c->ny);
+                               h.toth, a.F[0], a.F[1], a.F[2], a.F[3], a.F[4], a.F[5], t.line[0], t.len[0], c->px, c->ny);
         const size_t lds = tfsf_lds_bytes(t);
         if (lds <= kTfsfMaxLds)
             hipLaunchKernelGGL(k_tfsf_line<true>, dim3(1), dim3(1024), lds, c->stream, t, a.step, a.stepv);
@@ -3329,7 +3436,7 @@ void launch_tfsf(chiml_dev* c, StepArgs<T>& a) {
             hipLaunchKernelGGL(k_tfsf_line<false>, dim3(1), dim3(1024), 0, c->stream, t, a.step, a.stepv);
         if (h.tote > 0)
             hipLaunchKernelGGL(k_tfsf_add<T>, dim3(static_cast<unsigned>((h.tote + 255) / 256)), dim3(256), 0, c->stream, h.surf + h.nsh,
-                               h.nse, h.tote, a.F[0], a.F[1], a.F[2], a.F[3], a.F[4], a.F[5], t.line[0], t.len[0], c->nx, c->ny);
+                               h.nse, h.tote, a.F[0], a.F[1], a.F[2], a.F[3], a.F[4], a.F[5], t.line[0], t.len[0], c->px, c->ny);
     }
 }
 
@@ -3370,34 +3477,38 @@ void launch_fields(chiml_dev* c, StepArgs<T>& a) {
         });
         return;
     }
-    if (DIM == 3 && c->split) {
+    if (DIM == 3 && c->split && !c->cellwise) {
         constexpr int W = 16 / sizeof(T);
         const Box3 b = c->ibox;
         const int nyb = b.y1 - b.y0, by = b.by > 0 ? b.by : nyb;
         const long long ni = static_cast<long long>((b.x1 - b.x0) / W) * by * (b.z1 - b.z0) * ((nyb + by - 1) / by);
-        const long long ns = c->slab.nA + c->slab.nB + c->slab.nC;
+        const long long ns = static_cast<long long>(c->slab.nA) + c->slab.nB + c->slab.nC;
         const dim3 gi(static_cast<unsigned>((ni + 255) / 256)), gs(static_cast<unsigned>((ns + 255) / 256)), blk(256);
         const int nib = static_cast<int>(gi.x), ade_bpc = static_cast<int>((c->ade_groups + 255) / 256);
-        if constexpr (W == 4) {  // FP32: one launch per field
+        if (c->rows) {  // one launch per field
             const int nsbp = static_cast<int>((gs.x + 7) / 8 * 8);
             const dim3 gh(static_cast<unsigned>(ade_blocks(ade_bpc) + nsbp + nib)), ge(static_cast<unsigned>(nsbp + nib));
             if (gh.x > 0) {
                 Timed t(c, "update_h");
                 pick2(c->has_src, adv, [&](auto S, auto A) {
-                    hipLaunchKernelGGL((k_h3_all<T, W, decltype(S)::value, decltype(A)::value>), gh, blk, 0, c->stream, a, b, c->slab,
-                                       nib, nsbp, ade_bpc);
+                    auto go = [&](auto M) {
+                        hipLaunchKernelGGL((k_h3_all<T, W, decltype(S)::value, decltype(A)::value, decltype(M)::value>), gh, blk, 0, c->stream, a,
+                                           b, c->slab, nib, nsbp, ade_bpc);
+                    };
+                    if (c->fma_curl) go(std::true_type{});
+                    else go(std::false_type{});
                 });
             }
             launch_tfsf<T>(c, a);
             launch_cells<T>(c, a);
             if (ge.x > 0) {
                 Timed t(c, "update_e");
-                if (c->has_src)
-                    hipLaunchKernelGGL((k_e3_all<T, W, true>), ge, blk, 0, c->stream, a, b, c->slab, nib, nsbp, c->nmat[0], c->nmat[1], c->nmat[2]);
-                else
-                    hipLaunchKernelGGL((k_e3_all<T, W, false>), ge, blk, 0, c->stream, a, b, c->slab, nib, nsbp, c->nmat[0], c->nmat[1], c->nmat[2]);
+                pick2(c->has_src, c->fma_curl, [&](auto S, auto M) {
+                    hipLaunchKernelGGL((k_e3_all<T, W, decltype(S)::value, decltype(M)::value>), ge, blk, 0, c->stream, a, b, c->slab, nib, nsbp,
+                                       c->nmat[0], c->nmat[1], c->nmat[2]);
+                });
             }
-        } else {  // FP64: the pole update rides on the H interior launch as its first blocks
+        } else if constexpr (W == 2) {  // FP64: the pole update rides on the H interior launch as its first blocks
             const dim3 gh(static_cast<unsigned>(nib + ade_blocks(ade_bpc)));
             if (gh.x > 0) {
                 Timed t(c, "update_h");
@@ -3428,7 +3539,7 @@ void launch_fields(chiml_dev* c, StepArgs<T>& a) {
     }
     if (DIM == 2 && c->vec2d) {
         constexpr int W = 16 / sizeof(T);
-        const long long ng = static_cast<long long>(c->nx / W) * c->ny;
+        const long long ng = static_cast<long long>(c->px / W) * c->ny;
         const dim3 g(static_cast<unsigned>((ng + 255) / 256)), blk(256);
         {
             Timed t(c, "update_h");
@@ -3476,7 +3587,7 @@ void launch_ml(chiml_dev* c, StepArgs<T>& a) {
         int ex = q.bn[0] + 1, ey = q.bn[1] + 1, ez = (q.dim == 3) ? q.bn[2] + 1 : 1;
         int n = ex * ey * ez;
         if (!q.fold_addp)
-            hipLaunchKernelGGL(k_ml_addp<T>, dim3((n + 255) / 256, 3), dim3(256), 0, c->stream, q, a.F[0], a.F[1], a.F[2], c->nx, c->ny,
+            hipLaunchKernelGGL(k_ml_addp<T>, dim3((n + 255) / 256, 3), dim3(256), 0, c->stream, q, a.F[0], a.F[1], a.F[2], c->px, c->ny,
                                c->nz);
         dim3 g(qh.nblocks);
         {
@@ -3485,10 +3596,10 @@ void launch_ml(chiml_dev* c, StepArgs<T>& a) {
 #define CHIML_ML_TEAM(NN)                                                                                                       \
     case NN:                                                                                                                    \
         if (q.packed)                                                                                                           \
-            hipLaunchKernelGGL((k_ml_team<T, NN, true>), g, dim3(kMlThreads), 0, c->stream, q, a.F[0], a.F[1], a.F[2], c->nx, c->ny, \
+            hipLaunchKernelGGL((k_ml_team<T, NN, true>), g, dim3(kMlThreads), 0, c->stream, q, a.F[0], a.F[1], a.F[2], c->px, c->ny, \
                                c->nz, a.step, a.stepv);                                                                         \
         else                                                                                                                    \
-            hipLaunchKernelGGL((k_ml_team<T, NN, false>), g, dim3(kMlThreads), 0, c->stream, q, a.F[0], a.F[1], a.F[2], c->nx, c->ny, \
+            hipLaunchKernelGGL((k_ml_team<T, NN, false>), g, dim3(kMlThreads), 0, c->stream, q, a.F[0], a.F[1], a.F[2], c->px, c->ny, \
                                c->nz, a.step, a.stepv);                                                                         \
         break;
                 CHIML_ML_TEAM(2)
@@ -3629,7 +3740,7 @@ void* scratch_on(int dev) {
 int batch_class(const chiml_dev* c) {
     if (c->fused || c->capturing || !c->tfsf.empty() || c->cells.n > 0) return 0;  // TFSF and per-cell source steps stay on their own stream
     if (c->dim == 2 && c->vec2d) return 1;
-    if (c->dim == 3 && c->split) return 2;
+    if (c->dim == 3 && c->split && c->rows == (c->prec == 32)) return 2;
     return 0;
 }
 
@@ -3655,13 +3766,14 @@ BatchSlot<T> make_slot(chiml_dev* c, int p) {
     q.s.stepv = -1;
     for (int k = 0; k < 3; ++k) q.nm[k] = c->nmat[k];
     if (c->dim == 2) {
-        const long long ng = static_cast<long long>(c->nx / W) * c->ny;
+        const long long ng = static_cast<long long>(c->px / W) * c->ny;
         q.nblk[kPhH] = q.nblk[kPhE] = static_cast<int>((ng + 255) / 256);
     } else {
         const Box3 b = c->ibox;
         const int nyb = b.y1 - b.y0, by = b.by > 0 ? b.by : nyb;
         const long long ni = static_cast<long long>((b.x1 - b.x0) / W) * by * (b.z1 - b.z0) * ((nyb + by - 1) / by);
-        const long long ns = c->slab.nA + c->slab.nB + c->slab.nC;
+        const long long ns = static_cast<long long>(c->slab.nA) + c->slab.nB + c->slab.nC;
+        q.fma = c->fma_curl ? 1 : 0;
         q.b = b;
         q.m = c->slab;
         q.nib = static_cast<int>((ni + 255) / 256);
@@ -3967,7 +4079,7 @@ int chiml_dev_create(const chiml_problem_t* p, chiml_dev_t** out) {
         else build<double>(c.get(), p, c->a64, c->s64);
         if (c->dim == 2) {
             const int W = c->prec == 32 ? 4 : 2;
-            c->vec2d = (p->nx % W) == 0 && (p->pml_T[0] % W) == 0 && !c->hmap;
+            c->vec2d = c->vec;
             // the E kernel samples the point detectors when each point reads one
             // cell of Ez, Hx or Hy and there are few of them (every thread scans
             // the list), no flux box needs the sample launch anyway, no emitter
@@ -3984,29 +4096,23 @@ int chiml_dev_create(const chiml_problem_t* p, chiml_dev_t** out) {
         }
         if (c->dim == 3) {
             const int Tx = p->pml_T[0], Ty = p->pml_T[1], Tz = p->pml_T[2];
-            // FP32 (W = 4): the interior walk takes whole x rows of the y/z
-            // interior (one wavefront per 256-cell row, the x slabs' CPML terms
-            // applied inline) and the slab region covers the z and y slabs.
-            // FP64 (W = 2): the x slabs stay in the slab region, which measured
-            // faster there.
-            const bool rows = c->prec == 32;
-            Box3 b{rows ? 0 : Tx, rows ? p->nx : p->nx - Tx, Ty, p->ny - Ty, Tz, p->nz - Tz, 0};
+            // rows: the interior walk takes whole x rows of the y/z interior
+            // (the x slabs' CPML terms applied inline) and the slab region
+            // covers the z and y slabs; else the x slabs stay in the slab region.
+            Box3 b{c->rows ? 0 : Tx, c->rows ? c->px : p->nx - Tx, Ty, p->ny - Ty, Tz, p->nz - Tz, 0};
             b.by = (b.y1 - b.y0 + 7) / 8;  // one y band per XCD
-            // the split kernels take W = 16 / sizeof(T) cells per thread along x:
-            // x rows and x slabs must hold whole groups, and there is no magnetic map
             const int W = c->prec == 32 ? 4 : 2;
-            if (b.x1 > b.x0 && b.y1 > b.y0 && b.z1 > b.z0 && (Tx % W) == 0 && (p->nx % W) == 0 && !c->hmap) {
-                c->split = true;
+            if (c->split) {
                 c->ibox = b;
                 if (c->prec == 32) enable_fused<float>(c.get(), p, c->a32, c->s32);
                 SlabMap& m = c->slab;
-                m.nx = p->nx; m.ny = p->ny; m.nz = p->nz;
+                m.nx = c->px; m.ny = p->ny; m.nz = p->nz;
                 m.Tx = Tx; m.Ty = Ty; m.Tz = Tz;
                 m.W = W;
-                const long long gx = p->nx / W;
-                m.nA = 2LL * Tz * gx * p->ny;
-                m.nB = 2LL * Ty * gx * (p->nz - 2 * Tz);
-                m.nC = rows ? 0 : 2LL * (Tx / W) * (p->ny - 2 * Ty) * (p->nz - 2 * Tz);
+                const long long gx = c->px / W;
+                m.nA = static_cast<unsigned>(2LL * Tz * gx * p->ny);
+                m.nB = static_cast<unsigned>(2LL * Ty * gx * (p->nz - 2 * Tz));
+                m.nC = c->rows ? 0 : static_cast<unsigned>(2LL * (Tx / W) * (p->ny - 2 * Ty) * (p->nz - 2 * Tz));
 
                 for (int k = 0; k < 3; ++k) {
                     const int* bx = c->prec == 32 ? c->a32.box[k] : c->a64.box[k];
@@ -4125,18 +4231,26 @@ int chiml_dev_sync(chiml_dev_t* c) {
 
 int chiml_dev_read_field(chiml_dev_t* c, int comp, double* host) {
     if (!c || !host || comp < 0 || comp > 5) return fail(c, CHIML_E_INVALID, "invalid argument");
-    size_t N = static_cast<size_t>(c->nx) * c->ny * c->nz;
+    const size_t nr = static_cast<size_t>(c->ny) * c->nz, N = static_cast<size_t>(c->nx) * nr, Np = static_cast<size_t>(c->px) * nr;
     std::lock_guard<std::mutex> lk(g_capture_mu);
     try {
         HIP_TRY(hipStreamSynchronize(c->stream));
+        if (!(c->prec == 32 ? static_cast<void*>(c->a32.F[comp]) : static_cast<void*>(c->a64.F[comp]))) {
+            std::memset(host, 0, N * sizeof(double));
+            return CHIML_OK;
+        }
+        // rows leave their padding behind
         if (c->prec == 32) {
-            if (!c->a32.F[comp]) { std::memset(host, 0, N * sizeof(double)); return CHIML_OK; }
-            std::vector<float> tmp(N);
-            HIP_TRY(hipMemcpy(tmp.data(), c->a32.F[comp], N * sizeof(float), hipMemcpyDeviceToHost));
-            for (size_t i = 0; i < N; ++i) host[i] = tmp[i];
-        } else {
-            if (!c->a64.F[comp]) { std::memset(host, 0, N * sizeof(double)); return CHIML_OK; }
+            std::vector<float> tmp(Np);
+            HIP_TRY(hipMemcpy(tmp.data(), c->a32.F[comp], Np * sizeof(float), hipMemcpyDeviceToHost));
+            for (size_t r = 0; r < nr; ++r)
+                for (int x = 0; x < c->nx; ++x) host[r * c->nx + x] = tmp[r * c->px + x];
+        } else if (c->px == c->nx) {
             HIP_TRY(hipMemcpy(host, c->a64.F[comp], N * sizeof(double), hipMemcpyDeviceToHost));
+        } else {
+            std::vector<double> tmp(Np);
+            HIP_TRY(hipMemcpy(tmp.data(), c->a64.F[comp], Np * sizeof(double), hipMemcpyDeviceToHost));
+            for (size_t r = 0; r < nr; ++r) std::copy(tmp.data() + r * c->px, tmp.data() + r * c->px + c->nx, host + r * c->nx);
         }
     } catch (std::exception& e) {
         return fail(c, CHIML_E_HIP, e.what());

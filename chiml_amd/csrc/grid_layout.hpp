@@ -1,0 +1,46 @@
+// How a grid is stored and swept on the device, shared by the device layer
+// and the manager's byte accounting.
+#pragma once
+
+// Rows along x are stored in whole groups of W = 16 / sizeof(T) cells (one
+// 16-byte access each) and the x CPML's psi regions are widened to whole
+// groups with identity coefficients, so grids and slabs of any size take the
+// W-cell kernels.  The padding cells of a row stay zero.
+struct GridLayout {
+    int W;       // cells per group
+    bool vec;    // the W-cell kernels apply (else one thread per cell, rows as they are)
+    int px;      // stored cells per row
+    bool split;  // 3D: interior + CPML slab sweeps
+    bool rows;   // split: the interior takes whole rows (x slabs inline), H and E one launch each
+    bool cellwise;  // split, but stepped alone with one thread per cell
+};
+
+inline int round_up(int n, int w) { return (n + w - 1) / w * w; }
+inline int round_down(int n, int w) { return n / w * w; }
+
+// psi_lo / psi_hi0: the largest lower end and the smallest upper start of the
+// x psi regions over the components (T and nx - T for a CPML of T cells).
+// The W-cell form needs the two widened regions not to reach into each other's
+// unwidened part: a group belongs to one of them, or to neither.
+inline GridLayout grid_layout(int nx, int ny, int nz, const int* T, int psi_lo, int psi_hi0, bool fp32, bool hmap) {
+    GridLayout g;
+    g.W = fp32 ? 4 : 2;
+    const int lo = round_up(psi_lo, g.W), hi = round_down(psi_hi0, g.W);
+    g.vec = !hmap && lo <= hi;
+    g.px = g.vec ? round_up(nx, g.W) : nx;
+    // (the sweeps number groups in 32 bits)
+    g.split = g.vec && nz > 1 && nx > 2 * T[0] && ny > 2 * T[1] && nz > 2 * T[2] &&
+              static_cast<double>(g.px / g.W) * (ny + 8) * nz < 4.0e9;
+    const bool aligned = nx % g.W == 0 && T[0] % g.W == 0;
+    // FP64 leaves the x slabs of aligned grids to the slab sweep, which
+    // measured faster there (256^3: 0.603 against 0.619 ms per step)
+    g.rows = g.split && (fp32 || !aligned);
+    // Groups leave a small 3D grid about one wave per SIMD, each waiting for
+    // memory alone, so a small grid that had to be padded is stepped one thread
+    // per cell (FP32 64^3, 10-cell CPML: 23.5 us a step per cell, 26.2 in
+    // groups; 101x93x87: 69 and 49; FP64 65x64x63: 47 and 37); a batch of them
+    // fills the chip and takes the groups (56^3, 72^3 and 88^3 together with
+    // three 2D grids: 72 and 51 us a step).
+    g.cellwise = g.split && !aligned && static_cast<double>(nx) * ny * nz * (fp32 ? 4 : 8) < 1.5e6;
+    return g;
+}

@@ -30,6 +30,7 @@
 #include "../../include/chiml/chiml_dev.h"
 #include "../../include/chiml/chiml_out.h"
 #include "../../include/chiml/chiml_sim.h"
+#include "grid_layout.hpp"
 #include "qe_layout.hpp"
 #include "setup.hpp"
 
@@ -1614,11 +1615,12 @@ FDTDField::FDTDField(const std::string& deck) : IP(parseInputs(deck)) {
         const double nE = is3D ? 3.0 : 1.0, nH = is3D ? 3.0 : 2.0;
         cells = static_cast<double>(N);
         // interior box of the 3D split kernels (see device.hip); 2D uses one kernel each
-        const int W = IP.fp32 ? 4 : 2;  // x cells per thread of the split kernels
-        const bool split = is3D && T[0] < nx - T[0] && T[1] < ny - T[1] && T[2] < nz - T[2] && (T[0] % W) == 0 && (nx % W) == 0;
-        // interior kernel: whole x rows of the y/z interior in FP32 (x slabs
-        // included), the y/z interior without the x slabs in FP64
-        const bool rows = IP.fp32;
+        const bool hmap = P.mat_h[0] || P.mat_h[1] || P.mat_h[2];
+        const GridLayout gl = grid_layout(nx, ny, nz, T.data(), T[0], nx - T[0], IP.fp32, hmap);
+        const bool split = gl.split;
+        // interior kernel: whole x rows of the y/z interior (x slabs
+        // included), or the y/z interior without the x slabs
+        const bool rows = gl.rows;
         const double Ni = split ? static_cast<double>(rows ? nx : nx - 2 * T[0]) * (ny - 2 * T[1]) * (nz - 2 * T[2]) : cells;
         const double Ns = cells - Ni;
         auto inInt = [&](int x, int y, int z) {
@@ -2501,7 +2503,8 @@ int chiml_sim_estimate_bytes(const char* deck, size_t* bytes) {
         chiml::check_pml_axes(IP);
         auto n = IP.nVec();
         if (!IP.is3D()) n[2] = 1;
-        double cells = static_cast<double>(n[0]) * n[1] * n[2];
+        // rows are stored in whole 16-byte groups
+        double cells = static_cast<double>(round_up(n[0], IP.fp32 ? 4 : 2)) * n[1] * n[2];
         double s = IP.fp32 ? 4.0 : 8.0;
         double psi = 0.0;
         for (int a = 0; a < 3; ++a) {
