@@ -1822,6 +1822,427 @@ __global__ void __launch_bounds__(256) k_e2v(StepArgs<T> a, SampleArgs<T> sa, in
     e2v_sweep<T, W, SRC, DET>(a, sa, mt, blockIdx.x, gridDim.x);
 }
 
+// --------------------------------------------- 2D: several steps a launch ----
+// A 2D TMz grid is small: a step of 256^2 cells moves 4 MB, and launches, not
+// memory, set its time (two launches, 8.1 us a step).  k_tile2 advances up to
+// kTileSteps steps in one launch.  A block loads a tile of the grid with a
+// halo of kTileSteps cells on every side, keeps it in registers for all its
+// steps and writes the tile's own cells to the other field buffer (the
+// neighbours still read the old one); the halo cells are recomputed by every
+// block that holds them, and their outermost ring goes stale by one cell per
+// step.  A thread owns R consecutive rows of one column: the y neighbour is
+// its own register except at the ends of its strip (one row through LDS per
+// half step, one barrier each), the x neighbour is the next lane's register.
+// The CPML psi of the tile's cells are registers too, pole states are in LDS.
+// The arithmetic of a cell is that of h2v_sweep / e2v_sweep.
+//
+// A launch costs about 8 us of latency to get its tiles in and out and about
+// 0.8 us a step.  Small grids take small tiles, one or two a CU (4x the cells
+// in halos), large ones large tiles (1.8x).  A block has 8-16 waves of few
+// rows: the same 32 x 32 tile with 4 rows a thread (1 wave per SIMD) measured
+// 2.6 us a step, with 2 rows 1.85, with 1 row 1.7 but slower with poles;
+// 16-step launches (64 x 48 tiles) 2.9.  Measured with a read of the fields
+// per pass: 256^2 FP64 8.1 -> 1.9 us a step, 301x243 FP32 with a metal
+// cylinder 12.5 -> 2.0, 512^2 FP32 11.9 -> 4.2, 1024^2 FP32 19.9 -> 10.7.
+constexpr int kTileSteps = 8;
+constexpr int kTileDet = 64;  // detector points of one tile at most
+constexpr int kTileSets = 8;  // pole sets at most
+
+// A detector point of a tile: its thread and row, and where its samples go.
+struct TileDet {
+    double conv;
+    long long out;
+    int thr, row, comp, interval, cap, npts, pow;
+};
+
+template <typename T>
+struct TileArgs {
+    const T *ez, *hx, *hy;  // current buffers
+    T *ez_o, *hx_o, *hy_o;
+    int nx, ny, px, ntx, Tx, Ty;
+    T inv_dx, inv_dy;
+    const T *ch0, *ch1;
+    const uint8_t* mat;
+    const T *ce, *inveps;
+    const int *flags, *poleset;
+    int nmat;
+    // psi of Hx (y), Hy (x), Ez (x), Ez (y): region, profiles, current and next
+    int lo[4], hi0[4], hi1[4], S[4];
+    const T *b[4], *cd[4], *kinv[4], *psi[4];
+    T* psi_o[4];
+    int npole;  // poles of the largest set (0: no dispersive cell)
+    int nset;   // pole sets
+    const int* pole_count;
+    const T* pole_coef;
+    const T *P, *J;
+    T *P_o, *J_o;
+    int box[4];  // x0, x1, y0, y1 of the pole-state box
+    long long boxn;
+    int nsrc;
+    const int *src_comp, *src_box;
+    const T* src_amp;
+    const int* step;
+    int stepv;
+    int* step_next;
+    int nstep;  // steps of this launch, 1 .. kTileSteps
+    const int* det_ofs;  // [ntx nty + 1]: each tile's range in det
+    const TileDet* det;
+    double* det_out;
+    bool fma_curl;  // outside the CPML the curl's second product is fused (see enable_tiles)
+};
+
+// The next (up = true) or previous lane's value over the whole wave.  At the
+// wave's ends, and between the two rows of a wave that holds two, the value
+// is another cell's; those lanes hold the halo's outermost columns.
+template <bool UP>
+__device__ __forceinline__ float lane_nb(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), UP ? 0x130 : 0x138, 0xf, 0xf, false));
+}
+template <bool UP>
+__device__ __forceinline__ double lane_nb(double v) {
+    const long long l = __double_as_longlong(v);
+    const int a = __builtin_amdgcn_update_dpp(0, static_cast<int>(l), UP ? 0x130 : 0x138, 0xf, 0xf, false);
+    const int b = __builtin_amdgcn_update_dpp(0, static_cast<int>(l >> 32), UP ? 0x130 : 0x138, 0xf, 0xf, false);
+    return __longlong_as_double((static_cast<long long>(b) << 32) | static_cast<unsigned>(a));
+}
+
+// Tile shape: RX columns, NS strips of R rows.
+template <int RX, int R, int NS>
+struct TileShape {
+    static constexpr int rx = RX, r = R, ns = NS, ry = R * NS, threads = RX * NS;
+    static constexpr int ux = RX - 2 * kTileSteps, uy = R * NS - 2 * kTileSteps;  // the tile's own cells
+};
+
+template <typename T, typename SH>
+__device__ __forceinline__ void tile2_body(const TileArgs<T>& a, int bx, int nb) {
+    constexpr int RX = SH::rx, R = SH::r, NS = SH::ns, K = kTileSteps, NT = SH::threads;
+    static_assert(NT >= CHIML_MAX_MAT && NT >= 2 * SH::ry && NT >= kTileSets * CHIML_MAX_POLES * 3 && CHIML_MAX_SRC <= 64, "one thread per table entry");
+    __shared__ T s_ez[NS][RX], s_hx[NS][RX];
+    __shared__ MatLds<T> s_mt[CHIML_MAX_MAT];
+    __shared__ T s_y[2][3][SH::ry];  // y CPML b, c/d, 1/kappa of Hx and Ez by row
+    __shared__ T s_amp[K][CHIML_MAX_SRC];
+    __shared__ int4 s_box[CHIML_MAX_SRC];  // x0, x1, y0, y1 of the sources that touch the tile
+    __shared__ int s_comp[CHIML_MAX_SRC];
+    __shared__ TileDet s_det[kTileDet];
+    __shared__ T s_co[kTileSets * CHIML_MAX_POLES * 3];
+    __shared__ int s_np[kTileSets];
+    __shared__ int s_nsrc;
+    extern __shared__ __align__(16) unsigned char tile_lds[];
+    T* const s_P = reinterpret_cast<T*>(tile_lds);  // [npole][P, J][R][NT]
+    const int tid = threadIdx.x, col = tid % RX, strip = tid / RX;
+    const int tile = xcd_block(bx, nb);
+    const int ty = tile / a.ntx, tx = tile - ty * a.ntx;
+    const int x0 = tx * SH::ux - K, y0 = ty * SH::uy - K;
+    const int x = x0 + col, yb = y0 + strip * R;
+    const int nx = a.nx, ny = a.ny, px = a.px;
+    const int step = step_now(a.step, a.stepv);
+    const bool xin = x >= 0 && x < nx;
+    // slab position of pos: psi 0 Hx along y, 1 Hy along x, 2 Ez along x, 3 Ez along y
+    auto at = [&](int q, int pos) {
+        if (pos < 0) return -1;
+        if (pos < a.lo[q]) return pos;
+        if (pos >= a.hi0[q] && pos < a.hi1[q]) return a.lo[q] + pos - a.hi0[q];
+        return -1;
+    };
+    auto meets = [&](int q, int p0, int p1) { return a.S[q] > 0 && ((p0 < a.lo[q] && p1 > 0) || (p1 > a.hi0[q] && p0 < a.hi1[q])); };
+    const bool xp = meets(1, x0, x0 + RX) || meets(2, x0, x0 + RX), yp = meets(0, y0, y0 + SH::ry) || meets(3, y0, y0 + SH::ry);
+    // ---- every load of the tile, before the first wait ----
+    T ez[R], hx[R], hy[R];
+    unsigned id[R], in = 0;  // in: rows inside the grid
+    const int xc = min(max(x, 0), nx - 1);
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const int y = yb + r;
+        const long long i = xc + static_cast<long long>(px) * min(max(y, 0), ny - 1);
+        if (xin && y >= 0 && y < ny) in |= 1u << r;
+        ez[r] = a.ez[i];
+        hx[r] = a.hx[i];
+        hy[r] = a.hy[i];
+        id[r] = a.mat ? a.mat[i] : 0u;
+    }
+    T pxh[R], pxe[R], pyh[R], pye[R], xh[3] = {T(0), T(0), T(1)}, xe[3] = {T(0), T(0), T(1)}, yc[3] = {T(0), T(0), T(1)};
+#pragma unroll
+    for (int r = 0; r < R; ++r) pxh[r] = pxe[r] = pyh[r] = pye[r] = T(0);
+    const int sxh = xin ? at(1, x) : -1, sxe = xin ? at(2, x) : -1;
+    if (xp) {
+        if (sxh >= 0) {
+            xh[0] = a.b[1][x];
+            xh[1] = a.cd[1][x];
+            xh[2] = a.kinv[1][x];
+        }
+        if (sxe >= 0) {
+            xe[0] = a.b[2][x];
+            xe[1] = a.cd[2][x];
+            xe[2] = a.kinv[2][x];
+        }
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const int y = min(max(yb + r, 0), ny - 1);
+            if (sxh >= 0) pxh[r] = a.psi[1][sxh + static_cast<long long>(a.S[1]) * y];
+            if (sxe >= 0) pxe[r] = a.psi[2][sxe + static_cast<long long>(a.S[2]) * y];
+        }
+    }
+    if (yp) {
+        if (tid < 2 * SH::ry) {
+            const int q = tid < SH::ry ? 0 : 3, y = y0 + tid % SH::ry;
+            if (y < ny && at(q, y) >= 0) {
+                yc[0] = a.b[q][y];
+                yc[1] = a.cd[q][y];
+                yc[2] = a.kinv[q][y];
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const int s0 = yb + r < ny ? at(0, yb + r) : -1, s3 = yb + r < ny ? at(3, yb + r) : -1;
+            if (s0 >= 0) pyh[r] = a.psi[0][xc + static_cast<long long>(px) * s0];
+            if (s3 >= 0) pye[r] = a.psi[3][xc + static_cast<long long>(px) * s3];
+        }
+    }
+    MatLds<T> mt{T(0), T(0), 0, -1};
+    if (tid < a.nmat) mt = MatLds<T>{a.ce[tid], a.inveps[tid], a.flags[tid], a.poleset[tid]};
+    T co = T(0);
+    int np = 0;
+    if (a.npole) {
+        if (tid < a.nset * CHIML_MAX_POLES * 3) co = a.pole_coef[tid];
+        if (tid < a.nset) np = a.pole_count[tid];
+    }
+    const int d0 = a.det_ofs[tile], nd = min(a.det_ofs[tile + 1] - d0, kTileDet);
+    TileDet det{};
+    if (tid < nd) det = a.det[d0 + tid];
+    const T ch0 = a.ch0[0], ch1 = a.ch1[0];
+    int4 sb = make_int4(0, 0, 0, 0);
+    int scomp = 0;
+    T amp[K];
+    if (tid < a.nsrc) {  // one lane per source
+        sb = make_int4(a.src_box[6 * tid], a.src_box[6 * tid + 1], a.src_box[6 * tid + 2], a.src_box[6 * tid + 3]);
+        scomp = a.src_comp[tid];
+#pragma unroll
+        for (int s = 0; s < K; ++s) amp[s] = a.src_amp[static_cast<long long>(step + min(s, a.nstep - 1)) * a.nsrc + tid];
+    }
+    // ---- tables to LDS ----
+    if (tid < a.nmat) s_mt[tid] = mt;
+    if (yp && tid < 2 * SH::ry)
+        for (int k = 0; k < 3; ++k) s_y[tid < SH::ry ? 0 : 1][k][tid % SH::ry] = yc[k];
+    if (a.npole) {
+        if (tid < a.nset * CHIML_MAX_POLES * 3) s_co[tid] = co;
+        if (tid < a.nset) s_np[tid] = np;
+    }
+    if (tid < nd) {
+        // row .. pow as they are; interval counts down to the next sample, out is its place
+        const int first = det.interval - step % det.interval, slot = (step + first) / det.interval;
+        det.out += static_cast<long long>(slot) * det.npts;
+        det.cap -= slot;
+        det.thr |= det.row << 16;
+        det.row = first - 1;  // launch step of the next sample
+        s_det[tid] = det;
+    }
+    if (tid < 64) {  // the sources that touch the tile, in the table's order
+        const bool hit = tid < a.nsrc && sb.x < x0 + RX && sb.y > x0 && sb.z < y0 + SH::ry && sb.w > y0;
+        const unsigned long long m = __ballot(hit);
+        if (hit) {
+            const int n = __popcll(m & ((1ull << tid) - 1));
+            s_box[n] = sb;
+            s_comp[n] = scomp;
+#pragma unroll
+            for (int s = 0; s < K; ++s) s_amp[s][n] = amp[s];
+        }
+        if (tid == 0) s_nsrc = __popcll(m);
+    }
+    __syncthreads();
+    // ---- what the steps need per row, in registers ----
+    T ce[R], iev[R];
+    unsigned prow = 0, drow = 0, sets = 0, nps = 0;  // dispersive rows, D rows, pole set and pole count (4 bits a row)
+    unsigned long long dets = 0;                     // the thread's detector points
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const MatLds<T> m = s_mt[id[r]];
+        ce[r] = m.ce;
+        iev[r] = m.inveps;
+        const bool on = (in >> r) & 1u;
+        if (!on) ez[r] = hx[r] = hy[r] = T(0);
+        if (m.flags & CHIML_MAT_DCELL) drow |= 1u << r;
+        if (a.npole && on && m.poleset >= 0) {
+            prow |= 1u << r;
+            sets |= static_cast<unsigned>(m.poleset) << (4 * r);
+            const int n = s_np[m.poleset];
+            nps |= static_cast<unsigned>(n) << (4 * r);
+            const long long bi = (x - a.box[0]) + static_cast<long long>(a.box[1] - a.box[0]) * (yb + r - a.box[2]);
+            for (int p = 0; p < n; ++p) {
+                s_P[((2 * p) * R + r) * NT + tid] = a.P[p * a.boxn + bi];
+                s_P[((2 * p + 1) * R + r) * NT + tid] = a.J[p * a.boxn + bi];
+            }
+        }
+    }
+    for (int q = 0; q < nd; ++q)
+        if ((s_det[q].thr & 0xffff) == tid) dets |= 1ull << q;
+    const int nsrc = s_nsrc;
+    unsigned srows[3] = {0u, 0u, 0u};  // the rows that a source touches, per component (Ez, Hx, Hy)
+    for (int k = 0; k < nsrc; ++k) {
+        const int4 b = s_box[k];
+        const int f = max(b.z - yb, 0), l = min(b.w - yb, R);
+        if (x < b.x || x >= b.y || f >= l) continue;
+        const unsigned rows = ((1u << l) - 1) & ~((1u << f) - 1);
+        const int comp = s_comp[k];
+#pragma unroll
+        for (int c = 0; c < 3; ++c)
+            if (comp == 2 + c) srows[c] |= rows;
+    }
+    auto src_at = [&](int comp, int s, int y) {
+        T v = T(0);
+        for (int k = 0; k < nsrc; ++k) {
+            const int4 b = s_box[k];
+            if (s_comp[k] == comp && x >= b.x && x < b.y && y >= b.z && y < b.w) v += s_amp[s][k];
+        }
+        return v;
+    };
+    const bool hyv = x < nx - 1, plain = x >= a.Tx && x < nx - a.Tx;  // plain: outside the x CPML
+    // ---- the steps ----
+    for (int s = 0; s < a.nstep; ++s) {
+        s_ez[strip][col] = ez[0];
+        __syncthreads();
+        const T ez_up = strip + 1 < NS ? s_ez[strip + 1][col] : T(0);
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const T dy = (r + 1 < R ? ez[r + 1 < R ? r + 1 : r] : ez_up) - ez[r];
+            const T dx = lane_nb<true>(ez[r]) - ez[r];
+            T ty_ = dy * a.inv_dy, tx_ = dx * a.inv_dx;
+            const bool on = (in >> r) & 1u, hxon = on && yb + r < ny - 1, hyon = on && hyv;
+            if (yp) {
+                const int k = strip * R + r;
+                const T psi = fma(s_y[0][0][k], pyh[r], s_y[0][1][k] * dy);
+                if (hxon) pyh[r] = psi;
+                ty_ = fma(s_y[0][2][k], ty_, psi);
+            }
+            if (xp) {
+                const T psi = fma(xh[0], pxh[r], xh[1] * dx);
+                if (hyon) pxh[r] = psi;
+                tx_ = fma(xh[2], tx_, psi);
+            }
+            T vx = fma(ch0, -ty_, hx[r]), vy = fma(ch1, tx_, hy[r]);
+            if ((srows[1] >> r) & 1u) vx += src_at(3, s, yb + r);
+            if ((srows[2] >> r) & 1u) vy += src_at(4, s, yb + r);
+            hx[r] = hxon ? vx : hx[r];
+            hy[r] = hyon ? vy : hy[r];
+        }
+        s_hx[strip][col] = hx[R - 1];
+        __syncthreads();
+        const T hx_dn = strip > 0 ? s_hx[strip - 1][col] : T(0);
+        T acc[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const T d1 = hy[r] - lane_nb<false>(hy[r]);
+            const T d2 = hx[r] - (r > 0 ? hx[r > 0 ? r - 1 : 0] : hx_dn);
+            T t1 = d1 * a.inv_dx, t2 = d2 * a.inv_dy;
+            const bool fused = a.fma_curl && plain && yb + r >= a.Ty && yb + r < ny - a.Ty;
+            const T accf = fma(-a.inv_dy, d2, t1);
+            const bool on = (in >> r) & 1u;
+            if (xp) {
+                const T psi = fma(xe[0], pxe[r], xe[1] * d1);
+                if (on) pxe[r] = psi;
+                t1 = fma(xe[2], t1, psi);
+            }
+            if (yp) {
+                const int k = strip * R + r;
+                const T psi = fma(s_y[1][0][k], pye[r], s_y[1][1][k] * d2);
+                if (on) pye[r] = psi;
+                t2 = fma(s_y[1][2][k], t2, psi);
+            }
+            {
+#pragma clang fp contract(off)
+                acc[r] = fused ? accf : t1 - t2;
+            }
+        }
+        if (prow | srows[0]) {  // rare: poles and sources; a row without either keeps the plain form
+            T sv[R], jsum[R];
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                jsum[r] = T(0);
+                sv[r] = (srows[0] >> r) & 1u ? src_at(2, s, yb + r) : T(0);
+            }
+            if (prow)
+                for (int p = 0; p < a.npole; ++p) {
+                    T Pv[R], Jv[R];
+#pragma unroll
+                    for (int r = 0; r < R; ++r) {
+                        Pv[r] = s_P[((2 * p) * R + r) * NT + tid];
+                        Jv[r] = s_P[((2 * p + 1) * R + r) * NT + tid];
+                    }
+#pragma unroll
+                    for (int r = 0; r < R; ++r) {
+                        if (p >= static_cast<int>((nps >> (4 * r)) & 15u)) continue;
+                        const T* c = s_co + (((sets >> (4 * r)) & 15u) * CHIML_MAX_POLES + p) * 3;
+                        const T Jn = fma(c[2], ez[r] + sv[r], fma(c[0], Pv[r], c[1] * Jv[r]));
+                        s_P[((2 * p) * R + r) * NT + tid] = Pv[r] + Jn;
+                        s_P[((2 * p + 1) * R + r) * NT + tid] = Jn;
+                        jsum[r] += Jn;
+                    }
+                }
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+                if ((in >> r) & 1u) {
+                    const T base = (drow >> r) & 1u ? ez[r] : ez[r] + sv[r];
+                    ez[r] = fma(-iev[r], jsum[r], fma(ce[r], acc[r], base));
+                }
+        } else {
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+                if ((in >> r) & 1u) ez[r] = fma(ce[r], acc[r], ez[r]);
+        }
+        for (unsigned long long m = dets; m; m &= m - 1) {  // store_point's samples, at the advanced step
+            TileDet& q = s_det[__ffsll(static_cast<long long>(m)) - 1];
+            if (q.row != s) continue;
+            const int row = q.thr >> 16;
+            T f = T(0);
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+                if (r == row) f = q.comp == 2 ? ez[r] : (q.comp == 3 ? hx[r] : hy[r]);
+            double u = static_cast<double>(f);
+            if (q.pow) u = u * u;
+            double point = q.conv / 2.0 * u;
+            point = point + q.conv / 2.0 * u;
+            if (q.cap > 0) a.det_out[q.out] = point;
+            q.row = s + q.interval;
+            q.out += q.npts;
+            q.cap -= 1;
+        }
+    }
+    // ---- the tile's own cells go to the other buffers ----
+    const bool xown = xin && col >= K && col < RX - K;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const int row = strip * R + r, y = yb + r;
+        if (!xown || row < K || row >= SH::ry - K || !((in >> r) & 1u)) continue;
+        const long long i = x + static_cast<long long>(px) * y;
+        a.ez_o[i] = ez[r];
+        a.hx_o[i] = hx[r];
+        a.hy_o[i] = hy[r];
+        if (sxh >= 0) a.psi_o[1][sxh + static_cast<long long>(a.S[1]) * y] = pxh[r];
+        if (sxe >= 0) a.psi_o[2][sxe + static_cast<long long>(a.S[2]) * y] = pxe[r];
+        const int s0 = at(0, y), s3 = at(3, y);
+        if (s0 >= 0) a.psi_o[0][x + static_cast<long long>(px) * s0] = pyh[r];
+        if (s3 >= 0) a.psi_o[3][x + static_cast<long long>(px) * s3] = pye[r];
+        if ((prow >> r) & 1u) {
+            const long long bi = (x - a.box[0]) + static_cast<long long>(a.box[1] - a.box[0]) * (y - a.box[2]);
+            for (int p = 0; p < static_cast<int>((nps >> (4 * r)) & 15u); ++p) {
+                a.P_o[p * a.boxn + bi] = s_P[((2 * p) * R + r) * NT + tid];
+                a.J_o[p * a.boxn + bi] = s_P[((2 * p + 1) * R + r) * NT + tid];
+            }
+        }
+    }
+}
+
+template <typename T, typename SH>
+__global__ void __launch_bounds__(SH::threads) k_tile2(TileArgs<T> a) {
+    tile2_body<T, SH>(a, blockIdx.x, gridDim.x);
+    if (a.step_next && blockIdx.x == 0 && threadIdx.x == 0) *a.step_next = step_now(a.step, a.stepv) + a.nstep;
+}
+
+// 32 x 32 cells (16 x 16 own), 64 x 32 (48 x 16), 64 x 64 (48 x 48; FP32 only,
+// its FP64 registers spill: 1024^2 FP64 25 us a step, 16.5 with 64 x 32)
+using TileS = TileShape<32, 2, 16>;
+using TileM = TileShape<64, 2, 16>;
+using TileL = TileShape<64, 4, 16>;
+
 // ----------------------------------------------------- step counter ---------
 __global__ void k_set_step(int* step, int v) { *step = v; }
 
@@ -2740,6 +3161,17 @@ struct chiml_dev {
     void* fbuf[2][6] = {};      // fused: the two field buffers (fbuf[0] is the build's F)
     void* fpsi[2][3][3] = {};   // fused: the two psi buffers of each H component and axis
     bool vec2d = false;  // 2D TMz W-cell group kernels
+    // 2D: k_tile2 launches of up to kTileSteps steps on two sets of buffers;
+    // tile_cur is the set (and the step counter's slot) that holds the present
+    bool tile = false;
+    int tile_shape = 0, tile_cur = 0, tile_nx = 0, tile_ny = 0;
+    size_t tile_lds = 0;  // dynamic LDS (pole states)
+    int tile_npole = 0;
+    void* tbuf[2][9] = {};  // Ez, Hx, Hy, psi of Hx (y), Hy (x), Ez (x), Ez (y), P, J
+    const int* tile_det_ofs = nullptr;
+    const TileDet* tile_det = nullptr;
+    int tile_nset = 0;
+    hipGraphExec_t tile_exec[2] = {nullptr, nullptr};  // captured graphs, by the buffer set they start on
     bool fuse_sample = false;  // 2D: the E kernel takes the point detectors (no DFT, few single-cell points)
     bool det_single_field = true;  // every point detector reads one field (two cells) per point
     long long ade_groups = 0;  // largest pole-box group count over the E components (split path)
@@ -3683,6 +4115,236 @@ void do_steps(chiml_dev* c, StepArgs<T>& a, SampleArgs<T>& s, int n) {
     if (c->fused) set_fused_buffers<T>(c, a, s, c->steps_done - 1);
 }
 
+// ------------------------------------------------------- 2D tile launches ----
+template <typename T, typename F>
+void pick_tile(int shape, F&& f) {
+    if (shape == 0) f(TileS{});
+    else if (sizeof(T) == 8 || shape == 1) f(TileM{});
+    else f(std::conditional_t<sizeof(T) == 4, TileL, TileM>{});
+}
+
+// The pointers of the plain kernels and reads to buffer set k.
+template <typename T>
+void set_tile_buffers(chiml_dev* c, StepArgs<T>& a, SampleArgs<T>& s, int k) {
+    void* const* b = c->tbuf[k];
+    for (int j = 0; j < 3; ++j) {
+        a.F[2 + j] = static_cast<T*>(b[j]);
+        a.G[2 + j] = a.F[2 + j];
+        s.F[2 + j] = a.F[2 + j];
+    }
+    T** psi[4] = {&a.pml[3].psi[1], &a.pml[4].psi[0], &a.pml[2].psi[0], &a.pml[2].psi[1]};
+    for (int j = 0; j < 4; ++j) *psi[j] = static_cast<T*>(b[3 + j]);
+    a.P[2] = static_cast<T*>(b[7]);
+    a.J[2] = static_cast<T*>(b[8]);
+    c->tile_cur = k;
+}
+
+template <typename T>
+TileArgs<T> tile_args(const chiml_dev* c, const StepArgs<T>& a, int cur) {
+    TileArgs<T> t{};
+    void* const* in = c->tbuf[cur];
+    void* const* out = c->tbuf[1 - cur];
+    t.ez = static_cast<const T*>(in[0]);
+    t.hx = static_cast<const T*>(in[1]);
+    t.hy = static_cast<const T*>(in[2]);
+    t.ez_o = static_cast<T*>(out[0]);
+    t.hx_o = static_cast<T*>(out[1]);
+    t.hy_o = static_cast<T*>(out[2]);
+    t.nx = a.nx;
+    t.ny = a.ny;
+    t.px = a.px;
+    t.ntx = c->tile_nx;
+    t.inv_dx = a.inv_d[0];
+    t.inv_dy = a.inv_d[1];
+    t.ch0 = a.ch[0];
+    t.ch1 = a.ch[1];
+    t.mat = a.mat_e[2];
+    t.ce = a.ce[2];
+    t.inveps = a.inveps[2];
+    t.flags = a.flags[2];
+    t.poleset = a.poleset[2];
+    t.nmat = c->nmat[2];
+    const int comp[4] = {3, 4, 2, 2}, ax[4] = {1, 0, 0, 1};
+    for (int q = 0; q < 4; ++q) {
+        const PmlDev<T>& p = a.pml[comp[q]];
+        t.lo[q] = p.lo[ax[q]];
+        t.hi0[q] = p.hi0[ax[q]];
+        t.hi1[q] = p.hi1[ax[q]];
+        t.S[q] = p.S[ax[q]];
+        t.b[q] = p.b[ax[q]];
+        t.cd[q] = p.cd[ax[q]];
+        t.kinv[q] = p.kinv[ax[q]];
+        t.psi[q] = static_cast<const T*>(in[3 + q]);
+        t.psi_o[q] = static_cast<T*>(out[3 + q]);
+    }
+    t.npole = c->tile_npole;
+    t.pole_count = a.pole_count;
+    t.pole_coef = a.pole_coef;
+    t.P = static_cast<const T*>(in[7]);
+    t.J = static_cast<const T*>(in[8]);
+    t.P_o = static_cast<T*>(out[7]);
+    t.J_o = static_cast<T*>(out[8]);
+    for (int j = 0; j < 4; ++j) t.box[j] = a.box[2][j];
+    t.boxn = a.boxn[2];
+    t.nsrc = a.nsrc;
+    t.src_comp = a.src_comp;
+    t.src_box = a.src_box;
+    t.src_amp = a.src_amp;
+    t.det_ofs = c->tile_det_ofs;
+    t.det = c->tile_det;
+    t.det_out = c->det_out;
+    t.fma_curl = c->fma_curl;
+    t.Tx = a.Tp[0];
+    t.Ty = a.Tp[1];
+    t.nset = c->tile_nset;
+    return t;
+}
+
+// n steps in launches of up to kTileSteps.  Captured steps take an even
+// number of launches, so that a graph ends on the buffer set it starts on.
+template <typename T>
+void do_tile_steps(chiml_dev* c, StepArgs<T>& a, SampleArgs<T>& s, int n) {
+    if (n == 0) return;
+    const bool host = !c->capturing;
+    int* ctr = c->step_ctr.as<int>();
+    int launches = (n + kTileSteps - 1) / kTileSteps;
+    if (!host && launches % 2) ++launches;
+    int cur = c->tile_cur;
+    for (int l = 0, done = 0; l < launches; ++l) {
+        const int k = (n - done + launches - l - 1) / (launches - l);
+        TileArgs<T> t = tile_args<T>(c, a, cur);
+        t.step = ctr + cur;
+        t.stepv = host ? c->steps_done + done : -1;
+        t.step_next = host ? nullptr : ctr + (1 - cur);
+        t.nstep = k;
+        {
+            Timed tm(c, "update_tile");
+            pick_tile<T>(c->tile_shape, [&](auto sh) {
+                using SH = decltype(sh);
+                hipLaunchKernelGGL((k_tile2<T, SH>), dim3(static_cast<unsigned>(c->tile_nx * c->tile_ny)), dim3(SH::threads), c->tile_lds,
+                                   c->stream, t);
+            });
+        }
+        HIP_TRY(hipGetLastError());
+        done += k;
+        cur = 1 - cur;
+    }
+    c->steps_done += n;
+    c->enq_step = c->steps_done;
+    if (host) hipLaunchKernelGGL(k_set_step, dim3(1), dim3(1), 0, c->stream, ctr + cur, c->steps_done);
+    set_tile_buffers<T>(c, a, s, cur);
+}
+
+// 2D decks whose whole step is the field update and point samples of single
+// cells take k_tile2.  The tile shape is the one with the least estimated
+// time: tiles per CU in rounds of 256, times the tile's cells at 30 issue
+// slots each, plus the two barriers and exchanges of a step (about 400
+// cycles); a shape whose pole states do not fit LDS is left out.
+template <typename T>
+void enable_tiles(chiml_dev* c, const chiml_problem_t* p, StepArgs<T>& a, SampleArgs<T>& s) {
+    if (c->dim != 2 || c->hmap || !c->qes.empty() || !c->tfsf.empty() || c->cells.n > 0 || c->ndft > 0) return;
+    if (!c->det_single_field) return;
+    for (int t = 0; t < c->totpts; ++t) {
+        const int cu = p->det_comp[2 * t];
+        if (cu != p->det_comp[2 * t + 1] || p->det_cell[2 * t] != p->det_cell[2 * t + 1] || cu < 2 || cu > 4) return;
+    }
+    int npole = 0;
+    if (a.boxn[2] > 0 && a.P[2])
+        for (int k = 0; k < p->npoleset; ++k) npole = std::max(npole, p->pole_count[k]);
+    if (npole > 0 && p->npoleset > kTileSets) return;
+    int lds_max = 0;
+    HIP_TRY(hipDeviceGetAttribute(&lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, c->device));
+    int best = -1;
+    double best_t = 0.0;
+    size_t best_lds = 0;
+    for (int sh = 0; sh < (sizeof(T) == 4 ? 3 : 2); ++sh)
+        pick_tile<T>(sh, [&](auto shape) {
+            using SH = decltype(shape);
+            const size_t dyn = static_cast<size_t>(npole) * 2 * sizeof(T) * SH::rx * SH::ry;
+            hipFuncAttributes at{};
+            const void* fn = reinterpret_cast<const void*>(k_tile2<T, SH>);
+            HIP_TRY(hipFuncGetAttributes(&at, fn));
+            if (dyn + at.sharedSizeBytes > static_cast<size_t>(lds_max)) return;
+            const double nt = static_cast<double>((p->nx + SH::ux - 1) / SH::ux) * ((p->ny + SH::uy - 1) / SH::uy);
+            const double est = std::ceil(nt / 256.0) * SH::rx * SH::ry * 0.47 + 400.0;
+            if (best < 0 || est < best_t) {
+                best = sh;
+                best_t = est;
+                best_lds = dyn;
+            }
+        });
+    if (best < 0) return;
+    int ux = 0, uy = 0, rx = 0, rows = 0;
+    pick_tile<T>(best, [&](auto shape) {
+        using SH = decltype(shape);
+        ux = SH::ux;
+        uy = SH::uy;
+        rx = SH::rx;
+        rows = SH::r;
+        if (best_lds > 0)
+            HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(k_tile2<T, SH>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                        static_cast<int>(best_lds)));
+    });
+    const int ntx = (p->nx + ux - 1) / ux, nty = (p->ny + uy - 1) / uy;
+    // the detector points of each tile (points past the grid's edge read the
+    // zero ghost: their samples stay the zeros of the output buffer)
+    std::vector<std::vector<TileDet>> of(static_cast<size_t>(ntx) * nty);
+    for (int d = 0, t = 0; d < c->ndet; ++d)
+        for (int k = 0; k < c->det_npts[d]; ++k, ++t) {
+            const long long cell = p->det_cell[2 * t];
+            if (cell < 0) continue;
+            const int x = static_cast<int>(cell % p->nx), y = static_cast<int>(cell / p->nx);
+            const int lx = x % ux + kTileSteps, ly = y % uy + kTileSteps;
+            TileDet q{};
+            q.thr = ly / rows * rx + lx;
+            q.row = ly % rows;
+            q.comp = p->det_comp[2 * t];
+            q.interval = c->det_interval[d];
+            q.cap = c->det_cap[d];
+            q.npts = c->det_npts[d];
+            q.pow = p->det_pow[d];
+            q.conv = p->det_conv[d];
+            q.out = c->det_out_off[d] + k;
+            of[static_cast<size_t>(y / uy) * ntx + x / ux].push_back(q);
+        }
+    std::vector<int> ofs(1, 0);
+    std::vector<TileDet> pts;
+    for (auto& v : of) {
+        if (v.size() > static_cast<size_t>(kTileDet)) return;
+        pts.insert(pts.end(), v.begin(), v.end());
+        ofs.push_back(static_cast<int>(pts.size()));
+    }
+    if (pts.empty()) pts.emplace_back();
+    c->tile_det_ofs = c->upload<int>(ofs.data(), ofs.size());
+    c->tile_det = c->upload<TileDet>(pts.data(), pts.size());
+    c->tile_nset = p->npoleset;
+    const size_t N = static_cast<size_t>(c->px) * p->ny;
+    T* const psi[4] = {a.pml[3].psi[1], a.pml[4].psi[0], a.pml[2].psi[0], a.pml[2].psi[1]};
+    const size_t psin[4] = {static_cast<size_t>(a.pml[3].S[1]) * c->px, static_cast<size_t>(a.pml[4].S[0]) * p->ny,
+                            static_cast<size_t>(a.pml[2].S[0]) * p->ny, static_cast<size_t>(a.pml[2].S[1]) * c->px};
+    for (int j = 0; j < 3; ++j) {
+        c->tbuf[0][j] = a.F[2 + j];
+        c->tbuf[1][j] = c->zeros<T>(N);
+    }
+    for (int j = 0; j < 4; ++j) {
+        c->tbuf[0][3 + j] = psi[j];
+        c->tbuf[1][3 + j] = psi[j] ? c->zeros<T>(psin[j]) : nullptr;
+    }
+    if (npole > 0) {
+        c->tbuf[0][7] = a.P[2];
+        c->tbuf[0][8] = a.J[2];
+        c->tbuf[1][7] = c->zeros<T>(static_cast<size_t>(a.boxn[2]) * npole);
+        c->tbuf[1][8] = c->zeros<T>(static_cast<size_t>(a.boxn[2]) * npole);
+    }
+    c->tile = true;
+    c->tile_shape = best;
+    c->tile_nx = ntx;
+    c->tile_ny = nty;
+    c->tile_lds = best_lds;
+    c->tile_npole = npole;
+    set_tile_buffers<T>(c, a, s, 0);
+}
+
 void collect_profile(chiml_dev* c) {
     for (auto& pe : c->pending) {
         float ms = 0.0f;
@@ -3738,7 +4400,7 @@ void* scratch_on(int dev) {
 // Kernel class of a context for batched launches: 1 = 2D W-cell kernels,
 // 2 = 3D split sweeps; 0 = not batched (stepped on its own stream).
 int batch_class(const chiml_dev* c) {
-    if (c->fused || c->capturing || !c->tfsf.empty() || c->cells.n > 0) return 0;  // TFSF and per-cell source steps stay on their own stream
+    if (c->fused || c->tile || c->capturing || !c->tfsf.empty() || c->cells.n > 0) return 0;  // TFSF and per-cell source steps stay on their own stream
     if (c->dim == 2 && c->vec2d) return 1;
     if (c->dim == 3 && c->split && c->rows == (c->prec == 32)) return 2;
     return 0;
@@ -4093,6 +4755,8 @@ int chiml_dev_create(const chiml_problem_t* p, chiml_dev_t** out) {
                 single = cu == p->det_comp[2 * t + 1] && p->det_cell[2 * t] == p->det_cell[2 * t + 1] && cu >= 2 && cu <= 4;
             }
             c->fuse_sample = c->vec2d && single;
+            if (c->prec == 32) enable_tiles<float>(c.get(), p, c->a32, c->s32);
+            else enable_tiles<double>(c.get(), p, c->a64, c->s64);
         }
         if (c->dim == 3) {
             const int Tx = p->pml_T[0], Ty = p->pml_T[1], Tz = p->pml_T[2];
@@ -4139,7 +4803,10 @@ int chiml_dev_create(const chiml_problem_t* p, chiml_dev_t** out) {
 
 namespace {
 void enqueue_steps(chiml_dev* c, int n) {
-    if (c->prec == 32) do_steps<float>(c, c->a32, c->s32, n);
+    if (c->tile) {
+        if (c->prec == 32) do_tile_steps<float>(c, c->a32, c->s32, n);
+        else do_tile_steps<double>(c, c->a64, c->s64, n);
+    } else if (c->prec == 32) do_steps<float>(c, c->a32, c->s32, n);
     else do_steps<double>(c, c->a64, c->s64, n);
 }
 
@@ -4147,10 +4814,11 @@ void enqueue_steps(chiml_dev* c, int n) {
 // launch reads the step number from the device counter, so one graph serves
 // every chunk of the run.
 void ensure_graph(chiml_dev* c) {
-    if (c->gexec) return;
+    hipGraphExec_t& exec = c->tile ? c->tile_exec[c->tile_cur] : c->gexec;
+    if (exec) return;
     std::lock_guard<std::mutex> lk(g_capture_mu);
     hipGraph_t g = nullptr;
-    const int saved = c->steps_done;
+    const int saved = c->steps_done, saved_enq = c->enq_step;
     c->graph_parity = c->steps_done & 1;
     HIP_TRY(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
     c->capturing = true;
@@ -4165,8 +4833,9 @@ void ensure_graph(chiml_dev* c) {
     }
     c->capturing = false;
     HIP_TRY(hipStreamEndCapture(c->stream, &g));
-    c->steps_done = saved;  // capture enqueued nothing
-    hipError_t e = hipGraphInstantiate(&c->gexec, g, nullptr, nullptr, 0);
+    c->steps_done = saved;  // capture enqueued nothing (and tile launches ended on the buffers they started on)
+    c->enq_step = saved_enq;
+    hipError_t e = hipGraphInstantiate(&exec, g, nullptr, nullptr, 0);
     (void)hipGraphDestroy(g);
     HIP_TRY(e);
 }
@@ -4179,6 +4848,12 @@ int chiml_dev_step(chiml_dev_t* c, int n) {
         if (c->graph_steps > 0) {
             while (n >= c->graph_steps) {
                 ensure_graph(c);
+                if (c->tile) {
+                    HIP_TRY(hipGraphLaunch(c->tile_exec[c->tile_cur], c->stream));
+                    c->steps_done += c->graph_steps;
+                    n -= c->graph_steps;
+                    continue;
+                }
                 if ((c->steps_done & 1) != c->graph_parity) {  // realign the counter slot with one plain step
                     enqueue_steps(c, 1);
                     --n;
@@ -4202,6 +4877,10 @@ int chiml_dev_set_graph(chiml_dev_t* c, int steps_per_graph) {
     if (c->gexec) {
         (void)hipGraphExecDestroy(c->gexec);
         c->gexec = nullptr;
+    }
+    for (hipGraphExec_t& e : c->tile_exec) {
+        if (e) (void)hipGraphExecDestroy(e);
+        e = nullptr;
     }
     // even, so that every replay starts on the counter slot the graph was captured on
     c->graph_steps = steps_per_graph + (steps_per_graph & 1);
@@ -4428,6 +5107,8 @@ void chiml_dev_destroy(chiml_dev_t* c) {
     std::lock_guard<std::mutex> lk(g_capture_mu);
     (void)hipStreamSynchronize(c->stream);
     if (c->gexec) (void)hipGraphExecDestroy(c->gexec);
+    for (hipGraphExec_t e : c->tile_exec)
+        if (e) (void)hipGraphExecDestroy(e);
     for (auto& pe : c->pending) {
         (void)hipEventDestroy(pe.second.first);
         (void)hipEventDestroy(pe.second.second);
