@@ -8,7 +8,7 @@
 //                    (addPul, updateE/updateD, updateEPML, D2E)
 //                    3D FP32: k_h3_all / k_e3_all; 3D FP64: k_h3_int + k_h3_slab /
 //                    k_e3_int + k_e3_slab; 2D: k_h2v / k_e2v; else k_update_h / k_update_e
-//   3. emitters    : k_ml_addp, k_ml_team, then k_ml_pop_finish on recording steps
+//   3. emitters    : k_ml_addp, k_ml_entry, then k_ml_pop_finish on recording steps
 //                    (parallelQEBase::addQE)
 //   4. t_step += 1 : plain launches are given the step number by the host;
 //                    inside captured graphs the H launch advances a two-slot
@@ -2368,12 +2368,11 @@ struct QeDev {
     const double2* h0;      // [nmem][N*N]
     const double2* mu;      // [3][N*N]
     int ngam;
-    const int* gam_row;
-    const int* gam_col;
+    const int* gam_ptr;     // [N*N + 1]: the Lindblad entries of each row
+    const int* gam_col;     // [ngam], by row
     const double* gam_val;
-    const int* gam_colptr;  // [N + 1]: entries whose row lies in density column j
-    const int* gam_rc;      // [ngam]: row | col << 16 of each entry, in the same order
-    double na, hbar, dt;
+    double na, ih;          // ih = 1 / hbar
+    double ab[4], am[4];    // dt/24 (55, -59, 37, -9) and dt/24 (9, 19, -5, 1): predictor and corrector weights
     int bmin[3], bn[3];     // emitter box
     double* Pbox[3];        // (bn+2)^3 node polarization, z-extent bn+1+zoff
     double* Aprev[3];       // per touched E cell (bn+1)^3 previous back-coupling
@@ -2426,288 +2425,229 @@ __device__ __forceinline__ double2 cmul(double2 a, double2 b) { return make_doub
 __device__ __forceinline__ double2 cadd(double2 a, double2 b) { return make_double2(a.x + b.x, a.y + b.y); }
 __device__ __forceinline__ double2 cscale(double2 a, double s) { return make_double2(a.x * s, a.y * s); }
 
-// Rows i0 .. i0 + R - 1 of column j of d rho/dt for the matrices H and X
-// held in LDS (column-major): (i/hbar)(H X - X H)[i, j] + the Lindblad rows
-// among them.  grc / gv / gcp: the Lindblad entries (packed row | col << 16,
-// value) and column pointers, staged in LDS by the caller when they fit.
-// PK: only the stored rows i <= j are needed.
-template <int N, int R, bool PK>
-__device__ __forceinline__ void den_deriv_rows(const QeDev& q, const double2* H, const double2* X, int j, int i0, const int* grc,
-                                               const double* gv, const int* gcp, double2 (&out)[R]) {
-    const double ih = 1.0 / q.hbar;
-    // outer-product order over k (not unrolled): one column of H and of X
-    // in flight at a time keeps the register footprint small
-    double2 s1[R], s2[R];
-#pragma unroll
-    for (int r = 0; r < R; ++r) s1[r] = s2[r] = make_double2(0.0, 0.0);
-#pragma unroll 1
+// Entry (i, j) of d rho/dt for the matrices H and X of one emitter in LDS
+// (entry k of emitter t at [k EB + t], column-major): (i/hbar)(H X - X H)[i, j]
+// + the entry's Lindblad row.
+template <int N, int EB>
+__device__ __forceinline__ double2 den_deriv(double ih, const double2* H, const double2* X, int i, int j, const int* col, const double* val,
+                                             int g0, int g1) {
+    double2 s1 = make_double2(0.0, 0.0), s2 = s1;
+    // (three of the N terms in flight: all of them would cost half the waves)
+#pragma unroll 3
     for (int k = 0; k < N; ++k) {
-        const double2 xk = X[k + j * N], hk = H[k + j * N];
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-            const int i = i0 + r;
-            if (i >= N || (PK && i > j)) continue;
-            s1[r] = cadd(s1[r], cmul(H[i + k * N], xk));
-            s2[r] = cadd(s2[r], cmul(X[i + k * N], hk));
-        }
+        s1 = cadd(s1, cmul(H[(i + k * N) * EB], X[(k + j * N) * EB]));
+        s2 = cadd(s2, cmul(X[(i + k * N) * EB], H[(k + j * N) * EB]));
     }
-#pragma unroll
-    for (int r = 0; r < R; ++r) out[r] = make_double2(-(s1[r].y - s2[r].y) * ih, (s1[r].x - s2[r].x) * ih);
-    for (int g = gcp[j]; g < gcp[j + 1]; ++g) {
-        const int rc = grc[g];
-        const int rr = (rc & 0xffff) - j * N - i0;
-        if (rr < 0 || rr >= R) continue;
-        const double2 v = X[rc >> 16];
-        const double w = gv[g];
-#pragma unroll
-        for (int r = 0; r < R; ++r)
-            if (rr == r && !(PK && i0 + r > j)) {
-                out[r].x += v.x * w;
-                out[r].y += v.y * w;
-            }
+    double2 out = make_double2(-(s1.y - s2.y) * ih, (s1.x - s2.x) * ih);
+    for (int g = g0; g < g1; ++g) {
+        const double2 v = X[col[g] * EB];
+        out.x += v.x * val[g];
+        out.y += v.y * val[g];
     }
+    return out;
 }
 
-// Every emitter group (N >= 2): a team of lanes per emitter, each lane owning
-// R consecutive rows of one column j of rho, its history and its derivative
-// (R = N: the whole column), advanced by the Adams-Bashforth-Moulton
-// predictor-corrector (PCABAM4, parallelQE.hpp:751-770) cold-started from
-// zero history; the derivative history is a 4-slot ring instead of the
-// reference's three copies per step (density.hpp:65-70).  The kernel takes
-// any R; splitting a column over lanes (R = 2 or 3 for N = 6) cuts the VGPRs
-// from 236 to 138-162 (3 waves per SIMD instead of 2) but measured slower,
-// 0.59 / 0.49 ms against 0.45 ms per launch for 368,640 6-level emitters:
-// every extra lane repeats the shared-matrix reads of the commutator.
-// Lanes are grouped by (column, row chunk), lane = c * EB + team, so the
-// lanes of one chunk hold consecutive emitters and every rho / history
-// access of a wave is a few contiguous runs.  H = h0 - E.mu (formed once per
-// member, each lane its rows) and the matrix being differentiated are shared
-// through LDS with a per-emitter stride of N^2 + 1 elements, which spreads
-// the emitters of a wave over the LDS banks.
+// Every emitter group (N >= 2): one lane per stored entry of rho and emitter,
+// advanced by the Adams-Bashforth-Moulton predictor-corrector (PCABAM4,
+// parallelQE.hpp:751-770) cold-started from zero history; the derivative
+// history is a 4-slot ring instead of the reference's three copies per step
+// (density.hpp:65-70).  Lanes are grouped by entry, lane = k EB + emitter, so
+// every rho and history access of an entry is a contiguous run of EB complex
+// words.  H = h0 - E.mu (formed once per member, each lane its entry) and the
+// matrix being differentiated are shared through LDS, entry by entry with the
+// emitters side by side: consecutive lanes read consecutive words, no bank is
+// hit twice.
 //
 // PK (Hermitian packing): rho and the derivative history keep only the upper
-// triangle, entry (i, j) with i <= j stored at j (j + 1) / 2 + i, so a lane
-// loads and stores its rows i <= j; the lower entries are the conjugates of
-// the other lanes' entries, written to the shared matrices by those lanes.
+// triangle, entry (i, j) with i <= j stored at j (j + 1) / 2 + i; a lane also
+// writes the conjugate of its entry to the lower half of the shared matrices.
 // rho stays exactly Hermitian, which the full form keeps up to rounding (the
 // Lindblad sums of mirrored entries may add in another order).  Used when H0,
 // the dipoles and the Lindblad operator preserve hermiticity; the derivative
 // of a Hermitian rho is then Hermitian.
-constexpr int kMlThreads = 256;
+//
+// The kernel moves 7 words per stored entry (338,560 six-level emitters,
+// packed: 796 MB) and is bound by memory as long as enough waves are in flight
+// to cover its phases (load, two derivatives, store), so a lane holds one entry
+// (78 VGPRs, 6 waves per SIMD).  With one lane per column (236 VGPRs, 2 waves)
+// the same launch took 407 us, now 231 (3.4 TB/s); the copy rate would allow
+// 155.  4 waves per SIMD measured 275, blocks of 16 emitters 330.  32,768
+// two-level emitters: 10.1 -> 6.8 us.
 constexpr int kMlGamLds = 256;  // Lindblad entries staged in LDS (more are read from global memory)
 
 __host__ __device__ constexpr int ml_store_words(int n, bool pk) { return pk ? n * (n + 1) / 2 : n * n; }
-__host__ __device__ constexpr int ml_rows(int n) { return n; }
-__host__ __device__ constexpr int ml_lanes(int n) { return n * ((n + ml_rows(n) - 1) / ml_rows(n)); }  // lanes per emitter
+// emitters per block: the largest run whose lanes fit a block
+__host__ __device__ constexpr int ml_emitters(int n, bool pk) {
+    const int w = ml_store_words(n, pk);
+    return w * 64 <= 1024 ? 64 : (w * 32 <= 1024 ? 32 : 16);
+}
+__host__ __device__ constexpr int ml_threads(int n, bool pk) { return (ml_store_words(n, pk) * ml_emitters(n, pk) + 63) / 64 * 64; }
 
 template <typename T, int N, bool PK>
-__global__ void __launch_bounds__(kMlThreads) k_ml_team(QeDev q, T* E0, T* E1, T* E2, int nx, int ny, int nz,
-                                                        const int* stepp, int stepv) {
-    constexpr int S = N * N, R = ml_rows(N), NL = (N + R - 1) / R, LN = N * NL, EB = kMlThreads / LN, XS = S + 1,
-                  SP = ml_store_words(N, PK);
-    constexpr int XBYTES = EB * XS * 16, TAIL = kMlThreads * (3 * 8 + 16);
-    // Xs during the member loop; the polarisation and population reductions afterwards
-    __shared__ __align__(16) unsigned char lds[XBYTES > TAIL ? XBYTES : TAIL];
-    __shared__ double2 Hs[EB * XS];
+__global__ void __launch_bounds__(ml_threads(N, PK), 6) k_ml_entry(QeDev q, T* E0, T* E1, T* E2, int nx, int ny, int nz,
+                                                                const int* stepp, int stepv) {
+    constexpr int S = N * N, SP = ml_store_words(N, PK), EB = ml_emitters(N, PK);
+    static_assert(SP >= 3, "the first three entries' lanes gather the field components");
+    __shared__ double2 Hs[S * EB], Xs[S * EB];
     __shared__ double2 mus[3][S];
-    __shared__ int grc_s[kMlGamLds];
+    __shared__ double ef[3][EB];
+    __shared__ double2 pops[4][EB];
+    __shared__ int gc_s[kMlGamLds];
     __shared__ double gv_s[kMlGamLds];
-    __shared__ int gcp_s[N + 1];
-    double2* Xs = reinterpret_cast<double2*>(lds);
-    const int cl = threadIdx.x / EB, team = threadIdx.x - cl * EB;  // chunk lane (column j, rows i0..) and emitter
-    const int j = cl / NL, i0 = (cl - j * NL) * R;
+    const int k = threadIdx.x / EB, team = threadIdx.x - k * EB;  // stored entry and emitter
     const int e = blockIdx.x * EB + team;
-    const bool act = cl < LN && e < q.nemit;
-    const int step = step_now(stepp, stepv);
-    for (int k = threadIdx.x; k < 3 * S; k += blockDim.x) mus[k / S][k % S] = q.mu[k];
-    const bool gam_lds = q.ngam <= kMlGamLds;
-    if (gam_lds)
-        for (int g = threadIdx.x; g < q.ngam; g += blockDim.x) {
-            grc_s[g] = q.gam_rc[g];
-            gv_s[g] = q.gam_val[g];
-        }
-    for (int k = threadIdx.x; k <= N; k += blockDim.x) gcp_s[k] = q.gam_colptr[k];
-    const int* grc = gam_lds ? grc_s : q.gam_rc;
-    const double* gv = gam_lds ? gv_s : q.gam_val;
-    double2 pop[4] = {make_double2(0, 0), make_double2(0, 0), make_double2(0, 0), make_double2(0, 0)};
-    double P[3] = {0.0, 0.0, 0.0};
-    double ef[3] = {0.0, 0.0, 0.0};
-    T* const Es[3] = {E0, E1, E2};
-    int px = 0, py = 0, pz = 0;
-    // 2D with the fold: this emitter's addP result, stored after the first barrier
-    double fold_a = 0.0;
-    T fold_e = T(0);
-    long long fold_ai = -1, fold_ip = -1;
-    if (act) {
-        px = q.xyz[3 * e];
-        py = q.xyz[3 * e + 1];
-        pz = q.xyz[3 * e + 2];
-#pragma unroll
-        for (int c = 0; c < 3; ++c) {
-            if (!Es[c]) continue;
-            long long ip = px + static_cast<long long>(nx) * (py + static_cast<long long>(ny) * pz);
-            if (q.dim == 2) {
-                double ev = static_cast<double>(Es[c][ip]);
-                if (q.fold_addp && c == 2) {
-                    // k_ml_addp for this emitter's own E cell (in 2D no other
-                    // emitter's polarisation reaches it): E += A_prev - A
-                    const int bx = px - q.bmin[0] + 1, by = py - q.bmin[1] + 1;
-                    const double p0 = q.Pbox[c][bx + (q.bn[0] + 2) * by];
-                    fold_a = 0.5 * p0 / q.eps_node[ip] + 0.5 * p0 / q.eps_node[ip];
-                    fold_ai = bx + static_cast<long long>(q.bn[0] + 1) * by;
-                    fold_ip = ip;
-                    fold_e = static_cast<T>(ev + (q.Aprev[c][fold_ai] - fold_a));
-                    ev = static_cast<double>(fold_e);
-                }
-                ef[c] = ev;
-            } else {
-                // mean of the two Yee edges E_c(p) and E_c(p - e_c) (getE_TE)
-                const int qx = px - (c == 0), qy = py - (c == 1), qz = pz - (c == 2);
-                double v1 = (qx >= 0 && qy >= 0 && qz >= 0) ? static_cast<double>(Es[c][qx + static_cast<long long>(nx) * (qy + static_cast<long long>(ny) * qz)]) : 0.0;
-                ef[c] = 0.5 * static_cast<double>(Es[c][ip]) + 0.5 * v1;
-            }
-        }
+    const bool act = k < SP && e < q.nemit;
+    int i, j;
+    if (PK) {
+        j = 0;
+        while ((j + 1) * (j + 2) / 2 <= k && j < N - 1) ++j;
+        i = min(k - j * (j + 1) / 2, j);
+    } else {
+        j = min(k / N, N - 1);
+        i = k - (k / N) * N;
     }
+    const int kk = i + j * N;  // the entry's place in the full matrix
+    const int step = step_now(stepp, stepv);
     const int u = step & 3;
     const int s0 = (u + 3) & 3, s1 = (u + 2) & 3, s2 = (u + 1) & 3, s3 = u;
     const long long ld = static_cast<long long>(q.nmem) * q.nemit;
-    const double dt = q.dt;
-    double2* Xm = Xs + (act ? team : 0) * XS;
-    double2* Hm = Hs + (act ? team : 0) * XS;
-    // row i of this lane is kept in memory (upper triangle only when packed)
-    auto kept = [&](int i) { return i < N && !(PK && i > j); };
-    auto stored = [&](int i) -> long long { return PK ? j * (j + 1) / 2 + i : i + j * N; };
-    __syncthreads();  // mu and the Lindblad entries are staged; every lane has read E and A_prev
-    if (fold_ai >= 0 && cl == 0) {
-        q.Aprev[2][fold_ai] = fold_a;
-        Es[2][fold_ip] = fold_e;
+    long long at = k * ld + e;  // the entry of member 0
+    const long long slot = SP * ld;
+    double2 rk = make_double2(0.0, 0.0), f0 = rk, f1 = rk, f2 = rk, f3 = rk;
+    auto load = [&] {
+        if (!act) return;
+        rk = q.rho[at];
+        f0 = q.hist[s0 * slot + at];
+        f1 = q.hist[s1 * slot + at];
+        f2 = q.hist[s2 * slot + at];
+        f3 = q.hist[s3 * slot + at];
+    };
+    load();
+    for (int t = threadIdx.x; t < 3 * S; t += blockDim.x) mus[t / S][t % S] = q.mu[t];
+    const bool gam_lds = q.ngam <= kMlGamLds;
+    if (gam_lds)
+        for (int g = threadIdx.x; g < q.ngam; g += blockDim.x) {
+            gc_s[g] = q.gam_col[g];
+            gv_s[g] = q.gam_val[g];
+        }
+    const int* gc = gam_lds ? gc_s : q.gam_col;
+    const double* gv = gam_lds ? gv_s : q.gam_val;
+    const int g0 = act ? q.gam_ptr[kk] : 0, g1 = act ? q.gam_ptr[kk + 1] : 0;
+    // the lanes of entries 0..2 gather E_x, E_y, E_z at their emitter
+    T* const Ec = k == 0 ? E0 : (k == 1 ? E1 : (k == 2 ? E2 : nullptr));
+    if (k < 3 && act) {
+        const int px = q.xyz[3 * e], py = q.xyz[3 * e + 1], pz = q.xyz[3 * e + 2];
+        double ev = 0.0;
+        if (Ec) {
+            const long long ip = px + static_cast<long long>(nx) * (py + static_cast<long long>(ny) * pz);
+            ev = static_cast<double>(Ec[ip]);
+            if (q.dim != 2) {
+                // mean of the two Yee edges E_c(p) and E_c(p - e_c) (getE_TE)
+                const int qx = px - (k == 0), qy = py - (k == 1), qz = pz - (k == 2);
+                const double v1 = (qx >= 0 && qy >= 0 && qz >= 0) ? static_cast<double>(Ec[qx + static_cast<long long>(nx) * (qy + static_cast<long long>(ny) * qz)]) : 0.0;
+                ev = 0.5 * ev + 0.5 * v1;
+            } else if (q.fold_addp) {
+                // k_ml_addp for this emitter's own E cell (in 2D no other
+                // emitter's polarisation reaches it): E += A_prev - A
+                const int bx = px - q.bmin[0] + 1, by = py - q.bmin[1] + 1;
+                const double p0 = q.Pbox[2][bx + (q.bn[0] + 2) * by];
+                const double A = 0.5 * p0 / q.eps_node[ip] + 0.5 * p0 / q.eps_node[ip];
+                double* const Ap = q.Aprev[2] + bx + static_cast<long long>(q.bn[0] + 1) * by;
+                const T en = static_cast<T>(ev + (*Ap - A));
+                *Ap = A;
+                Ec[ip] = en;
+                ev = static_cast<double>(en);
+            }
+        }
+        ef[k][team] = ev;
     }
+    double2* const X = Xs + team;
+    double2* const H = Hs + team;
+    // population samples: every pop_interval steps while slots remain (QEPopDtc)
+    const bool record = q.npop > 0 && step % q.pop_interval == 0 && step / q.pop_interval < q.pop_cap;
+    double P = 0.0;
+    if (record && k == 0)
+        for (int jj = 0; jj < 4; ++jj) pops[jj][team] = make_double2(0.0, 0.0);
+    __syncthreads();  // mu, the Lindblad entries and E are staged
     for (int m = 0; m < q.nmem; ++m) {
-        const long long col = static_cast<long long>(m) * q.nemit + e;
-        double2 rc[R], fp[R];
+        double2 cr = rk;
         if (act) {
-#pragma unroll
-            for (int r = 0; r < R; ++r) {
-                const int i = i0 + r;
-                if (i >= N) continue;
-                const int k = i + j * N;
-                double2 h = q.h0[m * S + k];
-#pragma unroll
-                for (int c = 0; c < 3; ++c) {
-                    h.x -= ef[c] * mus[c][k].x;
-                    h.y -= ef[c] * mus[c][k].y;
-                }
-                Hm[k] = h;
-                if (!kept(i)) continue;
-                const long long ks = stored(i);
-                const double2 rk = q.rho[ks * ld + col];
-                const double2 f0 = q.hist[s0 * SP * ld + ks * ld + col];
-                const double2 f1 = q.hist[s1 * SP * ld + ks * ld + col];
-                const double2 f2 = q.hist[s2 * SP * ld + ks * ld + col];
-                const double2 f3 = q.hist[s3 * SP * ld + ks * ld + col];
-                double2 pr = rk;
-                pr = cadd(pr, cscale(f0, 55.0 * dt / 24.0));
-                pr = cadd(pr, cscale(f1, -59.0 * dt / 24.0));
-                pr = cadd(pr, cscale(f2, 37.0 * dt / 24.0));
-                pr = cadd(pr, cscale(f3, -9.0 * dt / 24.0));
-                Xm[k] = pr;
-                if (PK && i < j) Xm[j + i * N] = make_double2(pr.x, -pr.y);
-                double2 cr = rk;
-                cr = cadd(cr, cscale(f0, 19.0 * dt / 24.0));
-                cr = cadd(cr, cscale(f1, -5.0 * dt / 24.0));
-                cr = cadd(cr, cscale(f2, dt / 24.0));
-                rc[r] = cr;
-            }
-        }
-        __syncthreads();
-        if (act) den_deriv_rows<N, R, PK>(q, Hm, Xm, j, i0, grc, gv, gcp_s, fp);
-        __syncthreads();
-        if (act) {
-#pragma unroll
-            for (int r = 0; r < R; ++r) {
-                const int i = i0 + r;
-                if (!kept(i)) continue;
-                const int k = i + j * N;
-                rc[r] = cadd(rc[r], cscale(fp[r], 9.0 * dt / 24.0));
-                q.rho[stored(i) * ld + col] = rc[r];
-                Xm[k] = rc[r];
-                if (PK && i < j) Xm[j + i * N] = make_double2(rc[r].x, -rc[r].y);
-            }
-        }
-        __syncthreads();
-        if (act) {
-            den_deriv_rows<N, R, PK>(q, Hm, Xm, j, i0, grc, gv, gcp_s, fp);
-#pragma unroll
-            for (int r = 0; r < R; ++r)
-                if (kept(i0 + r)) q.hist[s3 * SP * ld + stored(i0 + r) * ld + col] = fp[r];
-#pragma unroll
-            for (int jj = 0; jj < 4; ++jj) {
-                if (jj >= q.npop) break;
-                const int k = q.pop_flat[jj];
-                const int ri = k % N, cj = k / N;
-#pragma unroll
-                for (int r = 0; r < R; ++r) {
-                    const int i = i0 + r;
-                    if (!kept(i)) continue;
-                    // entry (ri, cj) of the full matrix: stored (ri, cj), or with
-                    // packing below the diagonal the conjugate of (cj, ri)
-                    if ((!PK || ri <= cj) && i == ri && j == cj) pop[jj] = cadd(pop[jj], rc[r]);
-                    if (PK && ri > cj && i == cj && j == ri) pop[jj] = cadd(pop[jj], make_double2(rc[r].x, -rc[r].y));
-                }
-            }
+            double2 h = q.h0[m * S + kk];
 #pragma unroll
             for (int c = 0; c < 3; ++c) {
-                if (!Es[c]) continue;
+                h.x -= ef[c][team] * mus[c][kk].x;
+                h.y -= ef[c][team] * mus[c][kk].y;
+            }
+            H[kk * EB] = h;
+            double2 pr = rk;
+            pr = cadd(pr, cscale(f0, q.ab[0]));
+            pr = cadd(pr, cscale(f1, q.ab[1]));
+            pr = cadd(pr, cscale(f2, q.ab[2]));
+            pr = cadd(pr, cscale(f3, q.ab[3]));
+            X[kk * EB] = pr;
+            if (PK && i < j) {
+                H[(j + i * N) * EB] = make_double2(h.x, -h.y);
+                X[(j + i * N) * EB] = make_double2(pr.x, -pr.y);
+            }
+            cr = cadd(cr, cscale(f0, q.am[1]));
+            cr = cadd(cr, cscale(f1, q.am[2]));
+            cr = cadd(cr, cscale(f2, q.am[3]));
+        }
+        __syncthreads();
+        double2 fp = make_double2(0.0, 0.0);
+        if (act) fp = den_deriv<N, EB>(q.ih, H, X, i, j, gc, gv, g0, g1);
+        __syncthreads();
+        if (act) {
+            cr = cadd(cr, cscale(fp, q.am[0]));
+            q.rho[at] = cr;
+            X[kk * EB] = cr;
+            if (PK && i < j) X[(j + i * N) * EB] = make_double2(cr.x, -cr.y);
+        }
+        __syncthreads();
+        if (act) {
+            fp = den_deriv<N, EB>(q.ih, H, X, i, j, gc, gv, g0, g1);
+            q.hist[s3 * slot + at] = fp;
+            if (k < 3 && Ec) {  // polarisation of the emitter: sum of Re(conj(rho) mu)
                 double sacc = 0.0;
 #pragma unroll
-                for (int r = 0; r < R; ++r) {
-                    const int i = i0 + r;
-                    if (!kept(i)) continue;
-                    // Re(conj(rho_ij) mu_ij); with packing the mirrored entry
-                    // (j, i) adds the same again (rho and mu Hermitian)
-                    const double2 mu = mus[c][i + j * N];
-                    const double t = rc[r].x * mu.x + rc[r].y * mu.y;
-                    sacc += (PK && i < j) ? 2.0 * t : t;
-                }
-                P[c] += q.na * sacc;
+                for (int b = 0; b < N; ++b)
+#pragma unroll
+                    for (int a = 0; a < (PK ? b + 1 : N); ++a) {
+                        // with packing the mirrored entry adds the same again (rho and mu Hermitian)
+                        const double2 r = X[(a + b * N) * EB], mu = mus[k][a + b * N];
+                        const double t = r.x * mu.x + r.y * mu.y;
+                        sacc += (PK && a < b) ? 2.0 * t : t;
+                    }
+                P += q.na * sacc;
             }
+            if (record && k == 0)
+                for (int jj = 0; jj < q.npop; ++jj) pops[jj][team] = cadd(pops[jj][team], X[q.pop_flat[jj] * EB]);
         }
-        __syncthreads();  // Hs and Xs are rewritten by the next member
-    }
-    // polarisation of the emitter: sum of its lanes' parts
-    double (*Pl)[3] = reinterpret_cast<double (*)[3]>(lds);
-    double2* red = reinterpret_cast<double2*>(lds + kMlThreads * 3 * 8);
-#pragma unroll
-    for (int c = 0; c < 3; ++c) Pl[threadIdx.x][c] = P[c];
-    __syncthreads();
-    if (act && cl == 0) {
-        const int bx = px - q.bmin[0] + 1, by = py - q.bmin[1] + 1, bz = (q.dim == 3) ? pz - q.bmin[2] + 1 : 0;
-        const int PX = q.bn[0] + 2, PY = q.bn[1] + 2;
-        for (int c = 0; c < 3; ++c) {
-            if (!Es[c]) continue;
-            double sum = 0.0;
-            for (int l = 0; l < LN; ++l) sum += Pl[team + l * EB][c];
-            q.Pbox[c][bx + PX * (by + PY * bz)] = sum;
+        if (m + 1 < q.nmem) {
+            at += q.nemit;
+            load();
+            __syncthreads();  // Hs and Xs are rewritten by the next member
         }
     }
-    // Per-block population sums, only on the steps that record a sample
-    // (QEPopDtc: every pop_interval steps while slots remain); k_ml_pop_finish
-    // adds the blocks' sums in a fixed order.  A finish inside this launch
-    // (last block by an atomic ticket) needs a device-scope release per block,
-    // which writes back the XCD's L2 each time and more than doubled the
-    // launch.
-    if (q.npop == 0 || step % q.pop_interval != 0 || step / q.pop_interval >= q.pop_cap) return;
+    if (k < 3 && act && Ec) {
+        const int bx = q.xyz[3 * e] - q.bmin[0] + 1, by = q.xyz[3 * e + 1] - q.bmin[1] + 1, bz = (q.dim == 3) ? q.xyz[3 * e + 2] - q.bmin[2] + 1 : 0;
+        q.Pbox[k][bx + (q.bn[0] + 2) * (by + (q.bn[1] + 2) * bz)] = P;
+    }
+    // Per-block population sums by the first EB lanes, in a fixed order;
+    // k_ml_pop_finish adds the blocks' sums in a fixed order.  A finish inside
+    // this launch (last block by an atomic ticket) needs a device-scope release
+    // per block, which writes back the XCD's L2 each time and more than doubled
+    // the launch.
+    if (record && threadIdx.x < EB) {
+        for (int jj = 0; jj < q.npop; ++jj) {
+            double2 v = pops[jj][team];
 #pragma unroll
-    for (int jj = 0; jj < 4; ++jj) {
-        if (jj >= q.npop) break;
-        red[threadIdx.x] = pop[jj];
-        __syncthreads();
-        for (int w = blockDim.x / 2; w > 0; w >>= 1) {
-            if (threadIdx.x < w) red[threadIdx.x] = cadd(red[threadIdx.x], red[threadIdx.x + w]);
-            __syncthreads();
+            for (int w = EB / 2; w > 0; w >>= 1) {
+                v.x += __shfl_down(v.x, w, EB);
+                v.y += __shfl_down(v.y, w, EB);
+            }
+            if (threadIdx.x == 0) q.pop_partial[jj * gridDim.x + blockIdx.x] = v;
         }
-        if (threadIdx.x == 0) q.pop_partial[jj * gridDim.x + blockIdx.x] = red[0];
-        __syncthreads();
     }
 }
 
@@ -3698,36 +3638,33 @@ void build(chiml_dev* c, const chiml_problem_t* p, StepArgs<T>& a, SampleArgs<T>
         q.mu = reinterpret_cast<const double2*>(c->upload<double>(qi.mu, 2 * 3 * static_cast<size_t>(S)));
         q.ngam = qi.ngam;
         {
-            // Lindblad entries grouped by the density column their row lies in
-            // (stable, so each row keeps its accumulation order); gam_colptr[j]
-            // .. gam_colptr[j+1] are the entries a team's lane j applies.
+            // Lindblad entries by row (stable, so each row keeps its accumulation order)
             const int S = qi.nlevel * qi.nlevel;
             for (int g = 0; g < qi.ngam; ++g)
                 if (qi.gam_row[g] < 0 || qi.gam_row[g] >= S || qi.gam_col[g] < 0 || qi.gam_col[g] >= S)
                     throw std::runtime_error("Lindblad entry index outside nlevel^2");
             std::vector<int> order(qi.ngam);
             for (int g = 0; g < qi.ngam; ++g) order[g] = g;
-            std::stable_sort(order.begin(), order.end(), [&](int u, int v) { return qi.gam_row[u] / qi.nlevel < qi.gam_row[v] / qi.nlevel; });
-            std::vector<int> gr(std::max(qi.ngam, 1)), gc(std::max(qi.ngam, 1)), cp(qi.nlevel + 1, 0);
+            std::stable_sort(order.begin(), order.end(), [&](int u, int v) { return qi.gam_row[u] < qi.gam_row[v]; });
+            std::vector<int> gc(std::max(qi.ngam, 1)), ptr(S + 1, 0);
             std::vector<double> gv(std::max(qi.ngam, 1));
             for (int g = 0; g < qi.ngam; ++g) {
-                gr[g] = qi.gam_row[order[g]];
                 gc[g] = qi.gam_col[order[g]];
                 gv[g] = qi.gam_val[order[g]];
-                ++cp[gr[g] / qi.nlevel + 1];
+                ++ptr[qi.gam_row[order[g]] + 1];
             }
-            for (int j = 0; j < qi.nlevel; ++j) cp[j + 1] += cp[j];
-            q.gam_row = c->upload<int>(gr.data(), gr.size());
+            for (int r = 0; r < S; ++r) ptr[r + 1] += ptr[r];
+            q.gam_ptr = c->upload<int>(ptr.data(), ptr.size());
             q.gam_col = c->upload<int>(gc.data(), gc.size());
             q.gam_val = c->upload<double>(gv.data(), gv.size());
-            q.gam_colptr = c->upload<int>(cp.data(), cp.size());
-            std::vector<int> grc(gr.size());
-            for (size_t g = 0; g < gr.size(); ++g) grc[g] = gr[g] | (gc[g] << 16);
-            q.gam_rc = c->upload<int>(grc.data(), grc.size());
         }
         q.na = qi.na;
-        q.hbar = qi.hbar;
-        q.dt = p->dt;
+        q.ih = 1.0 / qi.hbar;
+        const double wab[4] = {55.0, -59.0, 37.0, -9.0}, wam[4] = {9.0, 19.0, -5.0, 1.0};
+        for (int k = 0; k < 4; ++k) {
+            q.ab[k] = wab[k] * p->dt / 24.0;
+            q.am[k] = wam[k] * p->dt / 24.0;
+        }
         q.dim = is3 ? 3 : 2;
         q.fold_addp = (!is3 && std::getenv("CHIML_ML_ADDP") == nullptr) ? 1 : 0;
         for (int k = 0; k < 3; ++k) {
@@ -3755,8 +3692,7 @@ void build(chiml_dev* c, const chiml_problem_t* p, StepArgs<T>& a, SampleArgs<T>
             if (qi.pop_flat[k] < 0 || qi.pop_flat[k] >= qi.nlevel * qi.nlevel) throw std::runtime_error("population detector index out of range");
         q.pop_flat = c->upload<int>(qi.pop_flat, std::max(qi.npop, 1));
         q.pop_interval = qi.pop_interval > 0 ? qi.pop_interval : 1;
-        // emitters per block of kMlThreads lanes
-        const int per_block = kMlThreads / ml_lanes(q.N);  // one team of lanes per emitter
+        const int per_block = ml_emitters(q.N, q.packed != 0);
         qh.nblocks = (q.nemit + per_block - 1) / per_block;
         q.pop_partial = reinterpret_cast<double2*>(c->zeros<double>(2 * 4 * static_cast<size_t>(qh.nblocks)));
         q.pop_cap = p->nsteps / q.pop_interval + 1;
@@ -4025,23 +3961,23 @@ void launch_ml(chiml_dev* c, StepArgs<T>& a) {
         {
             Timed t(c, "ml_density");
             switch (qh.N) {
-#define CHIML_ML_TEAM(NN)                                                                                                       \
+#define CHIML_ML_ENTRY(NN)                                                                                                       \
     case NN:                                                                                                                    \
         if (q.packed)                                                                                                           \
-            hipLaunchKernelGGL((k_ml_team<T, NN, true>), g, dim3(kMlThreads), 0, c->stream, q, a.F[0], a.F[1], a.F[2], c->px, c->ny, \
+            hipLaunchKernelGGL((k_ml_entry<T, NN, true>), g, dim3(ml_threads(NN, true)), 0, c->stream, q, a.F[0], a.F[1], a.F[2], c->px, c->ny, \
                                c->nz, a.step, a.stepv);                                                                         \
         else                                                                                                                    \
-            hipLaunchKernelGGL((k_ml_team<T, NN, false>), g, dim3(kMlThreads), 0, c->stream, q, a.F[0], a.F[1], a.F[2], c->px, c->ny, \
+            hipLaunchKernelGGL((k_ml_entry<T, NN, false>), g, dim3(ml_threads(NN, false)), 0, c->stream, q, a.F[0], a.F[1], a.F[2], c->px, c->ny, \
                                c->nz, a.step, a.stepv);                                                                         \
         break;
-                CHIML_ML_TEAM(2)
-                CHIML_ML_TEAM(3)
-                CHIML_ML_TEAM(4)
-                CHIML_ML_TEAM(5)
-                CHIML_ML_TEAM(6)
-                CHIML_ML_TEAM(7)
-                CHIML_ML_TEAM(8)
-#undef CHIML_ML_TEAM
+                CHIML_ML_ENTRY(2)
+                CHIML_ML_ENTRY(3)
+                CHIML_ML_ENTRY(4)
+                CHIML_ML_ENTRY(5)
+                CHIML_ML_ENTRY(6)
+                CHIML_ML_ENTRY(7)
+                CHIML_ML_ENTRY(8)
+#undef CHIML_ML_ENTRY
             }
         }
         if (q.npop > 0)
