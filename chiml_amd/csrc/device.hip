@@ -2360,6 +2360,61 @@ __global__ void __launch_bounds__(256) k_dft_flush(const T* stage, const double*
     }
 }
 
+// Flux through the faces of a box: the combined face fields (combineField,
+// parallelFlux.hpp:325-395), Ej Hk* - Ek Hj* over nt^2, the integration weight,
+// and a sum over the block's 256 points, one block row per frequency.  Each face
+// starts on a block boundary and the host adds a face's blocks in order.  Reads
+// 16 samples per point and frequency from the accumulators: a 61^3 box with 40
+// frequencies is read in 1.0 ms, where copying the accumulators to the host and
+// combining them there took 70 ms.
+constexpr int kFluxFaces = 6;
+struct FluxPlanDev {
+    int nface, start[kFluxFaces + 1];  // first point (padded) of each face
+    int npt[kFluxFaces];
+    double cw[kFluxFaces][4];
+    const int* ids;    // [16][start[nface]]
+    const double* sw;  // [start[nface]]
+};
+
+__global__ void __launch_bounds__(256) k_flux_faces(FluxPlanDev pl, const double2* __restrict__ F, int ndft, double inv_nt2,
+                                                    double2* __restrict__ partial) {
+    __shared__ double2 red[256];
+    const int total = pl.start[pl.nface], t = blockIdx.x * 256 + threadIdx.x;
+    int f = 0;
+    while (f + 1 < pl.nface && pl.start[f + 1] <= static_cast<int>(blockIdx.x) * 256) ++f;
+    const double2* Ff = F + static_cast<long long>(blockIdx.y) * ndft;
+    double2 v = make_double2(0.0, 0.0);
+    if (t - pl.start[f] < pl.npt[f]) {
+        double2 g[4];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            double2 acc = make_double2(0.0, 0.0);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const int id = pl.ids[(c * 4 + k) * static_cast<long long>(total) + t];
+                if (id < 0) continue;
+                const double2 u = Ff[id];
+                acc.x += pl.cw[f][c] * u.x;
+                acc.y += pl.cw[f][c] * u.y;
+            }
+            g[c] = acc;
+        }
+        const double w = pl.sw[t] * inv_nt2;
+        v.x = w * ((g[0].x * g[3].x + g[0].y * g[3].y) - (g[1].x * g[2].x + g[1].y * g[2].y));
+        v.y = w * ((g[0].y * g[3].x - g[0].x * g[3].y) - (g[1].y * g[2].x - g[1].x * g[2].y));
+    }
+    red[threadIdx.x] = v;
+    __syncthreads();
+    for (int w = 128; w > 0; w >>= 1) {
+        if (threadIdx.x < w) {
+            red[threadIdx.x].x += red[threadIdx.x + w].x;
+            red[threadIdx.x].y += red[threadIdx.x + w].y;
+        }
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) partial[blockIdx.y * static_cast<long long>(gridDim.x) + blockIdx.x] = red[0];
+}
+
 // ------------------------------------------------------------ emitters ------
 struct QeDev {
     int packed;             // rho and its history hold the upper triangle only (Hermitian)
@@ -3141,6 +3196,12 @@ struct chiml_dev {
         const double* phasor = nullptr;
     };
     std::vector<DftGroup> dgs;
+    struct FluxPlan {
+        FluxPlanDev dev{};
+        double2* partial = nullptr;  // [nfreq][blocks]
+        int blocks = 0;
+    };
+    std::vector<FluxPlan> flux_plans;
     std::vector<QeHost> qes;
     const QeHost* finish_with_sample = nullptr;  // the group whose population finish rides on this step's sample launch
     struct TfsfHost {  // one TFSF surface: its lines and its surface table (H adds, then E adds)
@@ -4915,6 +4976,28 @@ int chiml_dev_read_points(chiml_dev_t* c, int d, double* values, size_t cap, siz
     return CHIML_OK;
 }
 
+}  // extern "C"
+namespace {
+// The accumulators of group d with the samples of the open block added (in
+// d.tmp, leaving F as it is), enqueued on the context's stream.
+const double* dft_with_open_block(chiml_dev* c, const chiml_dev::DftGroup& d) {
+    const int kmax = c->steps_done / d.interval;
+    if ((kmax % kDftBlock) == kDftBlock - 1) return d.F;  // no open block
+    const size_t n = 2 * static_cast<size_t>(d.n) * d.nfreq;
+    HIP_TRY(hipMemcpyAsync(d.tmp, d.F, n * sizeof(double), hipMemcpyDeviceToDevice, c->stream));
+    const int last = kmax * d.interval;
+    if (c->prec == 32)
+        hipLaunchKernelGGL(k_dft_flush<float>, dim3((d.n + 255) / 256), dim3(256), 0, c->stream, static_cast<const float*>(d.stage),
+                           d.phasor, d.tmp, c->step_ctr.as<int>(), d.n, d.nfreq, d.interval, 1, last);
+    else
+        hipLaunchKernelGGL(k_dft_flush<double>, dim3((d.n + 255) / 256), dim3(256), 0, c->stream, static_cast<const double*>(d.stage),
+                           d.phasor, d.tmp, c->step_ctr.as<int>(), d.n, d.nfreq, d.interval, 1, last);
+    HIP_TRY(hipGetLastError());
+    return d.tmp;
+}
+}  // namespace
+extern "C" {
+
 int chiml_dev_read_dft_group(chiml_dev_t* c, int g, double* reim, size_t cap) {
     if (!c) return fail(nullptr, CHIML_E_INVALID, "null context");
     if (g < 0 || g >= static_cast<int>(c->dgs.size())) return fail(c, CHIML_E_INVALID, "DFT group index out of range");
@@ -4924,32 +5007,84 @@ int chiml_dev_read_dft_group(chiml_dev_t* c, int g, double* reim, size_t cap) {
     if (!reim || cap < n) return fail(c, CHIML_E_INVALID, "buffer too small");
     std::lock_guard<std::mutex> lk(g_capture_mu);
     try {
-        int kmax = c->steps_done / d.interval;
-        bool partial = (kmax % kDftBlock) != kDftBlock - 1;
         std::vector<double> host(n);
-        if (partial) {
-            // Contract samples kfirst..kmax of the open block into a copy of F.
-            HIP_TRY(hipMemcpyAsync(d.tmp, d.F, n * sizeof(double), hipMemcpyDeviceToDevice, c->stream));
-            int last = kmax * d.interval;
-            if (c->prec == 32)
-                hipLaunchKernelGGL(k_dft_flush<float>, dim3((d.n + 255) / 256), dim3(256), 0, c->stream, static_cast<const float*>(d.stage),
-                                   d.phasor, d.tmp, c->step_ctr.as<int>(), d.n, d.nfreq, d.interval, 1, last);
-            else
-                hipLaunchKernelGGL(k_dft_flush<double>, dim3((d.n + 255) / 256), dim3(256), 0, c->stream, static_cast<const double*>(d.stage),
-                                   d.phasor, d.tmp, c->step_ctr.as<int>(), d.n, d.nfreq, d.interval, 1, last);
-            HIP_TRY(hipGetLastError());
-            HIP_TRY(hipStreamSynchronize(c->stream));
-            HIP_TRY(hipMemcpy(host.data(), d.tmp, n * sizeof(double), hipMemcpyDeviceToHost));
-        } else {
-            HIP_TRY(hipStreamSynchronize(c->stream));
-            HIP_TRY(hipMemcpy(host.data(), d.F, n * sizeof(double), hipMemcpyDeviceToHost));
-        }
+        const double* F = dft_with_open_block(c, d);
+        HIP_TRY(hipStreamSynchronize(c->stream));
+        HIP_TRY(hipMemcpy(host.data(), F, n * sizeof(double), hipMemcpyDeviceToHost));
         // device layout [f][s] -> ABI layout [s][f]
         for (int f = 0; f < d.nfreq; ++f)
             for (int sm = 0; sm < d.n; ++sm) {
                 reim[2 * (static_cast<size_t>(sm) * d.nfreq + f)] = host[2 * (static_cast<size_t>(f) * d.n + sm)];
                 reim[2 * (static_cast<size_t>(sm) * d.nfreq + f) + 1] = host[2 * (static_cast<size_t>(f) * d.n + sm) + 1];
             }
+    } catch (std::exception& e) {
+        return fail(c, CHIML_E_HIP, e.what());
+    }
+    return CHIML_OK;
+}
+
+int chiml_dev_flux_plan(chiml_dev_t* c, int nface, const int* npt, const int* const* ids, const double* cw, const double* const* sw, int* plan) {
+    if (!c) return fail(nullptr, CHIML_E_INVALID, "null context");
+    if (nface < 1 || nface > kFluxFaces || !npt || !ids || !cw || !sw || !plan) return fail(c, CHIML_E_INVALID, "invalid argument");
+    if (c->dgs.empty() || c->dgs[0].n == 0) return fail(c, CHIML_E_INVALID, "no flux samples");
+    std::lock_guard<std::mutex> lk(g_capture_mu);
+    try {
+        chiml_dev::FluxPlan pl;
+        FluxPlanDev& d = pl.dev;
+        d.nface = nface;
+        for (int f = 0; f < nface; ++f) {
+            if (npt[f] < 0) throw std::runtime_error("flux plan: point count");
+            d.npt[f] = npt[f];
+            d.start[f + 1] = d.start[f] + (npt[f] + 255) / 256 * 256;
+            for (int k = 0; k < 4; ++k) d.cw[f][k] = cw[4 * f + k];
+        }
+        const size_t total = d.start[nface];
+        std::vector<int> hi(16 * std::max<size_t>(total, 1), -1);
+        std::vector<double> hw(std::max<size_t>(total, 1), 0.0);
+        for (int f = 0; f < nface; ++f)
+            for (int p = 0; p < npt[f]; ++p) {
+                hw[d.start[f] + p] = sw[f][p];
+                for (int k = 0; k < 16; ++k) {
+                    const int id = ids[f][static_cast<size_t>(k) * npt[f] + p];
+                    if (id >= c->dgs[0].n) throw std::runtime_error("flux plan: sample index out of range");
+                    hi[k * total + d.start[f] + p] = id;
+                }
+            }
+        d.ids = c->upload<int>(hi.data(), hi.size());
+        d.sw = c->upload<double>(hw.data(), hw.size());
+        pl.blocks = static_cast<int>(total / 256);
+        pl.partial = reinterpret_cast<double2*>(c->zeros<double>(2 * static_cast<size_t>(std::max(pl.blocks, 1)) * c->dgs[0].nfreq));
+        *plan = static_cast<int>(c->flux_plans.size());
+        c->flux_plans.push_back(pl);
+    } catch (std::exception& e) {
+        return fail(c, CHIML_E_HIP, e.what());
+    }
+    return CHIML_OK;
+}
+
+int chiml_dev_flux(chiml_dev_t* c, int plan, double nt, double* reim) {
+    if (!c) return fail(nullptr, CHIML_E_INVALID, "null context");
+    if (plan < 0 || plan >= static_cast<int>(c->flux_plans.size()) || !reim) return fail(c, CHIML_E_INVALID, "invalid argument");
+    const chiml_dev::FluxPlan& pl = c->flux_plans[plan];
+    const chiml_dev::DftGroup& d = c->dgs[0];
+    const int nf = d.nfreq, nb = pl.blocks;
+    std::fill(reim, reim + 2 * static_cast<size_t>(pl.dev.nface) * nf, 0.0);
+    if (nb == 0) return CHIML_OK;
+    std::lock_guard<std::mutex> lk(g_capture_mu);
+    try {
+        const double* F = dft_with_open_block(c, d);
+        hipLaunchKernelGGL(k_flux_faces, dim3(nb, nf), dim3(256), 0, c->stream, pl.dev, reinterpret_cast<const double2*>(F), d.n, 1.0 / (nt * nt),
+                           pl.partial);
+        HIP_TRY(hipGetLastError());
+        HIP_TRY(hipStreamSynchronize(c->stream));
+        std::vector<double2> part(static_cast<size_t>(nb) * nf);
+        HIP_TRY(hipMemcpy(part.data(), pl.partial, part.size() * sizeof(double2), hipMemcpyDeviceToHost));
+        for (int fc = 0; fc < pl.dev.nface; ++fc)
+            for (int f = 0; f < nf; ++f)
+                for (int b = pl.dev.start[fc] / 256; b < pl.dev.start[fc + 1] / 256; ++b) {
+                    reim[2 * (static_cast<size_t>(fc) * nf + f)] += part[static_cast<size_t>(f) * nb + b].x;
+                    reim[2 * (static_cast<size_t>(fc) * nf + f) + 1] += part[static_cast<size_t>(f) * nb + b].y;
+                }
     } catch (std::exception& e) {
         return fail(c, CHIML_E_HIP, e.what());
     }

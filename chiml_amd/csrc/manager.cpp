@@ -159,6 +159,7 @@ struct FluxBox {
     bool frontBack = false;  // the box extends in all three directions
     std::array<int, 3> sz{};  // sz_ of the box
     bool save = false;        // write <name>_fields.dat with the output files
+    int plan = -1;            // the faces' tables on the device (fluxPlan)
     // loaded incident fields times -1, the starting values of each face's
     // combined Ej, Ek, Hj, Hk [freq][transCor1][cor] (loadFields(-1.0), parallelFlux.hpp:664-722)
     std::vector<std::array<std::vector<cplx>, 4>> loaded;
@@ -549,6 +550,7 @@ class FDTDField {
     // incident flux per frequency from the TFSF incident records (getFlux's incident column)
     std::vector<cplx> fluxIncd(int f);
     std::vector<std::vector<cplx>> fluxFaces(int f);
+    int fluxPlan(int f);
     // per face the combined Ej, Ek, Hj, Hk [freq][transCor1][cor] (empty where absent)
     std::vector<std::array<std::vector<cplx>, 4>> fluxFields(int f);
     void saveFluxFields(int f, const std::string& path);
@@ -1956,14 +1958,120 @@ std::vector<std::array<std::vector<cplx>, 4>> FDTDField::fluxFields(int fi) {
     return out;
 }
 
+// simpson() as weights: the result for f is sum_i w[i] f[i].
+static std::vector<double> simpson_weights(int n, double d) {
+    std::vector<double> w(n, 0.0);
+    std::vector<cplx> unit(n, cplx(0.0, 0.0));
+    if (n < 8) {
+        for (int i = 0; i < n; ++i) {
+            unit[i] = 1.0;
+            w[i] = simpson(unit.data(), n, d).real();
+            unit[i] = 0.0;
+        }
+        return w;
+    }
+    if (n % 2 == 0) {
+        for (int i = 0; i < (n - 2) / 2; i++) {
+            w[2 * i] += d / 6.0;
+            w[2 * i + 1] += 4.0 * d / 6.0;
+            w[2 * i + 2] += d / 6.0;
+        }
+        for (int i = 1; i < n / 2; i++) {
+            w[2 * i - 1] += d / 6.0;
+            w[2 * i] += 4.0 * d / 6.0;
+            w[2 * i + 1] += d / 6.0;
+        }
+        for (int i : {0, 1, n - 1, n - 2}) w[i] += d / 4.0;
+    } else {
+        for (int i = 0; i < (n - 1) / 2; i++) {
+            w[2 * i] += d / 3.0;
+            w[2 * i + 1] += 4.0 * d / 3.0;
+            w[2 * i + 2] += d / 3.0;
+        }
+    }
+    return w;
+}
+
+// The faces of box fi as tables for the device (fluxFields' averaging and
+// fluxFaces' integration), uploaded at the first read of its flux.
+int FDTDField::fluxPlan(int fi) {
+    FluxBox& fb = fluxes.at(fi);
+    if (fb.plan >= 0) return fb.plan;
+    const int nface = static_cast<int>(fb.faces.size());
+    std::vector<int> npt(nface);
+    std::vector<std::vector<int>> ids(nface);
+    std::vector<std::vector<double>> sw(nface);
+    std::vector<double> cw(4 * static_cast<size_t>(nface), 0.0);
+    for (int v = 0; v < nface; ++v) {
+        Face& f = fb.faces[v];
+        const int n1 = f.sz[f.transCor1], n2 = f.sz[f.cor], np = n1 * n2;
+        npt[v] = np;
+        ids[v].assign(16 * static_cast<size_t>(np), -1);
+        sw[v].assign(np, 0.0);
+        std::vector<Store>* st[4] = {&f.Ej, &f.Ek, &f.Hj, &f.Hk};
+        const int pad[4] = {f.padEj, f.padEk, f.padHj, f.padHk};
+        for (int k = 0; k < 4; ++k) {
+            if (st[k]->empty()) continue;
+            const int nOff = pad[k] >= 0 ? 2 : 1;
+            cw[4 * v + k] = 1.0 / static_cast<double>(st[k]->size() * nOff);
+            int slot = 0;
+            for (auto& s : *st[k])
+                for (int o = 0; o < nOff; ++o, ++slot) {
+                    if (slot >= 4) throw std::logic_error("more than four samples per flux face point");
+                    for (int i1 = 0; i1 < n1; ++i1)
+                        for (int i2 = 0; i2 < n2; ++i2) {
+                            std::array<int, 3> q = {{0, 0, 0}};
+                            q[f.transCor1] = i1;
+                            q[f.cor] = i2;
+                            if (o == 1) q[pad[k]] += 1;
+                            if (q[0] >= s.n[0] || q[1] >= s.n[1] || q[2] >= s.n[2]) continue;
+                            ids[v][(4 * k + slot) * static_cast<size_t>(np) + i1 * n2 + i2] =
+                                s.ids[q[0] + static_cast<size_t>(s.n[0]) * (q[1] + static_cast<size_t>(s.n[1]) * q[2])];
+                        }
+                }
+        }
+        const double d1 = IP.d[f.transCor1], d2 = IP.d[f.cor];
+        std::vector<double> w1(n1, 1.0), w2(n2, 1.0);
+        if (n1 > 1 && n2 > 1) {
+            w1 = simpson_weights(n1, d1);
+            w2 = simpson_weights(n2, d2);
+        } else if (n2 > 1) {
+            w2 = simpson_weights(n2, d2);
+        } else {
+            w1 = simpson_weights(n1, d1);
+        }
+        for (int i1 = 0; i1 < n1; ++i1)
+            for (int i2 = 0; i2 < n2; ++i2) sw[v][static_cast<size_t>(i1) * n2 + i2] = w1[i1] * w2[i2];
+    }
+    std::vector<const int*> pi(nface);
+    std::vector<const double*> pw(nface);
+    for (int v = 0; v < nface; ++v) {
+        pi[v] = ids[v].data();
+        pw[v] = sw[v].data();
+    }
+    if (chiml_dev_flux_plan(dev_, nface, npt.data(), pi.data(), cw.data(), pw.data(), &fb.plan) != CHIML_OK)
+        throw std::runtime_error(chiml_dev_last_error(dev_));
+    return fb.plan;
+}
+
 // Per face and frequency: tempFlux = fluxConv_ * weight_ * simps2D(...).
 std::vector<std::vector<cplx>> FDTDField::fluxFaces(int fi) {
     FluxBox& fb = fluxes.at(fi);
-    const auto fields = fluxFields(fi);
     int steps = 0;
     chiml_dev_steps_done(dev_, &steps);
     const double nt = steps / fb.timeInt + 1;
     std::vector<std::vector<cplx>> out;
+    if (fb.loaded.empty() && ndft > 0) {  // combined, multiplied and integrated on the device
+        std::vector<double> reim(2 * fb.faces.size() * nfreq);
+        if (chiml_dev_flux(dev_, fluxPlan(fi), nt, reim.data()) != CHIML_OK) throw std::runtime_error(chiml_dev_last_error(dev_));
+        for (size_t v = 0; v < fb.faces.size(); ++v) {
+            std::vector<cplx>& fv = out.emplace_back(nfreq, 0.0);
+            for (int k = 0; k < nfreq; ++k)
+                fv[k] = fb.conv * fb.faces[v].weight * cplx(reim[2 * (v * nfreq + k)], reim[2 * (v * nfreq + k) + 1]);
+        }
+        return out;
+    }
+    const auto fields = fluxFields(fi);
     for (size_t v = 0; v < fb.faces.size(); ++v) {
         const Face& f = fb.faces[v];
         std::vector<cplx>& fv = out.emplace_back(nfreq, 0.0);
@@ -2266,13 +2374,14 @@ int chiml_sim_freq_values(chiml_sim_t* s, int d, double* reim, size_t cap) {
 int chiml_sim_flux(chiml_sim_t* s, int f, double* reim, size_t cap, int* nfreq) {
     if (!s || !nfreq) return sim_fail("null argument");
     try {
+        (void)s->f->fluxes.at(f);
+        *nfreq = s->f->nfreq;
+        if (!reim || cap < 2 * static_cast<size_t>(s->f->nfreq)) return CHIML_OK;  // the count alone
         auto v = s->f->flux(f);
-        *nfreq = static_cast<int>(v.size());
-        if (reim && cap >= 2 * v.size())
-            for (size_t k = 0; k < v.size(); ++k) {
-                reim[2 * k] = v[k].real();
-                reim[2 * k + 1] = v[k].imag();
-            }
+        for (size_t k = 0; k < v.size(); ++k) {
+            reim[2 * k] = v[k].real();
+            reim[2 * k + 1] = v[k].imag();
+        }
         return CHIML_OK;
     } catch (std::exception& e) {
         return sim_fail(e.what());

@@ -251,6 +251,17 @@ int chiml_dev_read_field(chiml_dev_t* ctx, int comp, double* host);
 int chiml_dev_read_points(chiml_dev_t* ctx, int d, double* values, size_t cap, size_t* nsamples);
 /* DFT accumulators as [ndft][nfreq] complex (re, im interleaved). */
 int chiml_dev_read_dft(chiml_dev_t* ctx, double* reim, size_t cap);
+/* Flux through the faces of a box, reduced on the device from the DFT
+ * accumulators of group 0 (the flux boxes').  chiml_dev_flux_plan uploads the
+ * faces' tables once and returns the plan's number: face f has npt[f] points;
+ * ids[f] is [16][npt[f]], for each of Ej, Ek, Hj, Hk the up to four DFT samples
+ * averaged onto a point (-1: none); cw[4 f ..] their weights; sw[f][p] the
+ * integration weight of point p.  chiml_dev_flux writes, per face and
+ * frequency (face-major), the complex sum over the points of
+ * sw (Ej Hk* - Ek Hj*) / nt^2. */
+int chiml_dev_flux_plan(chiml_dev_t* c, int nface, const int* npt, const int* const* ids, const double* cw, const double* const* sw, int* plan);
+int chiml_dev_flux(chiml_dev_t* c, int plan, double nt, double* reim);
+
 /* DFT group g (0 = the ndft cells, as chiml_dev_read_dft; 1.. = dftg[g - 1]):
  * reim[(cell * nfreq + f) * 2 + {0,1}].  Replaces the accumulators read by
  * parallelDetectorFREQ_Base::collectFreqFields (src/DTC/parallelDTC_FREQ.hpp:270-296). */
