@@ -41,10 +41,12 @@ thread_local std::string g_sim_err;  // last error of this host thread
 
 // Runs f(lo, hi, t) over [0, n) split into contiguous chunks, one per host
 // thread (up to 16); the first exception thrown by any chunk is rethrown.
+// cells: the grid cells the range covers; a thread takes 8192 at least (starting
+// one costs about as much as testing 2000 cells).
 template <typename F>
-int parallel_chunks(int n, F f) {
+int parallel_chunks(int n, size_t cells, F f) {
     int nt = static_cast<int>(std::thread::hardware_concurrency());
-    nt = std::max(1, std::min({nt, 16, n}));
+    nt = std::max(1, std::min({nt, 16, n, static_cast<int>(std::min<size_t>(cells / 8192 + 1, 16))}));
     std::vector<std::thread> th;
     std::vector<std::exception_ptr> err(nt);
     for (int t = 0; t < nt; ++t) {
@@ -567,7 +569,8 @@ class FDTDField {
 
   private:
     int objAt(std::array<double, 3> pt, bool ml) const;
-    void objAt2(const std::array<double, 3>& pt, int& withML, int& withoutML) const;
+    void objAt2(const std::array<double, 3>& pt, const std::vector<int>& cand, int& withML, int& withoutML) const;
+    void rowObjects(double y, double z, std::vector<int>& cand) const;
     void scanMatInPML();
 };
 
@@ -581,17 +584,30 @@ int FDTDField::objAt(std::array<double, 3> pt, bool ml) const {
     return id;
 }
 
-// objAt(pt, true) and objAt(pt, false) in one pass over the objects.
-void FDTDField::objAt2(const std::array<double, 3>& pt, int& withML, int& withoutML) const {
-    withML = withoutML = 0;
+// The objects, in order, that may hold a point of the x row at (y, z):
+// spheres that do not reach the row are left out (most of a grid's rows).
+void FDTDField::rowObjects(double y, double z, std::vector<int>& cand) const {
+    cand.clear();
     for (size_t oo = 1; oo < IP.objs.size(); ++oo) {
         const Object& o = *IP.objs[oo];
-        bool relevant = o.ML || !o.pols.empty() || o.anyEpsNotOne() || o.mu != 1.0;
-        if (!relevant) continue;
+        if (!(o.ML || !o.pols.empty() || o.anyEpsNotOne() || o.mu != 1.0)) continue;
+        if (o.shape == Shape::SPHERE) {
+            const double r = std::max(o.geo[0], o.geoML[0]) + 1e-3 * IP.d[0], dy = y - o.loc[1], dz = z - o.loc[2];
+            if (dy * dy + dz * dz > r * r) continue;
+        }
+        cand.push_back(static_cast<int>(oo));
+    }
+}
+
+// objAt(pt, true) and objAt(pt, false) in one pass over the row's objects.
+void FDTDField::objAt2(const std::array<double, 3>& pt, const std::vector<int>& cand, int& withML, int& withoutML) const {
+    withML = withoutML = 0;
+    for (int oo : cand) {
+        const Object& o = *IP.objs[oo];
         const bool a = o.isObj(pt, IP.d[0], true);
         const bool b = o.ML ? o.isObj(pt, IP.d[0], false) : a;
-        if (a) withML = static_cast<int>(oo);
-        if (b) withoutML = static_cast<int>(oo);
+        if (a) withML = oo;
+        if (b) withoutML = oo;
     }
 }
 
@@ -672,7 +688,7 @@ FDTDField::FDTDField(const std::string& deck) : IP(parseInputs(deck)) {
     // ---- material maps ------------------------------------------------------
     std::vector<int> ecomps = is3D ? std::vector<int>{0, 1, 2} : std::vector<int>{2};
     std::vector<int> hcomps = is3D ? std::vector<int>{3, 4, 5} : std::vector<int>{3, 4};
-    std::vector<std::vector<int>> physOf(6);  // object id per point (geoML), per component
+    std::unique_ptr<int[]> physOf[6];  // object id per point (geoML), per component
     std::vector<std::vector<uint8_t>> matE(3);
     std::vector<double> ceT[3], ievT[3];
     std::vector<int> flT[3], psT[3];
@@ -702,7 +718,7 @@ FDTDField::FDTDField(const std::string& deck) : IP(parseInputs(deck)) {
     for (int c : ecomps) {
         const int* st = kStag[c];
         matE[c].assign(N, 0);
-        physOf[c].assign(N, 0);
+        physOf[c].reset(new int[N]);
         // Material ids are numbered in order of first appearance in x-fastest
         // scan order.  Chunks of z-planes (y-rows in 2D) are scanned in
         // parallel with local numbering, then merged in chunk order, which
@@ -712,9 +728,10 @@ FDTDField::FDTDField(const std::string& deck) : IP(parseInputs(deck)) {
         std::vector<std::vector<Key>> lkeys(16);
         std::vector<std::array<int, 6>> lbox(16, std::array<int, 6>{{nx, -1, ny, -1, nz, -1}});
         std::vector<std::pair<int, int>> lrange(16, {0, 0});
-        const int nt = parallel_chunks(outer, [&](int lo, int hi, int t) {
+        const int nt = parallel_chunks(outer, N, [&](int lo, int hi, int t) {
             lrange[t] = {lo, hi};
             std::map<Key, int> lid;
+            std::vector<int> cand;
             Key last{-1, 0.0, -1};
             int lastId = -1;
             auto& bx = lbox[t];
@@ -722,12 +739,14 @@ FDTDField::FDTDField(const std::string& deck) : IP(parseInputs(deck)) {
                 const int z0 = is3D ? o : 0, z1 = is3D ? o + 1 : 1;
                 const int y0 = is3D ? 0 : o, y1 = is3D ? ny : o + 1;
                 for (int z = z0; z < z1; ++z)
-                    for (int y = y0; y < y1; ++y)
+                    for (int y = y0; y < y1; ++y) {
+                        std::array<double, 3> pt = {{0.0, coord(1, y, 0.5 * st[1]), is3D ? coord(2, z, 0.5 * st[2]) : 0.0}};
+                        if (!is3D) pt[2] = (-1 + 0.5 * st[2] - (nAll[2] - nAll[2] % 2) / 2.0) * IP.d[2];  // kk - 1 with kk = 0
+                        rowObjects(pt[1], pt[2], cand);
                         for (int x = 0; x < nx; ++x) {
-                            std::array<double, 3> pt = {{coord(0, x, 0.5 * st[0]), coord(1, y, 0.5 * st[1]), is3D ? coord(2, z, 0.5 * st[2]) : 0.0}};
-                            if (!is3D) pt[2] = (-1 + 0.5 * st[2] - (nAll[2] - nAll[2] % 2) / 2.0) * IP.d[2];  // kk - 1 with kk = 0
+                            pt[0] = coord(0, x, 0.5 * st[0]);
                             int phys, epsObj;
-                            objAt2(pt, phys, epsObj);
+                            objAt2(pt, cand, phys, epsObj);
                             const double eps = IP.objs[epsObj]->eps[c];
                             const size_t i = x + static_cast<size_t>(nx) * (y + static_cast<size_t>(ny) * z);
                             physOf[c][i] = phys;
@@ -763,6 +782,7 @@ FDTDField::FDTDField(const std::string& deck) : IP(parseInputs(deck)) {
                                 bx[5] = std::max(bx[5], z + 1);
                             }
                         }
+                    }
             }
         });
         // merge: global ids in first-appearance order over the chunks
@@ -791,7 +811,7 @@ FDTDField::FDTDField(const std::string& deck) : IP(parseInputs(deck)) {
                 remap[t].push_back(static_cast<uint8_t>(id));
             }
         }
-        parallel_chunks(nt, [&](int lo, int hi, int) {
+        parallel_chunks(nt, N, [&](int lo, int hi, int) {
             for (int t = lo; t < hi; ++t) {
                 const size_t plane = is3D ? static_cast<size_t>(nx) * ny : static_cast<size_t>(nx);
                 const size_t b = static_cast<size_t>(lrange[t].first) * plane, e = static_cast<size_t>(lrange[t].second) * plane;
@@ -831,24 +851,27 @@ FDTDField::FDTDField(const std::string& deck) : IP(parseInputs(deck)) {
         P.nmat_h[c] = 1;
         P.mat_h_ch[c] = &chv;
         const int* st = kStag[hc];
-        physOf[hc].assign(N, 0);
-        std::vector<int> muObj(N, 0);
-        parallel_chunks(nz * ny, [&](int lo, int hi, int) {
+        physOf[hc].reset(new int[N]);
+        bool anyMu = false;
+        for (auto& op : IP.objs) anyMu = anyMu || op->mu != 1.0;
+        std::vector<int> muObj(anyMu ? N : 0);
+        parallel_chunks(nz * ny, N, [&](int lo, int hi, int) {
+            std::vector<int> cand;
             for (int r = lo; r < hi; ++r) {
                 const int z = r / ny, y = r % ny;
+                std::array<double, 3> pt = {{0.0, coord(1, y, 0.5 * st[1]), is3D ? coord(2, z, 0.5 * st[2]) : 0.0}};
+                if (!is3D) pt[2] = (-1 + 0.5 * st[2] - (nAll[2] - nAll[2] % 2) / 2.0) * IP.d[2];  // kk - 1 with kk = 0
+                rowObjects(pt[1], pt[2], cand);
                 for (int x = 0; x < nx; ++x) {
-                    std::array<double, 3> pt = {{coord(0, x, 0.5 * st[0]), coord(1, y, 0.5 * st[1]), is3D ? coord(2, z, 0.5 * st[2]) : 0.0}};
-                    if (!is3D) pt[2] = (-1 + 0.5 * st[2] - (nAll[2] - nAll[2] % 2) / 2.0) * IP.d[2];  // kk - 1 with kk = 0
+                    pt[0] = coord(0, x, 0.5 * st[0]);
                     const size_t i = x + static_cast<size_t>(nx) * (y + static_cast<size_t>(ny) * z);
                     int phys, mo;
-                    objAt2(pt, phys, mo);
+                    objAt2(pt, cand, phys, mo);
                     physOf[hc][i] = phys;
-                    muObj[i] = mo;
+                    if (anyMu) muObj[i] = mo;
                 }
             }
         });
-        bool anyMu = false;
-        for (auto& op : IP.objs) anyMu = anyMu || op->mu != 1.0;
         if (!anyMu) continue;
         std::map<double, int> idOf;
         chT[c].clear();
@@ -930,15 +953,15 @@ FDTDField::FDTDField(const std::string& deck) : IP(parseInputs(deck)) {
                     }
                 return es * ms;
             };
-            std::vector<double> etaLo, etaHi;
-            for (int pl = 0; pl < Ta; ++pl) {
-                double v = etaPlane(pl);
-                if (v != 0.0) etaLo.push_back(v);
-            }
-            for (int pl = na - Ta; pl < na; ++pl) {
-                double v = etaPlane(pl);
-                if (v != 0.0 && static_cast<int>(etaHi.size()) < Ta) etaHi.push_back(v);
-            }
+            std::vector<double> etaLo, etaHi, eta(2 * static_cast<size_t>(Ta));
+            const size_t plane = static_cast<size_t>(ps[(a + 1) % 3]) * ps[(a + 2) % 3];
+            parallel_chunks(2 * Ta, 2 * Ta * plane, [&](int lo, int hi, int) {
+                for (int k = lo; k < hi; ++k) eta[k] = etaPlane(k < Ta ? k : na - 2 * Ta + k);
+            });
+            for (int pl = 0; pl < Ta; ++pl)
+                if (eta[pl] != 0.0) etaLo.push_back(eta[pl]);
+            for (int pl = Ta; pl < 2 * Ta; ++pl)
+                if (eta[pl] != 0.0 && static_cast<int>(etaHi.size()) < Ta) etaHi.push_back(eta[pl]);
             std::vector<double>& b = prof[comp][a][0];
             std::vector<double>& cd = prof[comp][a][1];
             std::vector<double>& kinv = prof[comp][a][2];
@@ -1655,23 +1678,28 @@ FDTDField::FDTDField(const std::string& deck) : IP(parseInputs(deck)) {
                     }
                     psiWords += w;
                 }
+        // dispersive cells inside and outside the interior, by pole set
+        std::vector<double> dispIn(pcount.size(), 0.0), dispOut(pcount.size(), 0.0);
         for (int c : ecomps) {
             const int* b = dispBox[c];
             for (int z = b[4]; z < b[5]; ++z)
-                for (int y = b[2]; y < b[3]; ++y)
+                for (int y = b[2]; y < b[3]; ++y) {
+                    const uint8_t* row = &matE[c][static_cast<size_t>(nx) * (y + static_cast<size_t>(ny) * z)];
                     for (int x = b[0]; x < b[1]; ++x) {
-                        int ps = psT[c][matE[c][x + static_cast<size_t>(nx) * (y + static_cast<size_t>(ny) * z)]];
-                        if (ps < 0) continue;
-                        dispMin += 2.0 * s + pcount[ps] * 4.0 * s;
-                        if (split) {
-                            // pole kernel: P and J read and written, E read, current sum written;
-                            // the E kernel reads the current sum back
-                            kbytes["ade"] += pcount[ps] * 4.0 * s + 2.0 * s;
-                            kbytes[inInt(x, y, z) ? "update_e" : "update_e_pml"] += s;
-                        } else {
-                            kbytes[inInt(x, y, z) ? "update_e" : "update_e_pml"] += pcount[ps] * 4.0 * s;
-                        }
+                        const int ps = psT[c][row[x]];
+                        if (ps >= 0) (inInt(x, y, z) ? dispIn : dispOut)[ps] += 1.0;
                     }
+                }
+        }
+        for (size_t ps = 0; ps < pcount.size(); ++ps) {
+            const double n = dispIn[ps] + dispOut[ps];
+            dispMin += n * (2.0 * s + pcount[ps] * 4.0 * s);
+            // split: the pole update reads and writes P and J, reads E and writes
+            // the current sum, and the E kernel reads the current sum back
+            const double each = split ? s : pcount[ps] * 4.0 * s;
+            if (split) kbytes["ade"] += n * (pcount[ps] * 4.0 * s + 2.0 * s);
+            if (dispIn[ps] > 0) kbytes["update_e"] += dispIn[ps] * each;
+            if (dispOut[ps] > 0) kbytes["update_e_pml"] += dispOut[ps] * each;
         }
         // the opt-in fused step (3D FP32 with the split layout): one pass that
         // reads and writes every field word once, three material bytes per
@@ -1679,16 +1707,10 @@ FDTDField::FDTDField(const std::string& deck) : IP(parseInputs(deck)) {
         if (split && rows) {
             kbytes["update_fused"] = cells * (2.0 * (nE + nH) * s + nE) + psiWords * 2.0 * s;
             kbytes["update_ade"] = 0.0;
-            for (int c : ecomps) {
-                const int* b = dispBox[c];
-                for (int z = b[4]; z < b[5]; ++z)
-                    for (int y = b[2]; y < b[3]; ++y)
-                        for (int x = b[0]; x < b[1]; ++x) {
-                            int ps = psT[c][matE[c][x + static_cast<size_t>(nx) * (y + static_cast<size_t>(ny) * z)]];
-                            if (ps < 0) continue;
-                            kbytes["update_ade"] += pcount[ps] * 4.0 * s + 2.0 * s;
-                            kbytes["update_fused"] += s;  // the pole-current sum read back
-                        }
+            for (size_t ps = 0; ps < pcount.size(); ++ps) {
+                const double n = dispIn[ps] + dispOut[ps];
+                kbytes["update_ade"] += n * (pcount[ps] * 4.0 * s + 2.0 * s);
+                kbytes["update_fused"] += n * s;  // the pole-current sum read back
             }
         }
         kbytes["ml_density"] = bytesML;
