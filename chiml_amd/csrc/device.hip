@@ -394,7 +394,15 @@ __device__ __forceinline__ void stv(T* p, const Pk<T, W>& v) {
 // Streaming forms for the words a kernel touches once (its own cells' field
 // values, CPML psi, pole currents, material ids): the nontemporal hint keeps
 // them from displacing the neighbour rows and planes the other threads of
-// the sweep still read from L2 (about 15% on the 256^3 step, FP32).
+// the sweep still read from L2.  A grid whose six fields fit the 256 MB
+// memory-side cache with room to spare does better without: the words of one
+// sweep then come from that cache in the next.  Measured without and with the
+// hint, us a step: FP32 128^3 51 and 58, 192^3 (170 MB) 123 and 135, 200^3
+// 152 and 153, 224^3 215 and 196, 256^3 324 and 274; FP64 128^3 93 and 108,
+// 152^3 (168 MB) 144 and 155, 160^3 172 and 166.  (Keeping only part of a
+// larger grid's rows cached lost: 256^3 with 30% of the rows 295.)  Emitter
+// state that each step streams counts with the fields.
+constexpr bool streams_past_caches(double bytes) { return bytes > 185e6; }
 template <typename T, int W>
 using NtVec = T __attribute__((ext_vector_type(W)));
 template <typename T, int W>
@@ -411,6 +419,16 @@ __device__ __forceinline__ void stv_nt(T* p, const Pk<T, W>& v) {
 #pragma unroll
     for (int w = 0; w < W; ++w) x[w] = v.v[w];
     __builtin_nontemporal_store(x, reinterpret_cast<NtVec<T, W>*>(p));
+}
+template <bool NT, typename T, int W>
+__device__ __forceinline__ Pk<T, W> ldc(const T* p) {
+    if constexpr (NT) return ldv_nt<T, W>(p);
+    else return ldv<T, W>(p);
+}
+template <bool NT, typename T, int W>
+__device__ __forceinline__ void stc(T* p, const Pk<T, W>& v) {
+    if constexpr (NT) stv_nt<T, W>(p, v);
+    else stv<T, W>(p, v);
 }
 template <typename T, int W>
 __device__ __forceinline__ Pk<T, W> zpk() {
@@ -523,7 +541,7 @@ __device__ __forceinline__ void pml_group(const PmlDev<T>& p, int ax, int pos0, 
 // One CPML term of a group along derivative axis AX (pml_group's arithmetic):
 // load() fetches psi and the profiles with the component's other loads, apply()
 // forms the term and stores psi.  ON = false: a region without this term.
-template <typename T, int W, int AX, bool ON>
+template <typename T, int W, int AX, bool ON, bool NT>
 struct PsiTerm {
     int s;
     T* at;
@@ -540,7 +558,7 @@ struct PsiTerm {
         else if (AX == 1) pi = x0 + static_cast<long long>(px) * (s + static_cast<long long>(p.S[1]) * z);
         else pi = x0 + static_cast<long long>(px) * (y + static_cast<long long>(ny) * s);
         at = p.psi[AX] + pi;
-        ps = ldv_nt<T, W>(at);
+        ps = ldc<NT, T, W>(at);
         if (AX == 0) {
             const Pk<T, W> vb = ldv<T, W>(p.b[0] + pos), vc = ldv<T, W>(p.cd[0] + pos), vk = ldv<T, W>(p.kinv[0] + pos);
 #pragma unroll
@@ -568,7 +586,7 @@ struct PsiTerm {
             if (valid & (1u << w)) ps.v[w] = psi;
             term[w] = fma(ki[k], term[w], psi);
         }
-        stv_nt<T, W>(at, ps);
+        stc<NT, T, W>(at, ps);
     }
 };
 
@@ -601,7 +619,7 @@ __device__ __forceinline__ unsigned cells_inside(int x0, int nx, int Tx) {
 // PX / PYZ: the group may lie in an x / in a y or z CPML slab.
 // nb: the next lane of the wave holds the next group of the same row, so the
 // first value of that group comes by a lane shuffle instead of a load.
-template <typename T, int W, bool PX, bool PYZ, bool SRC, bool FMA>
+template <typename T, int W, bool PX, bool PYZ, bool SRC, bool FMA, bool NT>
 __device__ __forceinline__ void h_group(const StepArgs<T>& a, int x0, int y, int z, bool nb = false) {
     const int nx = a.nx, ny = a.ny, nz = a.nz, px = a.px;
     const long long sy = px, sz = static_cast<long long>(px) * ny;
@@ -625,13 +643,13 @@ __device__ __forceinline__ void h_group(const StepArgs<T>& a, int x0, int y, int
             if (src) hv += src_value(a, 3 + c, x0 + w, y, z, step);
             h.v[w] = hv;
         }
-        stv_nt<T, W>(a.F[3 + c] + i, h);
+        stc<NT, T, W>(a.F[3 + c] + i, h);
     };
     if (yin && zin) {  // Hx += ch [dEy/dz - dEz/dy]
         const Pk<T, W> eyz = ldv<T, W>(Ey + i + sz), ezy = ldv<T, W>(Ez + i + sy);
-        Pk<T, W> h = ldv_nt<T, W>(a.F[3] + i);
-        PsiTerm<T, W, 2, PYZ> q1;
-        PsiTerm<T, W, 1, PYZ> q2;
+        Pk<T, W> h = ldc<NT, T, W>(a.F[3] + i);
+        PsiTerm<T, W, 2, PYZ, NT> q1;
+        PsiTerm<T, W, 1, PYZ, NT> q2;
         q1.load(a.pml[3], z, x0, y, z, px, ny);
         q2.load(a.pml[3], y, x0, y, z, px, ny);
 #pragma unroll
@@ -647,9 +665,9 @@ __device__ __forceinline__ void h_group(const StepArgs<T>& a, int x0, int y, int
     if (zin) {  // Hy += ch [dEz/dx - dEx/dz], x < nx - 1
         const Pk<T, W> exz = ldv<T, W>(Ex + i + sz);
         const T ezn = last ? T(0) : (nb ? ez_nb : Ez[i + W]);
-        Pk<T, W> h = ldv_nt<T, W>(a.F[4] + i);
-        PsiTerm<T, W, 0, PX> q1;
-        PsiTerm<T, W, 2, PYZ> q2;
+        Pk<T, W> h = ldc<NT, T, W>(a.F[4] + i);
+        PsiTerm<T, W, 0, PX, NT> q1;
+        PsiTerm<T, W, 2, PYZ, NT> q2;
         q1.load(a.pml[4], x0, x0, y, z, px, ny);
         q2.load(a.pml[4], z, x0, y, z, px, ny);
 #pragma unroll
@@ -665,9 +683,9 @@ __device__ __forceinline__ void h_group(const StepArgs<T>& a, int x0, int y, int
     if (yin) {  // Hz += ch [dEx/dy - dEy/dx], x < nx - 1
         const Pk<T, W> exy = ldv<T, W>(Ex + i + sy);
         const T eyn = last ? T(0) : (nb ? ey_nb : Ey[i + W]);
-        Pk<T, W> h = ldv_nt<T, W>(a.F[5] + i);
-        PsiTerm<T, W, 1, PYZ> q1;
-        PsiTerm<T, W, 0, PX> q2;
+        Pk<T, W> h = ldc<NT, T, W>(a.F[5] + i);
+        PsiTerm<T, W, 1, PYZ, NT> q1;
+        PsiTerm<T, W, 0, PX, NT> q2;
         q1.load(a.pml[5], y, x0, y, z, px, ny);
         q2.load(a.pml[5], x0, x0, y, z, px, ny);
 #pragma unroll
@@ -682,7 +700,7 @@ __device__ __forceinline__ void h_group(const StepArgs<T>& a, int x0, int y, int
     }
 }
 
-template <int W>
+template <int W, bool NT = true>
 __device__ __forceinline__ Pk<uint8_t, W> load_ids(const uint8_t* m, long long i) {
     if (!m) {
         Pk<uint8_t, W> z;
@@ -690,7 +708,7 @@ __device__ __forceinline__ Pk<uint8_t, W> load_ids(const uint8_t* m, long long i
         for (int w = 0; w < W; ++w) z.v[w] = 0;
         return z;
     }
-    return ldv_nt<uint8_t, W>(m + i);
+    return ldc<NT, uint8_t, W>(m + i);
 }
 
 // E of the W cells of a group from their curl acc, materials,
@@ -754,7 +772,7 @@ __device__ __forceinline__ Pk<T, W> e_finish_group(const StepArgs<T>& a, const M
 // the pole currents already advanced by ade_block.  PX, PYZ, FMA as in
 // h_group; mt: the material tables in LDS.
 // nb: the previous lane of the wave holds the previous group of the same row
-template <typename T, int W, bool PX, bool PYZ, bool SRC, bool FMA>
+template <typename T, int W, bool PX, bool PYZ, bool SRC, bool FMA, bool NT>
 __device__ __forceinline__ void e_group(const StepArgs<T>& a, const MatLds<T> (*mt)[CHIML_MAX_MAT], int x0, int y, int z,
                                         bool nb = false) {
     const int nx = a.nx, ny = a.ny, nz = a.nz, px = a.px;
@@ -771,8 +789,8 @@ __device__ __forceinline__ void e_group(const StepArgs<T>& a, const MatLds<T> (*
     const int step = src ? step_now(a.step, a.stepv) : 0;
     T d1[W], d2[W], t1[W], t2[W], acc[W];
     auto finish = [&](int c, unsigned valid) {
-        const Pk<uint8_t, W> id = load_ids<W>(a.mat_e[c], i);
-        Pk<T, W> e = ldv_nt<T, W>(a.F[c] + i);
+        const Pk<uint8_t, W> id = load_ids<W, NT>(a.mat_e[c], i);
+        Pk<T, W> e = ldc<NT, T, W>(a.F[c] + i);
         bool anyp = false;
 #pragma unroll
         for (int w = 0; w < W; ++w) anyp |= (mt[c][id.v[w]].poleset >= 0) && (valid & (1u << w));
@@ -791,13 +809,13 @@ __device__ __forceinline__ void e_group(const StepArgs<T>& a, const MatLds<T> (*
             const T jsum = m.poleset >= 0 ? js.v[w] : T(0);
             e.v[w] = fma(-m.inveps, jsum, fma(m.ce, acc[w], e_base));
         }
-        stv_nt<T, W>(a.F[c] + i, e);
+        stc<NT, T, W>(a.F[c] + i, e);
     };
     {  // Ex += ce [dHz/dy - dHy/dz], x < nx - 1
         const Pk<T, W> hzy = y > 0 ? ldv<T, W>(Hz + i - sy) : zpk<T, W>();
         const Pk<T, W> hyz = z > 0 ? ldv<T, W>(Hy + i - sz) : zpk<T, W>();
-        PsiTerm<T, W, 1, PYZ> q1;
-        PsiTerm<T, W, 2, PYZ> q2;
+        PsiTerm<T, W, 1, PYZ, NT> q1;
+        PsiTerm<T, W, 2, PYZ, NT> q2;
         q1.load(a.pml[0], y, x0, y, z, px, ny);
         q2.load(a.pml[0], z, x0, y, z, px, ny);
 #pragma unroll
@@ -813,8 +831,8 @@ __device__ __forceinline__ void e_group(const StepArgs<T>& a, const MatLds<T> (*
     if (yin) {  // Ey += ce [dHx/dz - dHz/dx]
         const Pk<T, W> hxz = z > 0 ? ldv<T, W>(Hx + i - sz) : zpk<T, W>();
         const T hzm = x0 > 0 ? (nb ? hz_nb : Hz[i - 1]) : T(0);
-        PsiTerm<T, W, 2, PYZ> q1;
-        PsiTerm<T, W, 0, PX> q2;
+        PsiTerm<T, W, 2, PYZ, NT> q1;
+        PsiTerm<T, W, 0, PX, NT> q2;
         q1.load(a.pml[1], z, x0, y, z, px, ny);
         q2.load(a.pml[1], x0, x0, y, z, px, ny);
 #pragma unroll
@@ -830,8 +848,8 @@ __device__ __forceinline__ void e_group(const StepArgs<T>& a, const MatLds<T> (*
     if (zin) {  // Ez += ce [dHy/dx - dHx/dy]
         const Pk<T, W> hxy = y > 0 ? ldv<T, W>(Hx + i - sy) : zpk<T, W>();
         const T hym = x0 > 0 ? (nb ? hy_nb : Hy[i - 1]) : T(0);
-        PsiTerm<T, W, 0, PX> q1;
-        PsiTerm<T, W, 1, PYZ> q2;
+        PsiTerm<T, W, 0, PX, NT> q1;
+        PsiTerm<T, W, 1, PYZ, NT> q2;
         q1.load(a.pml[2], x0, x0, y, z, px, ny);
         q2.load(a.pml[2], y, x0, y, z, px, ny);
 #pragma unroll
@@ -933,7 +951,7 @@ __device__ __forceinline__ bool int_group(const Box3& b, int blk, int& x0, int& 
 // (15 us less than a launch of its own on the 256^3 step).
 __host__ __device__ constexpr int ade_blocks(int ade_bpc) { return (3 * ade_bpc + 7) / 8 * 8; }
 
-template <typename T, int W, bool SRC>
+template <typename T, int W, bool SRC, bool NT>
 __device__ __forceinline__ void h3_int_sweep(const StepArgs<T>& a, const Box3& b, int nib, int ade_bpc, int bx) {
     const int nade = ade_blocks(ade_bpc);
     if (bx < nade) {
@@ -945,29 +963,29 @@ __device__ __forceinline__ void h3_int_sweep(const StepArgs<T>& a, const Box3& b
     if (!int_group<T, W>(b, xcd_block(bx - nade, nib), x0, y, z, col)) return;
     // consecutive threads walk a row: lane + 1 holds the next group unless this one ends the row
     const int lane = threadIdx.x & 63, gw = (b.x1 - b.x0) / W;
-    h_group<T, W, false, false, SRC, false>(a, x0, y, z, lane < 63 && col + 1 < gw);
+    h_group<T, W, false, false, SRC, false, NT>(a, x0, y, z, lane < 63 && col + 1 < gw);
 }
 
-template <typename T, int W, bool SRC, bool ADV>
+template <typename T, int W, bool SRC, bool ADV, bool NT>
 __global__ void __launch_bounds__(256) k_h3_int(StepArgs<T> a, Box3 b, int nib, int ade_bpc) {
-    h3_int_sweep<T, W, SRC>(a, b, nib, ade_bpc, blockIdx.x);
+    h3_int_sweep<T, W, SRC, NT>(a, b, nib, ade_bpc, blockIdx.x);
     if (ADV) advance_counter(a);
 }
 
-template <typename T, int W, bool SRC>
+template <typename T, int W, bool SRC, bool NT>
 __device__ __forceinline__ void e3_int_sweep(const StepArgs<T>& a, const MatLds<T> (*mt)[CHIML_MAX_MAT], const Box3& b, int bx, int nb) {
     int x0, y, z, col;
     if (!int_group<T, W>(b, xcd_block(bx, nb), x0, y, z, col)) return;
     const int lane = threadIdx.x & 63;
-    e_group<T, W, false, false, SRC, false>(a, mt, x0, y, z, lane > 0 && col > 0);
+    e_group<T, W, false, false, SRC, false, NT>(a, mt, x0, y, z, lane > 0 && col > 0);
 }
 
-template <typename T, int W, bool SRC>
+template <typename T, int W, bool SRC, bool NT>
 __global__ void __launch_bounds__(256) k_e3_int(StepArgs<T> a, Box3 b, int nm0, int nm1, int nm2) {
     __shared__ MatLds<T> mt[3][CHIML_MAX_MAT];
     const int nm[3] = {nm0, nm1, nm2};
     load_mat(a, mt, nm);
-    e3_int_sweep<T, W, SRC>(a, mt, b, blockIdx.x, gridDim.x);
+    e3_int_sweep<T, W, SRC, NT>(a, mt, b, blockIdx.x, gridDim.x);
 }
 
 // CPML slab groups: the union of the z slabs, the y slabs inside the z range
@@ -1014,33 +1032,33 @@ __device__ __forceinline__ bool slab_group(const SlabMap& m, unsigned t, int& x0
     return true;
 }
 
-template <typename T, int W, bool SRC>
+template <typename T, int W, bool SRC, bool NT>
 __device__ __forceinline__ void h3_slab_sweep(const StepArgs<T>& a, const SlabMap& m, int bx, int nb) {
     int x0, y, z, col, rowlen;
     if (!slab_group(m, static_cast<unsigned>(xcd_block(bx, nb)) * blockDim.x + threadIdx.x, x0, y, z, col, rowlen)) return;
     // the z- and y-slab regions start on row boundaries (nA is whole rows), so
     // lane + 1 holds the next group of the row unless this one ends it
-    h_group<T, W, true, true, SRC, false>(a, x0, y, z, (threadIdx.x & 63) < 63 && col + 1 < rowlen);
+    h_group<T, W, true, true, SRC, false, NT>(a, x0, y, z, (threadIdx.x & 63) < 63 && col + 1 < rowlen);
 }
 
-template <typename T, int W, bool SRC>
+template <typename T, int W, bool SRC, bool NT>
 __global__ void __launch_bounds__(256) k_h3_slab(StepArgs<T> a, SlabMap m) {
-    h3_slab_sweep<T, W, SRC>(a, m, blockIdx.x, gridDim.x);
+    h3_slab_sweep<T, W, SRC, NT>(a, m, blockIdx.x, gridDim.x);
 }
 
-template <typename T, int W, bool SRC>
+template <typename T, int W, bool SRC, bool NT>
 __device__ __forceinline__ void e3_slab_sweep(const StepArgs<T>& a, const MatLds<T> (*mt)[CHIML_MAX_MAT], const SlabMap& m, int bx, int nb) {
     int x0, y, z, col, rowlen;
     if (!slab_group(m, static_cast<unsigned>(xcd_block(bx, nb)) * blockDim.x + threadIdx.x, x0, y, z, col, rowlen)) return;
-    e_group<T, W, true, true, SRC, false>(a, mt, x0, y, z);  // (the lane shuffle measured slower here)
+    e_group<T, W, true, true, SRC, false, NT>(a, mt, x0, y, z);  // (the lane shuffle measured slower here)
 }
 
-template <typename T, int W, bool SRC>
+template <typename T, int W, bool SRC, bool NT>
 __global__ void __launch_bounds__(256) k_e3_slab(StepArgs<T> a, SlabMap m, int nm0, int nm1, int nm2) {
     __shared__ MatLds<T> mt[3][CHIML_MAX_MAT];
     const int nm[3] = {nm0, nm1, nm2};
     load_mat(a, mt, nm);
-    e3_slab_sweep<T, W, SRC>(a, mt, m, blockIdx.x, gridDim.x);
+    e3_slab_sweep<T, W, SRC, NT>(a, mt, m, blockIdx.x, gridDim.x);
 }
 
 // Whole-row layout (GridLayout::rows): the whole 3D sweep of a field in one
@@ -1051,7 +1069,7 @@ __global__ void __launch_bounds__(256) k_e3_slab(StepArgs<T> a, SlabMap m, int n
 // tails per step go away (5% on the 256^3 FP32 step).  Aligned FP64 grids keep
 // separate launches: there the interior kernel carries no CPML code and runs
 // at a higher occupancy than a merged kernel would.
-template <typename T, int W, bool SRC, bool FMA>
+template <typename T, int W, bool SRC, bool FMA, bool NT>
 __device__ __forceinline__ void h3_all_sweep(const StepArgs<T>& a, const Box3& b, const SlabMap& m, int nib, int nsbp,
                                              int ade_bpc, int bx) {
     const int nade = ade_blocks(ade_bpc);
@@ -1064,44 +1082,44 @@ __device__ __forceinline__ void h3_all_sweep(const StepArgs<T>& a, const Box3& b
     if (bx < nsbp) {
         int x0, y, z, col, rowlen;
         if (!slab_group(m, static_cast<unsigned>(xcd_block(bx, nsbp)) * blockDim.x + threadIdx.x, x0, y, z, col, rowlen)) return;
-        h_group<T, W, true, true, SRC, FMA>(a, x0, y, z, (threadIdx.x & 63) < 63 && col + 1 < rowlen);
+        h_group<T, W, true, true, SRC, FMA, NT>(a, x0, y, z, (threadIdx.x & 63) < 63 && col + 1 < rowlen);
         return;
     }
     bx -= nsbp;
     int x0, y, z, col;
     if (!int_group<T, W>(b, xcd_block(bx, nib), x0, y, z, col)) return;
     const int lane = threadIdx.x & 63, gw = (b.x1 - b.x0) / W;
-    h_group<T, W, true, false, SRC, FMA>(a, x0, y, z, lane < 63 && col + 1 < gw);
+    h_group<T, W, true, false, SRC, FMA, NT>(a, x0, y, z, lane < 63 && col + 1 < gw);
 }
 
-template <typename T, int W, bool SRC, bool ADV, bool FMA>
+template <typename T, int W, bool SRC, bool ADV, bool FMA, bool NT>
 __global__ void __launch_bounds__(256) k_h3_all(StepArgs<T> a, Box3 b, SlabMap m, int nib, int nsbp, int ade_bpc) {
-    h3_all_sweep<T, W, SRC, FMA>(a, b, m, nib, nsbp, ade_bpc, blockIdx.x);
+    h3_all_sweep<T, W, SRC, FMA, NT>(a, b, m, nib, nsbp, ade_bpc, blockIdx.x);
     if (ADV) advance_counter(a);
 }
 
-template <typename T, int W, bool SRC, bool FMA>
+template <typename T, int W, bool SRC, bool FMA, bool NT>
 __device__ __forceinline__ void e3_all_sweep(const StepArgs<T>& a, const MatLds<T> (*mt)[CHIML_MAX_MAT], const Box3& b, const SlabMap& m,
                                              int nib, int nsbp, int bx) {
     if (bx < nsbp) {
         int x0, y, z, col, rowlen;
         if (!slab_group(m, static_cast<unsigned>(xcd_block(bx, nsbp)) * blockDim.x + threadIdx.x, x0, y, z, col, rowlen)) return;
-        e_group<T, W, true, true, SRC, FMA>(a, mt, x0, y, z);
+        e_group<T, W, true, true, SRC, FMA, NT>(a, mt, x0, y, z);
         return;
     }
     bx -= nsbp;
     int x0, y, z, col;
     if (!int_group<T, W>(b, xcd_block(bx, nib), x0, y, z, col)) return;
     const int lane = threadIdx.x & 63;
-    e_group<T, W, true, false, SRC, FMA>(a, mt, x0, y, z, lane > 0 && col > 0);
+    e_group<T, W, true, false, SRC, FMA, NT>(a, mt, x0, y, z, lane > 0 && col > 0);
 }
 
-template <typename T, int W, bool SRC, bool FMA>
+template <typename T, int W, bool SRC, bool FMA, bool NT>
 __global__ void __launch_bounds__(256) k_e3_all(StepArgs<T> a, Box3 b, SlabMap m, int nib, int nsbp, int nm0, int nm1, int nm2) {
     __shared__ MatLds<T> mt[3][CHIML_MAX_MAT];
     const int nm[3] = {nm0, nm1, nm2};
     load_mat(a, mt, nm);
-    e3_all_sweep<T, W, SRC, FMA>(a, mt, b, m, nib, nsbp, blockIdx.x);
+    e3_all_sweep<T, W, SRC, FMA, NT>(a, mt, b, m, nib, nsbp, blockIdx.x);
 }
 
 // ------------------------------------------------------- fused 3D step ----
@@ -3041,18 +3059,18 @@ __global__ void __launch_bounds__(256) k_be2v(const BatchSlot<T>* __restrict__ s
     e2v_sweep<T, W, true, false>(q.a, q.s, mt, bx, q.nblk[kPhE]);
 }
 
-template <typename T, int W>
+template <typename T, int W, bool NT>
 __global__ void __launch_bounds__(256) k_bh3_all(const BatchSlot<T>* __restrict__ sl, const int* __restrict__ begin, int n) {
     const int k = batch_slot(begin, n, blockIdx.x);
     const int bx = blockIdx.x - begin[k];
     const BatchSlot<T>& q = sl[k];
     if (bx >= q.nblk[kPhH]) return;
-    if (q.fma) h3_all_sweep<T, W, true, true>(q.a, q.b, q.m, q.nib, q.nsbp, q.ade_bpc, bx);
-    else h3_all_sweep<T, W, true, false>(q.a, q.b, q.m, q.nib, q.nsbp, q.ade_bpc, bx);
+    if (q.fma) h3_all_sweep<T, W, true, true, NT>(q.a, q.b, q.m, q.nib, q.nsbp, q.ade_bpc, bx);
+    else h3_all_sweep<T, W, true, false, NT>(q.a, q.b, q.m, q.nib, q.nsbp, q.ade_bpc, bx);
     advance_counter_at(q.a, bx);
 }
 
-template <typename T, int W>
+template <typename T, int W, bool NT>
 __global__ void __launch_bounds__(256) k_be3_all(const BatchSlot<T>* __restrict__ sl, const int* __restrict__ begin, int n) {
     __shared__ MatLds<T> mt[3][CHIML_MAX_MAT];
     const int k = batch_slot(begin, n, blockIdx.x);
@@ -3060,30 +3078,30 @@ __global__ void __launch_bounds__(256) k_be3_all(const BatchSlot<T>* __restrict_
     const BatchSlot<T>& q = sl[k];
     if (bx >= q.nblk[kPhE]) return;
     load_mat(q.a, mt, q.nm);
-    if (q.fma) e3_all_sweep<T, W, true, true>(q.a, mt, q.b, q.m, q.nib, q.nsbp, bx);
-    else e3_all_sweep<T, W, true, false>(q.a, mt, q.b, q.m, q.nib, q.nsbp, bx);
+    if (q.fma) e3_all_sweep<T, W, true, true, NT>(q.a, mt, q.b, q.m, q.nib, q.nsbp, bx);
+    else e3_all_sweep<T, W, true, false, NT>(q.a, mt, q.b, q.m, q.nib, q.nsbp, bx);
 }
 
-template <typename T, int W>
+template <typename T, int W, bool NT>
 __global__ void __launch_bounds__(256) k_bh3_int(const BatchSlot<T>* __restrict__ sl, const int* __restrict__ begin, int n) {
     const int k = batch_slot(begin, n, blockIdx.x);
     const int bx = blockIdx.x - begin[k];
     const BatchSlot<T>& q = sl[k];
     if (bx >= q.nblk[kPhH]) return;
-    h3_int_sweep<T, W, true>(q.a, q.b, q.nib, q.ade_bpc, bx);
+    h3_int_sweep<T, W, true, NT>(q.a, q.b, q.nib, q.ade_bpc, bx);
     advance_counter_at(q.a, bx);
 }
 
-template <typename T, int W>
+template <typename T, int W, bool NT>
 __global__ void __launch_bounds__(256) k_bh3_slab(const BatchSlot<T>* __restrict__ sl, const int* __restrict__ begin, int n) {
     const int k = batch_slot(begin, n, blockIdx.x);
     const int bx = blockIdx.x - begin[k];
     const BatchSlot<T>& q = sl[k];
     if (bx >= q.nblk[kPhHs]) return;
-    h3_slab_sweep<T, W, true>(q.a, q.m, bx, q.nblk[kPhHs]);
+    h3_slab_sweep<T, W, true, NT>(q.a, q.m, bx, q.nblk[kPhHs]);
 }
 
-template <typename T, int W>
+template <typename T, int W, bool NT>
 __global__ void __launch_bounds__(256) k_be3_int(const BatchSlot<T>* __restrict__ sl, const int* __restrict__ begin, int n) {
     __shared__ MatLds<T> mt[3][CHIML_MAX_MAT];
     const int k = batch_slot(begin, n, blockIdx.x);
@@ -3091,10 +3109,10 @@ __global__ void __launch_bounds__(256) k_be3_int(const BatchSlot<T>* __restrict_
     const BatchSlot<T>& q = sl[k];
     if (bx >= q.nblk[kPhE]) return;
     load_mat(q.a, mt, q.nm);
-    e3_int_sweep<T, W, true>(q.a, mt, q.b, bx, q.nblk[kPhE]);
+    e3_int_sweep<T, W, true, NT>(q.a, mt, q.b, bx, q.nblk[kPhE]);
 }
 
-template <typename T, int W>
+template <typename T, int W, bool NT>
 __global__ void __launch_bounds__(256) k_be3_slab(const BatchSlot<T>* __restrict__ sl, const int* __restrict__ begin, int n) {
     __shared__ MatLds<T> mt[3][CHIML_MAX_MAT];
     const int k = batch_slot(begin, n, blockIdx.x);
@@ -3102,7 +3120,7 @@ __global__ void __launch_bounds__(256) k_be3_slab(const BatchSlot<T>* __restrict
     const BatchSlot<T>& q = sl[k];
     if (bx >= q.nblk[kPhEs]) return;
     load_mat(q.a, mt, q.nm);
-    e3_slab_sweep<T, W, true>(q.a, mt, q.m, bx, q.nblk[kPhEs]);
+    e3_slab_sweep<T, W, true, NT>(q.a, mt, q.m, bx, q.nblk[kPhEs]);
 }
 
 template <typename T>
@@ -3160,6 +3178,8 @@ struct chiml_dev {
     hipGraphExec_t gexec = nullptr;
     bool split = false;  // 3D interior + CPML-slab kernels
     bool rows = false;   // split: whole-row interior, one launch per field
+    double step_bytes = 0;     // fields and emitter state
+    bool stream_hint = false;  // split: once-touched words go past the caches (streams_past_caches)
     bool cellwise = false;  // split, but stepped alone with one thread per cell (GridLayout::cellwise)
     bool fma_curl = false;  // rows or x CPML no whole groups: curls as the per-cell kernels round them (curl_of)
     bool fused = false;  // 3D: one fused H + E launch per step on ping-pong buffers
@@ -3781,6 +3801,10 @@ void build(chiml_dev* c, const chiml_problem_t* p, StepArgs<T>& a, SampleArgs<T>
     }
     build_tfsf(c, p, a);
     build_cells<T>(c, p);
+    c->step_bytes = 6.0 * N * sizeof(T);
+    for (const QeHost& qh : c->qes)
+        c->step_bytes += 5.0 * 16 * ml_store_words(qh.N, qh.dev.packed != 0) * static_cast<double>(qh.dev.nmem) * qh.dev.nemit;
+    c->stream_hint = streams_past_caches(c->step_bytes);
 }
 
 template <typename T>
@@ -3948,8 +3972,12 @@ void launch_fields(chiml_dev* c, StepArgs<T>& a) {
                 Timed t(c, "update_h");
                 pick2(c->has_src, adv, [&](auto S, auto A) {
                     auto go = [&](auto M) {
-                        hipLaunchKernelGGL((k_h3_all<T, W, decltype(S)::value, decltype(A)::value, decltype(M)::value>), gh, blk, 0, c->stream, a,
-                                           b, c->slab, nib, nsbp, ade_bpc);
+                        if (c->stream_hint)
+                            hipLaunchKernelGGL((k_h3_all<T, W, decltype(S)::value, decltype(A)::value, decltype(M)::value, true>), gh, blk, 0, c->stream,
+                                               a, b, c->slab, nib, nsbp, ade_bpc);
+                        else
+                            hipLaunchKernelGGL((k_h3_all<T, W, decltype(S)::value, decltype(A)::value, decltype(M)::value, false>), gh, blk, 0, c->stream,
+                                               a, b, c->slab, nib, nsbp, ade_bpc);
                     };
                     if (c->fma_curl) go(std::true_type{});
                     else go(std::false_type{});
@@ -3960,8 +3988,12 @@ void launch_fields(chiml_dev* c, StepArgs<T>& a) {
             if (ge.x > 0) {
                 Timed t(c, "update_e");
                 pick2(c->has_src, c->fma_curl, [&](auto S, auto M) {
-                    hipLaunchKernelGGL((k_e3_all<T, W, decltype(S)::value, decltype(M)::value>), ge, blk, 0, c->stream, a, b, c->slab, nib, nsbp,
-                                       c->nmat[0], c->nmat[1], c->nmat[2]);
+                    if (c->stream_hint)
+                        hipLaunchKernelGGL((k_e3_all<T, W, decltype(S)::value, decltype(M)::value, true>), ge, blk, 0, c->stream, a, b, c->slab, nib,
+                                           nsbp, c->nmat[0], c->nmat[1], c->nmat[2]);
+                    else
+                        hipLaunchKernelGGL((k_e3_all<T, W, decltype(S)::value, decltype(M)::value, false>), ge, blk, 0, c->stream, a, b, c->slab, nib,
+                                           nsbp, c->nmat[0], c->nmat[1], c->nmat[2]);
                 });
             }
         } else if constexpr (W == 2) {  // FP64: the pole update rides on the H interior launch as its first blocks
@@ -3969,26 +4001,33 @@ void launch_fields(chiml_dev* c, StepArgs<T>& a) {
             if (gh.x > 0) {
                 Timed t(c, "update_h");
                 pick2(c->has_src, adv, [&](auto S, auto A) {
-                    hipLaunchKernelGGL((k_h3_int<T, W, decltype(S)::value, decltype(A)::value>), gh, blk, 0, c->stream, a, b, nib,
-                                       ade_bpc);
+                    if (c->stream_hint)
+                        hipLaunchKernelGGL((k_h3_int<T, W, decltype(S)::value, decltype(A)::value, true>), gh, blk, 0, c->stream, a, b, nib, ade_bpc);
+                    else
+                        hipLaunchKernelGGL((k_h3_int<T, W, decltype(S)::value, decltype(A)::value, false>), gh, blk, 0, c->stream, a, b, nib, ade_bpc);
                 });
             }
             if (ns > 0) {
                 Timed t(c, "update_h_pml");
-                if (c->has_src) hipLaunchKernelGGL((k_h3_slab<T, W, true>), gs, blk, 0, c->stream, a, c->slab);
-                else hipLaunchKernelGGL((k_h3_slab<T, W, false>), gs, blk, 0, c->stream, a, c->slab);
+                pick2(c->has_src, c->stream_hint, [&](auto S, auto H) {
+                    hipLaunchKernelGGL((k_h3_slab<T, W, decltype(S)::value, decltype(H)::value>), gs, blk, 0, c->stream, a, c->slab);
+                });
             }
             launch_tfsf<T>(c, a);
             launch_cells<T>(c, a);
             {
                 Timed t(c, "update_e");
-                if (c->has_src) hipLaunchKernelGGL((k_e3_int<T, W, true>), gi, blk, 0, c->stream, a, b, c->nmat[0], c->nmat[1], c->nmat[2]);
-                else hipLaunchKernelGGL((k_e3_int<T, W, false>), gi, blk, 0, c->stream, a, b, c->nmat[0], c->nmat[1], c->nmat[2]);
+                pick2(c->has_src, c->stream_hint, [&](auto S, auto H) {
+                    hipLaunchKernelGGL((k_e3_int<T, W, decltype(S)::value, decltype(H)::value>), gi, blk, 0, c->stream, a, b, c->nmat[0], c->nmat[1],
+                                       c->nmat[2]);
+                });
             }
             if (ns > 0) {
                 Timed t(c, "update_e_pml");
-                if (c->has_src) hipLaunchKernelGGL((k_e3_slab<T, W, true>), gs, blk, 0, c->stream, a, c->slab, c->nmat[0], c->nmat[1], c->nmat[2]);
-                else hipLaunchKernelGGL((k_e3_slab<T, W, false>), gs, blk, 0, c->stream, a, c->slab, c->nmat[0], c->nmat[1], c->nmat[2]);
+                pick2(c->has_src, c->stream_hint, [&](auto S, auto H) {
+                    hipLaunchKernelGGL((k_e3_slab<T, W, decltype(S)::value, decltype(H)::value>), gs, blk, 0, c->stream, a, c->slab, c->nmat[0],
+                                       c->nmat[1], c->nmat[2]);
+                });
             }
         }
         return;
@@ -4504,6 +4543,9 @@ void batch_group(chiml_dev** g, int n, int nsteps, hipStream_t bs, unsigned char
     const BatchSlot<T>* ds = reinterpret_cast<const BatchSlot<T>*>(dev);
     const int* db = reinterpret_cast<const int*>(dev + 2 * n * sizeof(BatchSlot<T>));
     const dim3 blk(256);
+    double state = 0;  // the batch's simulations share the caches
+    for (int i = 0; i < n; ++i) state += g[i]->step_bytes;
+    const bool stream_hint = streams_past_caches(state);
     for (int j = 0; j < nsteps; ++j) {
         const BatchSlot<T>* t = ds + (j & 1) * n;  // every slot's counter parity flips each step
         const int* bH = db + kPhH * (n + 1);
@@ -4514,14 +4556,21 @@ void batch_group(chiml_dev** g, int n, int nsteps, hipStream_t bs, unsigned char
         if (g[0]->dim == 2) {
             if (total[kPhH]) hipLaunchKernelGGL((k_bh2v<T, W>), dim3(total[kPhH]), blk, 0, bs, t, bH, n);
             if (total[kPhE]) hipLaunchKernelGGL((k_be2v<T, W>), dim3(total[kPhE]), blk, 0, bs, t, bE, n);
-        } else if (W == 4) {
-            if (total[kPhH]) hipLaunchKernelGGL((k_bh3_all<T, W>), dim3(total[kPhH]), blk, 0, bs, t, bH, n);
-            if (total[kPhE]) hipLaunchKernelGGL((k_be3_all<T, W>), dim3(total[kPhE]), blk, 0, bs, t, bE, n);
         } else {
-            if (total[kPhH]) hipLaunchKernelGGL((k_bh3_int<T, W>), dim3(total[kPhH]), blk, 0, bs, t, bH, n);
-            if (total[kPhHs]) hipLaunchKernelGGL((k_bh3_slab<T, W>), dim3(total[kPhHs]), blk, 0, bs, t, bHs, n);
-            if (total[kPhE]) hipLaunchKernelGGL((k_be3_int<T, W>), dim3(total[kPhE]), blk, 0, bs, t, bE, n);
-            if (total[kPhEs]) hipLaunchKernelGGL((k_be3_slab<T, W>), dim3(total[kPhEs]), blk, 0, bs, t, bEs, n);
+            auto go = [&](auto H) {
+                constexpr bool NT = decltype(H)::value;
+                if constexpr (W == 4) {
+                    if (total[kPhH]) hipLaunchKernelGGL((k_bh3_all<T, W, NT>), dim3(total[kPhH]), blk, 0, bs, t, bH, n);
+                    if (total[kPhE]) hipLaunchKernelGGL((k_be3_all<T, W, NT>), dim3(total[kPhE]), blk, 0, bs, t, bE, n);
+                } else {
+                    if (total[kPhH]) hipLaunchKernelGGL((k_bh3_int<T, W, NT>), dim3(total[kPhH]), blk, 0, bs, t, bH, n);
+                    if (total[kPhHs]) hipLaunchKernelGGL((k_bh3_slab<T, W, NT>), dim3(total[kPhHs]), blk, 0, bs, t, bHs, n);
+                    if (total[kPhE]) hipLaunchKernelGGL((k_be3_int<T, W, NT>), dim3(total[kPhE]), blk, 0, bs, t, bE, n);
+                    if (total[kPhEs]) hipLaunchKernelGGL((k_be3_slab<T, W, NT>), dim3(total[kPhEs]), blk, 0, bs, t, bEs, n);
+                }
+            };
+            if (stream_hint) go(std::true_type{});
+            else go(std::false_type{});
         }
         // emitters per simulation, on the batch stream, between the E update and the sampling
         for (int i = 0; i < n; ++i) {
