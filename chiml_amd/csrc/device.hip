@@ -2803,8 +2803,13 @@ __global__ void __launch_bounds__(256) k_ml_pop_gather(QeDev q, int j0, double2*
 // FP64 incident lines (six components, set 0 read by the surface adds, set 1
 // the shorter pulse line whose values are recorded for the flux
 // normalisation).  They are a few hundred to a few thousand points long, so
-// one block steps all of them (k_tfsf_line) between the H and E updates of
-// the main grid; k_tfsf_add then adds pf * Re(line) to the surface cells.
+// one block steps all of them, between the H and E updates of the main grid,
+// beside the blocks that add pf * Re(line) to the surface cells of H
+// (k_tfsf_step); k_tfsf_add then adds to the cells of E.  256^3 FP32 with a
+// 201^3 box: H adds 11.4 us and lines 16.2 us one after the other, 21.2 us
+// together.  The adds are bound by the faces of constant x, where each point
+// moves a cache line of its own; the sweeps, which hold those cells anyway,
+// lost more to the search for them (k_h3_all 107 -> 167 us).
 struct TfsfLineArgs {
     int len[2], present[6], margin, pulse_at, pulse_n, psi_n, rec_idx, rec_off[6];
     int nterm[6], tsrc[6][2], tpos[6][2], tneg[6][2];
@@ -2817,6 +2822,7 @@ struct TfsfLineArgs {
     const double2* amp;   // [nsteps][6][pulse_n]
     double2* rec;         // [6][nrec]
     long long nrec;
+    double2* snap[2];     // [6][len[0]] by step parity: the lines line[0] after the step, for the H adds of the next
 };
 
 // One line point: pulse, the derivative terms in the reference's order, then
@@ -2852,7 +2858,7 @@ __device__ void tfsf_point(const TfsfLineArgs& t, double2* L, double2* psi, cons
     L[c * len + n] = v;
 }
 
-// LDS bytes of the staged form of k_tfsf_line: both sets of lines, their
+// LDS bytes of the staged form of k_tfsf_step: both sets of lines, their
 // CPML fields, the coefficients and one step of pulse values.
 __host__ __device__ inline size_t tfsf_lds_bytes(const TfsfLineArgs& t) {
     return 16 * (6 * static_cast<size_t>(t.len[0] + t.len[1]) + 2 * 6 * 4 * static_cast<size_t>(t.psi_n) + 6 * static_cast<size_t>(t.pulse_n)) +
@@ -2867,8 +2873,7 @@ __host__ __device__ inline size_t tfsf_lds_bytes(const TfsfLineArgs& t) {
 // staged in shared memory first (one batch of loads) and written back after;
 // lines too long for it are stepped in global memory.
 template <bool LDS>
-__global__ void __launch_bounds__(1024) k_tfsf_line(TfsfLineArgs ta, const int* stepp, int stepv) {
-    extern __shared__ __align__(16) unsigned char tfsf_lds[];
+__device__ __forceinline__ void tfsf_lines(const TfsfLineArgs& ta, unsigned char* tfsf_lds, int step) {
     // the parameter block is read by every pass: one copy into LDS, read in
     // parallel, instead of a chain of dependent argument loads per pass
     __shared__ TfsfLineArgs t;
@@ -2876,7 +2881,6 @@ __global__ void __launch_bounds__(1024) k_tfsf_line(TfsfLineArgs ta, const int* 
     for (unsigned w = threadIdx.x; w < sizeof(TfsfLineArgs) / 4; w += blockDim.x)
         reinterpret_cast<int*>(&t)[w] = reinterpret_cast<const int*>(&ta)[w];
     __syncthreads();
-    const int step = step_now(stepp, stepv);
     double2* L[2] = {t.line[0], t.line[1]};
     const int np = 6 * 4 * t.psi_n;
     double2* psi = t.psi;
@@ -2909,6 +2913,7 @@ __global__ void __launch_bounds__(1024) k_tfsf_line(TfsfLineArgs ta, const int* 
         }
     };
     record(3);
+    __syncthreads();
     for (int ph = 0; ph < 2; ++ph) {  // H lines (3..5), then E lines (0..2)
         // the line is uniform across the block, so its parameters are scalar
         // loads; the lines of one phase are independent of each other
@@ -2920,6 +2925,8 @@ __global__ void __launch_bounds__(1024) k_tfsf_line(TfsfLineArgs ta, const int* 
         __syncthreads();
     }
     record(0);
+    double2* const snap = t.snap[step & 1];
+    for (int q = threadIdx.x; q < 6 * t.len[0]; q += blockDim.x) snap[q] = L[0][q];
     if (LDS) {
         for (int s = 0; s < 2; ++s)
             for (int q = threadIdx.x; q < 6 * t.len[s]; q += blockDim.x) t.line[s][q] = L[s][q];
@@ -2942,36 +2949,36 @@ __device__ __forceinline__ bool tfsf_in(const TfsfSurfD& q, const int* x, int& i
 }
 
 // U += pf * Re(line[src][incd0 + i1 s1 + i2 s2]) over the surfaces of one
-// family (addIncdFields, parallelTFSF.cpp:78-84).  Each surface starts on a
-// block boundary, so a block's surface and the table reads are uniform; the
-// threads of a block run along x where the surface contains x (coalesced).
+// family (addIncdFields, parallelTFSF.cpp:78-84), for the 256 points from b0
+// on (t: which of them).  Each surface starts on a multiple of 256, so the
+// surface and the table reads are uniform; the points run along x where the
+// surface contains x (coalesced).
 // A cell on several surfaces of its component (an edge of the box) takes all
 // their adds in order from the thread of its first surface, so the sums keep
 // the reference's order.
 template <typename T>
-__global__ void __launch_bounds__(256) k_tfsf_add(const TfsfSurfD* __restrict__ sf, int ns, long long total, T* F0, T* F1, T* F2,
-                                                  T* F3, T* F4, T* F5, const double2* __restrict__ line, int len, int nx, int ny) {
-    const long long b0 = blockIdx.x * 256LL;
-    if (b0 >= total) return;
+struct TfsfFields {
+    T* F[6];
+};
+template <typename T>
+__device__ __forceinline__ void tfsf_add(const TfsfSurfD* __restrict__ sf, int ns, long long b0, int t, const TfsfFields<T>& f,
+                                         const double2* __restrict__ line, int len, int nx, int ny) {
     int s = 0;
     while (s + 1 < ns && sf[s + 1].start <= b0) ++s;
     const TfsfSurfD& q = sf[s];
-    const long long pnt = b0 + threadIdx.x - q.start;
+    const long long pnt = b0 + t - q.start;
     const long long np = static_cast<long long>(q.n1) * q.n2;
     if (pnt >= np) return;
     int x[3] = {q.o[0], q.o[1], q.o[2]};
-    if (q.a2 == 0) {  // rows along x: x fastest
-        x[q.a2] += static_cast<int>(pnt % q.n2);
-        x[q.a1] += static_cast<int>(pnt / q.n2);
-    } else {
-        x[q.a1] += static_cast<int>(pnt % q.n1);
-        x[q.a2] += static_cast<int>(pnt / q.n1);
-    }
+    // x fastest where the surface has rows along x
+    const int fast = q.a2 == 0 ? q.a2 : q.a1, slow = q.a2 == 0 ? q.a1 : q.a2;
+    const unsigned n = static_cast<unsigned>(q.a2 == 0 ? q.n2 : q.n1), up = static_cast<unsigned>(pnt), row = up / n;
+    x[fast] += static_cast<int>(up - row * n);
+    x[slow] += static_cast<int>(row);
     int i1, i2;
     for (int k = 0; k < s; ++k)
         if (sf[k].comp == q.comp && tfsf_in(sf[k], x, i1, i2)) return;
-    T* const Fs[6] = {F0, F1, F2, F3, F4, F5};
-    T* F = Fs[q.comp];
+    T* F = f.F[q.comp];
     const long long idx = x[0] + static_cast<long long>(nx) * (x[1] + static_cast<long long>(ny) * x[2]);
     T v = F[idx];
     for (int k = s; k < ns; ++k) {
@@ -2980,6 +2987,28 @@ __global__ void __launch_bounds__(256) k_tfsf_add(const TfsfSurfD* __restrict__ 
         v += static_cast<T>(r.pf * line[r.src * len + r.incd0 + i1 * r.s1 + i2 * r.s2].x);
     }
     F[idx] = v;
+}
+
+template <typename T>
+__global__ void __launch_bounds__(256) k_tfsf_add(const TfsfSurfD* __restrict__ sf, int ns, long long total, TfsfFields<T> f,
+                                                  const double2* __restrict__ line, int len, int nx, int ny) {
+    const long long b0 = blockIdx.x * 256LL;
+    if (b0 < total) tfsf_add<T>(sf, ns, b0, threadIdx.x, f, line, len, nx, ny);
+}
+
+// Block 0: the lines; the others: the H adds, which read the lines as the step
+// before left them, 1024 points a block.
+template <typename T, bool LDS>
+__global__ void __launch_bounds__(1024) k_tfsf_step(TfsfLineArgs ta, const TfsfSurfD* __restrict__ sf, int ns, long long total,
+                                                    TfsfFields<T> f, int nx, int ny, const int* stepp, int stepv) {
+    extern __shared__ __align__(16) unsigned char tfsf_lds[];
+    const int step = step_now(stepp, stepv);
+    if (blockIdx.x == 0) {
+        tfsf_lines<LDS>(ta, tfsf_lds, step);
+        return;
+    }
+    const long long b0 = ((blockIdx.x - 1) * 4LL + (threadIdx.x >> 8)) * 256;
+    if (b0 < total) tfsf_add<T>(sf, ns, b0, threadIdx.x & 255, f, ta.snap[(step + 1) & 1], ta.len[0], nx, ny);
 }
 
 // Per-cell soft-source adds (oblique sources, parallelSourceOblique.cpp:17-23),
@@ -3301,7 +3330,7 @@ T* upload_cast(chiml_dev* c, const double* src, size_t n) {
     return c->upload<T>(tmp.data(), n);
 }
 
-constexpr size_t kTfsfMaxLds = 160 * 1024 - 1024;  // dynamic LDS of k_tfsf_line: a gfx950 workgroup's 160 KB less its static parameter copy
+constexpr size_t kTfsfMaxLds = 160 * 1024 - 1024;  // dynamic LDS of k_tfsf_step: a gfx950 workgroup's 160 KB less its static parameter copy
 
 // Per-cell source table: components, points and columns checked on the host.
 template <typename T>
@@ -3344,7 +3373,7 @@ void build_tfsf(chiml_dev* c, const chiml_problem_t* p, const StepArgs<T>& a) {
     if (p->ntfsf == 0) return;
     c->nrec = 2LL * (p->nsteps + 1) + 2;
     c->incd_rec = reinterpret_cast<double2*>(c->zeros<double>(2 * 6 * static_cast<size_t>(c->nrec)));
-    HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(k_tfsf_line<true>), hipFuncAttributeMaxDynamicSharedMemorySize,
+    HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(k_tfsf_step<T, true>), hipFuncAttributeMaxDynamicSharedMemorySize,
                                 static_cast<int>(kTfsfMaxLds)));
     auto need = [](bool ok, const char* what) {
         if (!ok) throw std::runtime_error(std::string("TFSF table: ") + what);
@@ -3409,6 +3438,7 @@ void build_tfsf(chiml_dev* c, const chiml_problem_t* p, const StepArgs<T>& a) {
         t.psi = reinterpret_cast<double2*>(c->zeros<double>(2 * 2 * 6 * 4 * static_cast<size_t>(std::max(tf.psi_n, 1))));
         t.scoef = c->upload<double>(tf.seg_coef, 6 * 4 * static_cast<size_t>(tf.psi_n) * 3);
         t.amp = reinterpret_cast<const double2*>(c->upload<double>(tf.amp, 2 * static_cast<size_t>(p->nsteps) * 6 * tf.pulse_n));
+        for (double2*& q : t.snap) q = reinterpret_cast<double2*>(c->zeros<double>(2 * 6 * static_cast<size_t>(tf.len0)));
         t.rec = c->incd_rec;
         t.nrec = c->nrec;
         // surfaces: H adds first, then E adds, each with flat point offsets
@@ -3899,24 +3929,23 @@ void pick2(bool s, bool adv, F&& f) {
     }
 }
 
-// adv: the H launch advances the two-slot step counter (steps being captured)
 // The TFSF part of a step, between the H and E updates of the main grid:
 // H surface adds, the incident lines, E surface adds (parallelFDTDField.hpp:1236-1256).
 template <typename T>
 void launch_tfsf(chiml_dev* c, StepArgs<T>& a) {
+    TfsfFields<T> f;
+    for (int k = 0; k < 6; ++k) f.F[k] = a.F[k];
     for (const auto& h : c->tfsf) {
         const TfsfLineArgs& t = h.line;
-        if (h.toth > 0)
-            hipLaunchKernelGGL(k_tfsf_add<T>, dim3(static_cast<unsigned>((h.toth + 255) / 256)), dim3(256), 0, c->stream, h.surf, h.nsh,
-                               h.toth, a.F[0], a.F[1], a.F[2], a.F[3], a.F[4], a.F[5], t.line[0], t.len[0], c->px, c->ny);
+        const dim3 g(static_cast<unsigned>(1 + (h.toth + 1023) / 1024));
         const size_t lds = tfsf_lds_bytes(t);
         if (lds <= kTfsfMaxLds)
-            hipLaunchKernelGGL(k_tfsf_line<true>, dim3(1), dim3(1024), lds, c->stream, t, a.step, a.stepv);
+            hipLaunchKernelGGL((k_tfsf_step<T, true>), g, dim3(1024), lds, c->stream, t, h.surf, h.nsh, h.toth, f, c->px, c->ny, a.step, a.stepv);
         else
-            hipLaunchKernelGGL(k_tfsf_line<false>, dim3(1), dim3(1024), 0, c->stream, t, a.step, a.stepv);
+            hipLaunchKernelGGL((k_tfsf_step<T, false>), g, dim3(1024), 0, c->stream, t, h.surf, h.nsh, h.toth, f, c->px, c->ny, a.step, a.stepv);
         if (h.tote > 0)
             hipLaunchKernelGGL(k_tfsf_add<T>, dim3(static_cast<unsigned>((h.tote + 255) / 256)), dim3(256), 0, c->stream, h.surf + h.nsh,
-                               h.nse, h.tote, a.F[0], a.F[1], a.F[2], a.F[3], a.F[4], a.F[5], t.line[0], t.len[0], c->px, c->ny);
+                               h.nse, h.tote, f, t.line[0], t.len[0], c->px, c->ny);
     }
 }
 
