@@ -168,18 +168,48 @@ __device__ __forceinline__ long long lidx(int x, int y, int z, int nx, int ny) {
 // psi' = b psi + (c/d) dV (psi-carrying positions), term = dV/(kappa d) + psi'.
 // Elsewhere in the PML region the term is dV/d (kappa = 1, no psi).
 template <typename T>
+struct PmlCell {
+    T b, cd, kinv, psi;
+    T* at = nullptr;  // null: no psi here
+    __device__ __forceinline__ void load(const PmlDev<T>& p, int a, int pos, int x, int y, int z, int nx, int ny) {
+        int s;
+        if (pos < p.lo[a]) s = pos;
+        else if (pos >= p.hi0[a] && pos < p.hi1[a]) s = p.lo[a] + pos - p.hi0[a];
+        else return;
+        long long pi;
+        if (a == 0) pi = s + static_cast<long long>(p.S[0]) * (y + static_cast<long long>(ny) * z);
+        else if (a == 1) pi = x + static_cast<long long>(nx) * (s + static_cast<long long>(p.S[1]) * z);
+        else pi = x + static_cast<long long>(nx) * (y + static_cast<long long>(ny) * s);
+        at = p.psi[a] + pi;
+        psi = *at;
+        b = p.b[a][pos];
+        cd = p.cd[a][pos];
+        kinv = p.kinv[a][pos];
+    }
+    __device__ __forceinline__ T term(T dV, T dVd) {
+        if (!at) return dVd;
+        psi = fma(b, psi, cd * dV);
+        *at = psi;
+        return fma(kinv, dVd, psi);
+    }
+};
+template <typename T>
 __device__ __forceinline__ T pml_term(const PmlDev<T>& p, int a, int pos, int x, int y, int z, int nx, int ny, T dV, T dVd) {
-    int s;
-    if (pos < p.lo[a]) s = pos;
-    else if (pos >= p.hi0[a] && pos < p.hi1[a]) s = p.lo[a] + pos - p.hi0[a];
-    else return dVd;
-    long long pi;
-    if (a == 0) pi = s + static_cast<long long>(p.S[0]) * (y + static_cast<long long>(ny) * z);
-    else if (a == 1) pi = x + static_cast<long long>(nx) * (s + static_cast<long long>(p.S[1]) * z);
-    else pi = x + static_cast<long long>(nx) * (y + static_cast<long long>(ny) * s);
-    T psi = p.b[a][pos] * p.psi[a][pi] + p.cd[a][pos] * dV;
-    p.psi[a][pi] = psi;
-    return p.kinv[a][pos] * dVd + psi;
+    PmlCell<T> q;
+    q.load(p, a, pos, x, y, z, nx, ny);
+    return q.term(dV, dVd);
+}
+// d1/dA - d2/dB of a cell with its CPML terms: one rounding less outside the
+// CPML, as the compiler contracts the difference of two products
+template <typename T>
+__device__ __forceinline__ T curl_cell(PmlCell<T>& q1, PmlCell<T>& q2, bool inpml, T d1, T i1, T d2, T i2) {
+    const T p1 = d1 * i1;
+    if (!inpml) return fma(-i2, d2, p1);
+    const T t1 = q1.term(d1, p1), t2 = q2.term(d2, d2 * i2);
+    {
+#pragma clang fp contract(off)
+        return t1 - t2;
+    }
 }
 
 template <typename T>
@@ -193,10 +223,31 @@ __device__ __forceinline__ T src_value(const StepArgs<T>& a, int comp, int x, in
     return v;
 }
 
+// src_value of the components c0 .. c0 + 2 of a cell
+template <typename T>
+__device__ __forceinline__ void src_values(const StepArgs<T>& a, int c0, int x, int y, int z, int step, T (&v)[3]) {
+    for (int s = 0; s < a.nsrc; ++s) {
+        const int c = a.src_comp[s] - c0;
+        const int* b = a.src_box + 6 * s;
+        if (!(x >= b[0] && x < b[1] && y >= b[2] && y < b[3] && z >= b[4] && z < b[5])) continue;
+        const T amp = a.src_amp[static_cast<long long>(step) * a.nsrc + s];
+#pragma unroll
+        for (int k = 0; k < 3; ++k)
+            if (c == k) v[k] += amp;
+    }
+}
+
 // ----------------------------------------------------------- H update -------
 // 3D: Hx += ch[(Ey(z+1)-Ey)/dz - (Ez(y+1)-Ez)/dy], Hy += ch[(Ez(x+1)-Ez)/dx -
 // (Ex(z+1)-Ex)/dz], Hz += ch[(Ex(y+1)-Ex)/dy - (Ey(x+1)-Ey)/dx]; 2D TMz keeps
 // the Ez terms of Hx and Hy (OneCompCurlK/J, src/UTIL/FDTD_up_eq.cpp:10-35).
+//
+// One thread per cell: small unaligned 3D grids, H maps and grids that no
+// other kernel takes.  Few waves are in flight on a small grid, so the time is
+// that of the longest chain of dependent accesses: every load of a cell is
+// issued before its first store, which the next component's loads could not
+// pass.  64^3 FP32 with a metal block and soft sources: H 6.8 -> 6.1 us, E
+// 10.3 -> 9.2 us.
 template <typename T, int DIM, bool HMAP, bool SRC>
 __device__ __forceinline__ void update_h_cells(const StepArgs<T>& a) {
     const int x = blockIdx.x * blockDim.x + threadIdx.x;
@@ -210,55 +261,71 @@ __device__ __forceinline__ void update_h_cells(const StepArgs<T>& a) {
                        (DIM == 3 && ((z < a.Tp[2]) || (z >= nz - a.Tp[2])));
     int step = 0;
     if (SRC) step = step_now(a.step, a.stepv);
-    T* Ex = a.F[0];
-    T* Ey = a.F[1];
-    T* Ez = a.F[2];
-    // Hx: valid y < ny-1 (and z < nz-1 in 3D)
-    if (y < ny - 1 && (DIM == 2 || z < nz - 1)) {
-        T ez = Ez[i];
-        T dEz = Ez[i + sy] - ez;
-        T acc;
-        if (DIM == 3) {
-            T dEy = Ey[i + sz] - Ey[i];
-            if (!inpml) acc = dEy * a.inv_d[2] - dEz * a.inv_d[1];
-            else acc = pml_term(a.pml[3], 2, z, x, y, z, px, ny, dEy, dEy * a.inv_d[2]) - pml_term(a.pml[3], 1, y, x, y, z, px, ny, dEz, dEz * a.inv_d[1]);
-        } else {
+    const bool xin = x < nx - 1, yin = y < ny - 1;
+    const T *Ex = a.F[0], *Ey = a.F[1], *Ez = a.F[2];
+    T ch[3] = {};
+    PmlCell<T> q[6];
+    T sv[3] = {};
+    if constexpr (DIM == 3) {
+        const bool zin = z < nz - 1;
+        const T ex = Ex[i], ey = Ey[i], ez = Ez[i];
+        const T ezx = xin ? Ez[i + 1] : T(0), eyx = xin ? Ey[i + 1] : T(0);
+        const T exy = yin ? Ex[i + sy] : T(0), ezy = yin ? Ez[i + sy] : T(0);
+        const T exz = zin ? Ex[i + sz] : T(0), eyz = zin ? Ey[i + sz] : T(0);
+        const T h0 = a.F[3][i], h1 = a.F[4][i], h2 = a.F[5][i];
+#pragma unroll
+        for (int c = 0; c < 3; ++c) ch[c] = HMAP ? a.ch[c][a.mat_h[c][i]] : a.ch[c][0];
+        if (inpml) {
+            if (yin && zin) {
+                q[0].load(a.pml[3], 2, z, x, y, z, px, ny);
+                q[1].load(a.pml[3], 1, y, x, y, z, px, ny);
+            }
+            if (xin && zin) {
+                q[2].load(a.pml[4], 0, x, x, y, z, px, ny);
+                q[3].load(a.pml[4], 2, z, x, y, z, px, ny);
+            }
+            if (xin && yin) {
+                q[4].load(a.pml[5], 1, y, x, y, z, px, ny);
+                q[5].load(a.pml[5], 0, x, x, y, z, px, ny);
+            }
+        }
+        if (SRC) src_values(a, 3, x, y, z, step, sv);
+        if (yin && zin) {
+            T h = fma(ch[0], curl_cell(q[0], q[1], inpml, eyz - ey, a.inv_d[2], ezy - ez, a.inv_d[1]), h0);
+            if (SRC) h += sv[0];
+            a.F[3][i] = h;
+        }
+        if (xin && zin) {
+            T h = fma(ch[1], curl_cell(q[2], q[3], inpml, ezx - ez, a.inv_d[0], exz - ex, a.inv_d[2]), h1);
+            if (SRC) h += sv[1];
+            a.F[4][i] = h;
+        }
+        if (xin && yin) {
+            T h = fma(ch[2], curl_cell(q[4], q[5], inpml, exy - ex, a.inv_d[1], eyx - ey, a.inv_d[0]), h2);
+            if (SRC) h += sv[2];
+            a.F[5][i] = h;
+        }
+    } else {
+        if (yin) {  // Hx
+            const T dEz = Ez[i + sy] - Ez[i];
+            T acc;
             if (!inpml) acc = -(dEz * a.inv_d[1]);
             else acc = -pml_term(a.pml[3], 1, y, x, y, z, px, ny, dEz, dEz * a.inv_d[1]);
+            const T ch0 = HMAP ? a.ch[0][a.mat_h[0][i]] : a.ch[0][0];
+            T h = a.F[3][i] + ch0 * acc;
+            if (SRC) h += src_value(a, 3, x, y, z, step);
+            a.F[3][i] = h;
         }
-        T ch = HMAP ? a.ch[0][a.mat_h[0][i]] : a.ch[0][0];
-        T h = a.F[3][i] + ch * acc;
-        if (SRC) h += src_value(a, 3, x, y, z, step);
-        a.F[3][i] = h;
-    }
-    // Hy: valid x < nx-1 (and z < nz-1 in 3D)
-    if (x < nx - 1 && (DIM == 2 || z < nz - 1)) {
-        T dEz = Ez[i + 1] - Ez[i];
-        T acc;
-        if (DIM == 3) {
-            T dEx = Ex[i + sz] - Ex[i];
-            if (!inpml) acc = dEz * a.inv_d[0] - dEx * a.inv_d[2];
-            else acc = pml_term(a.pml[4], 0, x, x, y, z, px, ny, dEz, dEz * a.inv_d[0]) - pml_term(a.pml[4], 2, z, x, y, z, px, ny, dEx, dEx * a.inv_d[2]);
-        } else {
+        if (xin) {  // Hy
+            const T dEz = Ez[i + 1] - Ez[i];
+            T acc;
             if (!inpml) acc = dEz * a.inv_d[0];
             else acc = pml_term(a.pml[4], 0, x, x, y, z, px, ny, dEz, dEz * a.inv_d[0]);
+            const T ch1 = HMAP ? a.ch[1][a.mat_h[1][i]] : a.ch[1][0];
+            T h = a.F[4][i] + ch1 * acc;
+            if (SRC) h += src_value(a, 4, x, y, z, step);
+            a.F[4][i] = h;
         }
-        T ch = HMAP ? a.ch[1][a.mat_h[1][i]] : a.ch[1][0];
-        T h = a.F[4][i] + ch * acc;
-        if (SRC) h += src_value(a, 4, x, y, z, step);
-        a.F[4][i] = h;
-    }
-    // Hz (3D only): valid x < nx-1, y < ny-1
-    if (DIM == 3 && x < nx - 1 && y < ny - 1) {
-        T dEx = Ex[i + sy] - Ex[i];
-        T dEy = Ey[i + 1] - Ey[i];
-        T acc;
-        if (!inpml) acc = dEx * a.inv_d[1] - dEy * a.inv_d[0];
-        else acc = pml_term(a.pml[5], 1, y, x, y, z, px, ny, dEx, dEx * a.inv_d[1]) - pml_term(a.pml[5], 0, x, x, y, z, px, ny, dEy, dEy * a.inv_d[0]);
-        T ch = HMAP ? a.ch[2][a.mat_h[2][i]] : a.ch[2][0];
-        T h = a.F[5][i] + ch * acc;
-        if (SRC) h += src_value(a, 5, x, y, z, step);
-        a.F[5][i] = h;
     }
 }
 
@@ -269,18 +336,28 @@ __global__ void __launch_bounds__(256) k_update_h(StepArgs<T> a) {
 }
 
 // ----------------------------------------------------------- E update -------
-template <typename T, bool SRC>
-__device__ __forceinline__ void e_finish(const StepArgs<T>& a, int c, long long i, int x, int y, int z, T acc, int step) {
-    const uint8_t id = a.mat_e[c] ? a.mat_e[c][i] : 0;
-    const T ce = a.ce[c][id];
-    const int fl = a.flags[c][id];
-    const int ps = a.poleset[c][id];
-    T e_old = a.F[c][i];
-    T src = SRC ? src_value(a, c, x, y, z, step) : T(0);
+// What the E update of a component reads at its own cell.
+template <typename T>
+struct ECell {
+    T ce, inveps, e;
+    int fl, ps;
+    __device__ __forceinline__ void load(const StepArgs<T>& a, int c, long long i) {
+        const uint8_t id = a.mat_e[c] ? a.mat_e[c][i] : 0;
+        e = a.F[c][i];
+        ce = a.ce[c][id];
+        fl = a.flags[c][id];
+        ps = a.poleset[c][id];
+        inveps = a.inveps[c][id];
+    }
+};
+template <typename T>
+__device__ __forceinline__ void e_finish(const StepArgs<T>& a, const ECell<T>& m, int c, long long i, int x, int y, int z, T acc, T src) {
+    const int ps = m.ps;
+    const T e_old = m.e;
     // A soft source on a D cell reaches the ADE but not E: D2E overwrites E
     // from D, which the source never touched (parallelFDTDField.hpp:1261-1281).
-    T e_base = (fl & CHIML_MAT_DCELL) ? e_old : e_old + src;
-    T e_ade = e_old + src;
+    const T e_base = (m.fl & CHIML_MAT_DCELL) ? e_old : e_old + src;
+    const T e_ade = e_old + src;
     T jsum = 0;
     if (ps >= 0) {
         const int* bx = a.box[c];
@@ -297,7 +374,7 @@ __device__ __forceinline__ void e_finish(const StepArgs<T>& a, int c, long long 
             jsum += Jn;
         }
     }
-    a.F[c][i] = e_base + ce * acc - a.inveps[c][id] * jsum;
+    a.F[c][i] = fma(-m.inveps, jsum, fma(m.ce, acc, e_base));
 }
 
 // 3D: Ex += ce[(Hz-Hz(y-1))/dy - (Hy-Hy(z-1))/dz], Ey += ce[(Hx-Hx(z-1))/dz -
@@ -319,38 +396,47 @@ __global__ void __launch_bounds__(256) k_update_e(StepArgs<T> a) {
     const T* Hx = a.F[3];
     const T* Hy = a.F[4];
     const T* Hz = a.F[5];
-    if (DIM == 3) {
-        if (x < nx - 1) {  // Ex
-            T dHz = Hz[i] - (y > 0 ? Hz[i - sy] : T(0));
-            T dHy = Hy[i] - (z > 0 ? Hy[i - sz] : T(0));
-            T acc;
-            if (!inpml) acc = dHz * a.inv_d[1] - dHy * a.inv_d[2];
-            else acc = pml_term(a.pml[0], 1, y, x, y, z, px, ny, dHz, dHz * a.inv_d[1]) - pml_term(a.pml[0], 2, z, x, y, z, px, ny, dHy, dHy * a.inv_d[2]);
-            e_finish<T, SRC>(a, 0, i, x, y, z, acc, step);
+    T sv[3] = {};
+    ECell<T> m[3];
+    if constexpr (DIM == 3) {
+        const bool xin = x < nx - 1, yin = y < ny - 1, zin = z < nz - 1;
+        const T hx = Hx[i], hy = Hy[i], hz = Hz[i];
+        const T hyx = x > 0 ? Hy[i - 1] : T(0), hzx = x > 0 ? Hz[i - 1] : T(0);
+        const T hxy = y > 0 ? Hx[i - sy] : T(0), hzy = y > 0 ? Hz[i - sy] : T(0);
+        const T hxz = z > 0 ? Hx[i - sz] : T(0), hyz = z > 0 ? Hy[i - sz] : T(0);
+        PmlCell<T> q[6];
+#pragma unroll
+        for (int c = 0; c < 3; ++c) m[c].load(a, c, i);
+        if (inpml) {
+            if (xin) {
+                q[0].load(a.pml[0], 1, y, x, y, z, px, ny);
+                q[1].load(a.pml[0], 2, z, x, y, z, px, ny);
+            }
+            if (yin) {
+                q[2].load(a.pml[1], 2, z, x, y, z, px, ny);
+                q[3].load(a.pml[1], 0, x, x, y, z, px, ny);
+            }
+            if (zin) {
+                q[4].load(a.pml[2], 0, x, x, y, z, px, ny);
+                q[5].load(a.pml[2], 1, y, x, y, z, px, ny);
+            }
         }
-        if (y < ny - 1) {  // Ey
-            T dHx = Hx[i] - (z > 0 ? Hx[i - sz] : T(0));
-            T dHz = Hz[i] - (x > 0 ? Hz[i - 1] : T(0));
-            T acc;
-            if (!inpml) acc = dHx * a.inv_d[2] - dHz * a.inv_d[0];
-            else acc = pml_term(a.pml[1], 2, z, x, y, z, px, ny, dHx, dHx * a.inv_d[2]) - pml_term(a.pml[1], 0, x, x, y, z, px, ny, dHz, dHz * a.inv_d[0]);
-            e_finish<T, SRC>(a, 1, i, x, y, z, acc, step);
-        }
-        if (z < nz - 1) {  // Ez
-            T dHy = Hy[i] - (x > 0 ? Hy[i - 1] : T(0));
-            T dHx = Hx[i] - (y > 0 ? Hx[i - sy] : T(0));
-            T acc;
-            if (!inpml) acc = dHy * a.inv_d[0] - dHx * a.inv_d[1];
-            else acc = pml_term(a.pml[2], 0, x, x, y, z, px, ny, dHy, dHy * a.inv_d[0]) - pml_term(a.pml[2], 1, y, x, y, z, px, ny, dHx, dHx * a.inv_d[1]);
-            e_finish<T, SRC>(a, 2, i, x, y, z, acc, step);
-        }
+        if (SRC) src_values(a, 0, x, y, z, step, sv);
+        const T i0 = a.inv_d[0], i1 = a.inv_d[1], i2 = a.inv_d[2];
+        if (xin) e_finish(a, m[0], 0, i, x, y, z, curl_cell(q[0], q[1], inpml, hz - hzy, i1, hy - hyz, i2), sv[0]);
+        if (yin) e_finish(a, m[1], 1, i, x, y, z, curl_cell(q[2], q[3], inpml, hx - hxz, i2, hz - hzx, i0), sv[1]);
+        if (zin) e_finish(a, m[2], 2, i, x, y, z, curl_cell(q[4], q[5], inpml, hy - hyx, i0, hx - hxy, i1), sv[2]);
     } else {
-        T dHy = Hy[i] - (x > 0 ? Hy[i - 1] : T(0));
-        T dHx = Hx[i] - (y > 0 ? Hx[i - sy] : T(0));
-        T acc;
-        if (!inpml) acc = dHy * a.inv_d[0] - dHx * a.inv_d[1];
-        else acc = pml_term(a.pml[2], 0, x, x, y, z, px, ny, dHy, dHy * a.inv_d[0]) - pml_term(a.pml[2], 1, y, x, y, z, px, ny, dHx, dHx * a.inv_d[1]);
-        e_finish<T, SRC>(a, 2, i, x, y, z, acc, step);
+        const T hx = Hx[i], hy = Hy[i];
+        const T hyx = x > 0 ? Hy[i - 1] : T(0), hxy = y > 0 ? Hx[i - sy] : T(0);
+        PmlCell<T> q[2];
+        m[2].load(a, 2, i);
+        if (inpml) {
+            q[0].load(a.pml[2], 0, x, x, y, z, px, ny);
+            q[1].load(a.pml[2], 1, y, x, y, z, px, ny);
+        }
+        if (SRC) src_values(a, 0, x, y, z, step, sv);
+        e_finish(a, m[2], 2, i, x, y, z, curl_cell(q[0], q[1], inpml, hy - hyx, a.inv_d[0], hx - hxy, a.inv_d[1]), sv[2]);
     }
 }
 
