@@ -7,7 +7,8 @@
 //   2. E sweep     : soft E sources, pole currents, E += curl H with CPML psi
 //                    (addPul, updateE/updateD, updateEPML, D2E)
 //                    3D FP32: k_h3_all / k_e3_all; 3D FP64: k_h3_int + k_h3_slab /
-//                    k_e3_int + k_e3_slab; 2D: k_h2v / k_e2v; else k_update_h / k_update_e
+//                    k_e3_int + k_e3_slab; 2D: k_tile2 (several steps) or k_h2v / k_e2v;
+//                    else k_update_h / k_update_e
 //   3. emitters    : k_ml_addp, k_ml_entry, then k_ml_pop_finish on recording steps
 //                    (parallelQEBase::addQE)
 //   4. t_step += 1 : plain launches are given the step number by the host;
