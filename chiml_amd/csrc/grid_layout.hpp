@@ -37,10 +37,14 @@ inline GridLayout grid_layout(int nx, int ny, int nz, const int* T, int psi_lo, 
     g.rows = g.split && (fp32 || !aligned);
     // Groups leave a small 3D grid about one wave per SIMD, each waiting for
     // memory alone, so a small grid that had to be padded is stepped one thread
-    // per cell (FP32 64^3, 10-cell CPML: 23.5 us a step per cell, 26.2 in
-    // groups; 101x93x87: 69 and 49; FP64 65x64x63: 47 and 37); a batch of them
-    // fills the chip and takes the groups (56^3, 72^3 and 88^3 together with
-    // three 2D grids: 72 and 51 us a step).
-    g.cellwise = g.split && !aligned && static_cast<double>(nx) * ny * nz * (fp32 ? 4 : 8) < 1.5e6;
+    // per cell.  The line goes by the bytes of a component over the threads
+    // launched (blocks of 64 x 4 cells: a row of 66 takes two).  us a step per
+    // cell / in groups, FP32: 30^3 13.0/16.4, 64^3 15.4/17.9, 45x75x75 (1.46 MB)
+    // 16.2/18.2, 33x85x81 (1.82) 18.7/17.9, 66x60x60 (1.84) 20.8/17.5, 72^3 (2.65)
+    // 23.9/18.5; FP64: 50^3 (1.33) 16.1/16.8, 126x42x42 (1.89) 20.2/18.8, 65^3
+    // 30.6/20.6.  A batch of such grids fills the chip and takes the groups (56^3,
+    // 72^3 and 88^3 together with three 2D grids: 72 and 51 us a step).
+    const double threads = static_cast<double>(round_up(nx, 64)) * round_up(ny, 4) * nz;
+    g.cellwise = g.split && !aligned && threads * (fp32 ? 4 : 8) < 1.48e6;
     return g;
 }
