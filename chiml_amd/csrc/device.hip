@@ -4439,7 +4439,7 @@ void enable_tiles(chiml_dev* c, const chiml_problem_t* p, StepArgs<T>& a, Sample
     HIP_TRY(hipDeviceGetAttribute(&lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, c->device));
     int best = -1;
     double best_t = 0.0;
-    size_t best_lds = 0;
+    size_t best_lds = 0, lds_limit = 0;
     for (int sh = 0; sh < (sizeof(T) == 4 ? 3 : 2); ++sh)
         pick_tile<T>(sh, [&](auto shape) {
             using SH = decltype(shape);
@@ -4454,6 +4454,7 @@ void enable_tiles(chiml_dev* c, const chiml_problem_t* p, StepArgs<T>& a, Sample
                 best = sh;
                 best_t = est;
                 best_lds = dyn;
+                lds_limit = static_cast<size_t>(lds_max) - at.sharedSizeBytes;
             }
         });
     if (best < 0) return;
@@ -4464,9 +4465,11 @@ void enable_tiles(chiml_dev* c, const chiml_problem_t* p, StepArgs<T>& a, Sample
         uy = SH::uy;
         rx = SH::rx;
         rows = SH::r;
+        // the limit is the process's, not this context's: all that a block may
+        // have, whatever this deck needs of it
         if (best_lds > 0)
             HIP_TRY(hipFuncSetAttribute(reinterpret_cast<const void*>(k_tile2<T, SH>), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                        static_cast<int>(best_lds)));
+                                        static_cast<int>(lds_limit)));
     });
     const int ntx = (p->nx + ux - 1) / ux, nty = (p->ny + uy - 1) / uy;
     // the detector points of each tile (points past the grid's edge read the

@@ -1,0 +1,83 @@
+"""Host-side choices of the device layer (which kernels a call launches, with
+what shared memory, and what happens when memory runs out), seen on the CPU:
+a stand-in for the HIP runtime (tests/c/fake_hip.cpp) records the calls that
+libchiml_amd.so makes.  Each test runs in a process of its own, since the
+stand-in has to be loaded before the library."""
+import json
+import os
+import shutil
+import subprocess
+import sys
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+PRELUDE = """
+import ctypes, json, sys
+fake = ctypes.CDLL({fake!r}, mode=ctypes.RTLD_GLOBAL)
+fake.fake_hip_log.restype = ctypes.c_char_p
+fake.fake_hip_fail_size.argtypes = [ctypes.c_size_t]
+import chiml_amd
+from chiml_amd import decks
+
+def deck2(n, prec, poles=0, steps=400, pml=8, flux=False):
+    d = 0.05
+    dk = decks.empty_deck((n[0], n[1], 1), d, steps, pml, precision=prec)
+    dk["ObjectList"].append({{"shape": "cylinder", "material": "custom", "eps": 2.5, "pols": decks.gold_like_pols()[:poles],
+                             "radius": 5.3 * d, "length": 1.0, "loc": [0.0] * 3, "Basis_Set": [],
+                             "unit_vectors": [{{"uvec": [1, 0, 0]}}, {{"uvec": [0, 0, 1]}}, {{"uvec": [0, 1, 0]}}]}})
+    dk["SourceList"].append({{"pol": "Ez", "size": [0.0] * 3, "loc": [0.0] * 3, "PulseList": [decks.gaussian_pulse(0.2, 0.2, 3.0, 1.0)]}})
+    if flux:
+        dk["FluxList"].append({{"name": "f", "size": [20 * d, 20 * d, 0.0], "loc": [0.0] * 3, "lamL": 2.0, "lamR": 9.0, "nfreq": 3}})
+    return json.dumps(dk)
+
+def log():
+    out = fake.fake_hip_log().decode().split("\\n")[:-1]
+    fake.fake_hip_clear()
+    return [line.split() for line in out]
+
+def kernels(lines):
+    # the launched kernels by their short names, the step counter's left out
+    names = ["k_" + line[1].split("k_", 1)[1].split("I", 1)[0] for line in lines if line[0] in ("launch", "capture")]
+    return [k for k in names if not k.startswith("k_set_step")]
+"""
+
+
+@pytest.fixture(scope="module")
+def fake(tmp_path_factory):
+    gxx = shutil.which("g++")
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    if not gxx or not os.path.exists(os.path.join(rocm, "include", "hip", "hip_runtime_api.h")):
+        pytest.skip("needs g++ and the HIP headers")
+    so = str(tmp_path_factory.mktemp("fake") / "fake_hip.so")
+    subprocess.check_call([gxx, "-O1", "-std=c++17", "-shared", "-fPIC", "-D__HIP_PLATFORM_AMD__", "-I", os.path.join(rocm, "include"),
+                           "-o", so, os.path.join(ROOT, "tests", "c", "fake_hip.cpp")])
+    return so
+
+
+def run(fake, body):
+    """Runs body after PRELUDE; what it prints last is JSON."""
+    r = subprocess.run([sys.executable, "-c", PRELUDE.format(fake=fake) + body], cwd=ROOT, capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, r.stderr[-2000:]
+    return json.loads(r.stdout.strip().split("\n")[-1])
+
+
+def test_tile_lds_limit_outlives_a_smaller_deck(fake):
+    """A kernel's limit of dynamic LDS belongs to the process: a deck with
+    fewer poles must not lower it below what a live one launches with."""
+    lines = run(fake, """
+a = chiml_amd.FDTDField(deck2((64, 64), "fp32", poles=3))
+b = chiml_amd.FDTDField(deck2((64, 64), "fp32", poles=1))
+for sim in (a, b, a):
+    sim.step(8)
+print(json.dumps(log()))
+""")
+    limit, tiles = {}, 0
+    for line in lines:
+        if line[0] == "attribute":
+            limit[line[1]] = int(line[2])
+        elif line[0] == "launch" and "k_tile2" in line[1]:
+            tiles += 1
+            assert int(line[4]) <= limit[line[1]]
+    assert tiles == 3

@@ -1,0 +1,61 @@
+"""Calls whose kernels depend on more than the deck -- several live contexts,
+step counts, batches -- against the same deck stepped alone, bit for bit, or
+against the FP64 oracle."""
+import json
+
+import numpy as np
+import pytest
+
+import chiml_amd
+from chiml_amd import decks
+
+pytestmark = pytest.mark.gpu
+
+
+def _deck2(n, prec, poles=0, pml=8, steps=200, flux=False):
+    d = 0.05
+    dk = decks.empty_deck((n[0], n[1], 1), d, steps, pml, precision=prec)
+    r = (min(n) - 2 * pml) / 4.0 + 0.3
+    dk["ObjectList"].append({"shape": "cylinder", "material": "custom", "eps": 2.5, "pols": decks.gold_like_pols()[:poles], "radius": r * d,
+                             "length": 1.0, "loc": [0.2 * d, -0.3 * d, 0.0], "Basis_Set": [],
+                             "unit_vectors": [{"uvec": [1, 0, 0]}, {"uvec": [0, 0, 1]}, {"uvec": [0, 1, 0]}]})
+    for pol, x, y in (("Ez", n[0] // 2 + 2, n[1] // 2), ("Hx", pml + 1, n[1] // 2 - 3)):
+        pulse = decks.gaussian_pulse(0.3, 1.0, 3.0, 1.0)
+        pulse["t_0"] = 0.1
+        dk["SourceList"].append({"pol": pol, "size": [0.0] * 3, "loc": [decks._pos(x, n[0], d), decks._pos(y, n[1], d), 0.0], "PulseList": [pulse]})
+    dk["DetectorList"].append({"type": "Ez", "dtc_class": "cout", "fname": "d", "size": [0.0] * 3,
+                               "loc": [decks._pos(n[0] // 2 - 4, n[0], d), decks._pos(n[1] // 2 + 5, n[1], d), 0.0]})
+    if flux:
+        dk["FluxList"].append({"name": "flux", "size": [(n[0] // 2) * d, (n[1] // 2) * d, 0.0], "loc": [0.0] * 3, "lamL": 2.0, "lamR": 9.0,
+                               "nfreq": 4})
+    return json.dumps(dk)
+
+
+def _results(sim):
+    sim.sync()
+    r = {f"f{c}": sim.field(c) for c in range(6)}
+    r.update({f"d{k}": d.series()[1] for k, d in enumerate(sim.dtcArr())})
+    r.update({f"x{k}": f.getFlux() for k, f in enumerate(sim.fluxArr())})
+    return r
+
+
+def _same(a, b, label):
+    assert a.keys() == b.keys(), label
+    assert np.max(np.abs(a["f2"])) > 0, label
+    for k in a:
+        assert np.array_equal(a[k], b[k]), (label, k, float(np.max(np.abs(a[k] - b[k]))))
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+def test_live_decks_of_different_pole_counts(prec):
+    """One tile shape, three pole counts alive at once, stepped in turn."""
+    sims = [chiml_amd.FDTDField(_deck2((64, 60), prec, poles=p)) for p in (3, 1, 2)]
+    for _ in range(3):
+        for sim in sims:
+            sim.step(20)
+    for p, sim in zip((3, 1, 2), sims):
+        alone = chiml_amd.FDTDField(_deck2((64, 60), prec, poles=p))
+        alone.step(60)
+        _same(_results(alone), _results(sim), p)
+        alone.close()
+        sim.close()
