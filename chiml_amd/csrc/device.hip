@@ -4472,13 +4472,13 @@ void enable_tiles(chiml_dev* c, const chiml_problem_t* p, StepArgs<T>& a, Sample
                                         static_cast<int>(lds_limit)));
     });
     const int ntx = (p->nx + ux - 1) / ux, nty = (p->ny + uy - 1) / uy;
-    // the detector points of each tile (points past the grid's edge read the
-    // zero ghost: their samples stay the zeros of the output buffer)
+    // the detector points of each tile (points outside the grid read the zero
+    // ghost: their samples stay the zeros of the output buffer)
     std::vector<std::vector<TileDet>> of(static_cast<size_t>(ntx) * nty);
     for (int d = 0, t = 0; d < c->ndet; ++d)
         for (int k = 0; k < c->det_npts[d]; ++k, ++t) {
             const long long cell = p->det_cell[2 * t];
-            if (cell < 0) continue;
+            if (cell < 0 || cell >= static_cast<long long>(p->nx) * p->ny) continue;
             const int x = static_cast<int>(cell % p->nx), y = static_cast<int>(cell / p->nx);
             const int lx = x % ux + kTileSteps, ly = y % uy + kTileSteps;
             TileDet q{};

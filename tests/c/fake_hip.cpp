@@ -17,7 +17,11 @@
 
 namespace {
 std::string g_log;
-std::map<const void*, std::string> g_names;
+// (the library's kernels may be registered before this file's own start-up)
+std::map<const void*, std::string>& names() {
+    static auto* m = new std::map<const void*, std::string>;
+    return *m;
+}
 size_t g_fail_size = 0;
 int g_fail_seen = 0;
 bool g_capturing = false;
@@ -43,7 +47,7 @@ void** __hipRegisterFatBinary(const void*) {
 }
 void __hipUnregisterFatBinary(void**) {}
 void __hipRegisterFunction(void**, const void* host, char*, const char* name, unsigned, void*, void*, void*, void*, int*) {
-    g_names[host] = name;
+    names()[host] = name;
 }
 void __hipRegisterVar(void**, void*, char*, char*, int, size_t, int, int) {}
 hipError_t __hipPushCallConfiguration(dim3 g, dim3 b, size_t shm, hipStream_t s) {
@@ -58,7 +62,7 @@ hipError_t __hipPopCallConfiguration(dim3* g, dim3* b, size_t* shm, hipStream_t*
     return hipSuccess;
 }
 hipError_t hipLaunchKernel(const void* fn, dim3 g, dim3 b, void**, size_t shm, hipStream_t) {
-    put((g_capturing ? "capture " : "launch ") + g_names[fn] + " " + std::to_string(g.x) + " " + std::to_string(b.x) + " " + std::to_string(shm));
+    put((g_capturing ? "capture " : "launch ") + names()[fn] + " " + std::to_string(g.x) + " " + std::to_string(b.x) + " " + std::to_string(shm));
     return hipSuccess;
 }
 hipError_t hipFuncGetAttributes(hipFuncAttributes* a, const void*) {
@@ -67,7 +71,7 @@ hipError_t hipFuncGetAttributes(hipFuncAttributes* a, const void*) {
     return hipSuccess;
 }
 hipError_t hipFuncSetAttribute(const void* fn, hipFuncAttribute, int v) {
-    put("attribute " + g_names[fn] + " " + std::to_string(v));
+    put("attribute " + names()[fn] + " " + std::to_string(v));
     return hipSuccess;
 }
 hipError_t hipDeviceGetAttribute(int* v, hipDeviceAttribute_t, int) {

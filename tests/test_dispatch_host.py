@@ -81,3 +81,13 @@ print(json.dumps(log()))
             tiles += 1
             assert int(line[4]) <= limit[line[1]]
     assert tiles == 3
+
+
+def test_detector_cell_past_the_grid(fake, tmp_path):
+    """A detector cell outside a 2D grid is never sampled; the tables of the
+    tiles must not be written for it."""
+    exe, lib = str(tmp_path / "far_detector"), os.path.join(ROOT, "chiml_amd", "libchiml_amd.so")
+    subprocess.check_call(["gcc", "-std=c99", "-I", os.path.join(ROOT, "include"), "-o", exe, os.path.join(ROOT, "tests", "c", "far_detector.c"),
+                           "-Wl,--no-as-needed", fake, lib, "-Wl,-rpath," + os.path.dirname(lib), "-Wl,--unresolved-symbols=ignore-in-shared-libs"])
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0 and r.stdout.strip() == "OK", (r.returncode, r.stdout, r.stderr)
