@@ -4501,26 +4501,30 @@ void enable_tiles(chiml_dev* c, const chiml_problem_t* p, StepArgs<T>& a, Sample
         ofs.push_back(static_cast<int>(pts.size()));
     }
     if (pts.empty()) pts.emplace_back();
-    c->tile_det_ofs = c->upload<int>(ofs.data(), ofs.size());
-    c->tile_det = c->upload<TileDet>(pts.data(), pts.size());
-    c->tile_nset = p->npoleset;
     const size_t N = static_cast<size_t>(c->px) * p->ny;
     T* const psi[4] = {a.pml[3].psi[1], a.pml[4].psi[0], a.pml[2].psi[0], a.pml[2].psi[1]};
     const size_t psin[4] = {static_cast<size_t>(a.pml[3].S[1]) * c->px, static_cast<size_t>(a.pml[4].S[0]) * p->ny,
                             static_cast<size_t>(a.pml[2].S[0]) * p->ny, static_cast<size_t>(a.pml[2].S[1]) * c->px};
-    for (int j = 0; j < 3; ++j) {
-        c->tbuf[0][j] = a.F[2 + j];
-        c->tbuf[1][j] = c->zeros<T>(N);
+    const size_t held = c->bufs.size(), footprint = c->footprint;
+    try {
+        c->tile_det_ofs = c->upload<int>(ofs.data(), ofs.size());
+        c->tile_det = c->upload<TileDet>(pts.data(), pts.size());
+        for (int j = 0; j < 3; ++j) c->tbuf[1][j] = c->zeros<T>(N);
+        for (int j = 0; j < 4; ++j) c->tbuf[1][3 + j] = psi[j] ? c->zeros<T>(psin[j]) : nullptr;
+        for (int j = 7; npole > 0 && j < 9; ++j) c->tbuf[1][j] = c->zeros<T>(static_cast<size_t>(a.boxn[2]) * npole);
+    } catch (const std::exception&) {
+        // no room for the second set: the sweeps need none
+        (void)hipGetLastError();
+        c->bufs.resize(held);
+        c->footprint = footprint;
+        return;
     }
-    for (int j = 0; j < 4; ++j) {
-        c->tbuf[0][3 + j] = psi[j];
-        c->tbuf[1][3 + j] = psi[j] ? c->zeros<T>(psin[j]) : nullptr;
-    }
+    c->tile_nset = p->npoleset;
+    for (int j = 0; j < 3; ++j) c->tbuf[0][j] = a.F[2 + j];
+    for (int j = 0; j < 4; ++j) c->tbuf[0][3 + j] = psi[j];
     if (npole > 0) {
         c->tbuf[0][7] = a.P[2];
         c->tbuf[0][8] = a.J[2];
-        c->tbuf[1][7] = c->zeros<T>(static_cast<size_t>(a.boxn[2]) * npole);
-        c->tbuf[1][8] = c->zeros<T>(static_cast<size_t>(a.boxn[2]) * npole);
     }
     c->tile = true;
     c->tile_shape = best;

@@ -91,3 +91,26 @@ def test_detector_cell_past_the_grid(fake, tmp_path):
                            "-Wl,--no-as-needed", fake, lib, "-Wl,-rpath," + os.path.dirname(lib), "-Wl,--unresolved-symbols=ignore-in-shared-libs"])
     r = subprocess.run([exe], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0 and r.stdout.strip() == "OK", (r.returncode, r.stdout, r.stderr)
+
+
+@pytest.mark.parametrize("prec,word", [("fp32", 4), ("fp64", 8)])
+def test_no_memory_for_a_second_set_of_fields(fake, prec, word):
+    """A 2D deck whose second set of fields does not fit runs on the sweeps,
+    which need one set, and holds no part of the second."""
+    out = run(fake, f"""
+fake.fake_hip_fail_size(68 * 61 * {word})  # the second set's fields: the first set's three are one allocation
+a = chiml_amd.FDTDField(deck2((68, 61), "{prec}", poles=1))
+refused = [line for line in log() if line[0] == "refused"]
+a.step(3)
+k = kernels(log())
+fake.fake_hip_fail_size(0)
+b = chiml_amd.FDTDField(deck2((68, 61), "{prec}", poles=1))
+log()
+b.step(3)
+print(json.dumps([len(refused), k, kernels(log()), a.footprint(), b.footprint(), float(abs(a.field(2)).max())]))
+""")
+    refused, sweeps, tiles, one, two, _ = out
+    assert refused == 1
+    assert sweeps == ["k_h2v", "k_e2v"] * 3
+    assert tiles == ["k_tile2"]
+    assert one < two
