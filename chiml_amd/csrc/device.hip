@@ -3360,7 +3360,12 @@ struct chiml_dev {
     bool profile = false;
     std::string profile_only;  // non-empty: time only launches of this kernel
     std::map<std::string, std::pair<double, int>> prof;
-    std::vector<std::pair<std::string, std::pair<hipEvent_t, hipEvent_t>>> pending;
+    struct Span {  // an event pair around a launch, or around the launches of n steps
+        std::string name;
+        hipEvent_t e0, e1;
+        int n;
+    };
+    std::vector<Span> pending;
 
     template <typename T>
     T* upload(const T* src, size_t n) {
@@ -3962,9 +3967,10 @@ struct Timed {
     chiml_dev* c;
     const char* name;
     hipEvent_t e0 = nullptr, e1 = nullptr;
+    int count;
     bool on;
-    Timed(chiml_dev* c_, const char* n)
-        : c(c_), name(n), on(c_->profile && !c_->device_flush && (c_->profile_only.empty() || in_name_list(c_->profile_only, n))) {
+    Timed(chiml_dev* c_, const char* n, int count_ = 1)
+        : c(c_), name(n), count(count_), on(c_->profile && !c_->device_flush && (c_->profile_only.empty() || in_name_list(c_->profile_only, n))) {
         if (on) {
             (void)hipEventCreate(&e0);
             (void)hipEventCreate(&e1);
@@ -3974,7 +3980,7 @@ struct Timed {
     ~Timed() {
         if (on) {
             (void)hipEventRecord(e1, c->stream);
-            c->pending.push_back({name, {e0, e1}});
+            c->pending.push_back({name, e0, e1, count});
         }
     }
 };
@@ -4401,6 +4407,7 @@ void do_tile_steps(chiml_dev* c, StepArgs<T>& a, SampleArgs<T>& s, int n) {
         t.step_next = host ? nullptr : ctr + (1 - cur);
         t.nstep = k;
         {
+            Timed fs(c, "field_step", k);
             Timed tm(c, "update_tile");
             pick_tile<T>(c->tile_shape, [&](auto sh) {
                 using SH = decltype(sh);
@@ -4538,13 +4545,13 @@ void enable_tiles(chiml_dev* c, const chiml_problem_t* p, StepArgs<T>& a, Sample
 void collect_profile(chiml_dev* c) {
     for (auto& pe : c->pending) {
         float ms = 0.0f;
-        (void)hipEventSynchronize(pe.second.second);
-        (void)hipEventElapsedTime(&ms, pe.second.first, pe.second.second);
-        auto& slot = c->prof[pe.first];
+        (void)hipEventSynchronize(pe.e1);
+        (void)hipEventElapsedTime(&ms, pe.e0, pe.e1);
+        auto& slot = c->prof[pe.name];
         slot.first += ms;
-        slot.second += 1;
-        (void)hipEventDestroy(pe.second.first);
-        (void)hipEventDestroy(pe.second.second);
+        slot.second += pe.n;
+        (void)hipEventDestroy(pe.e0);
+        (void)hipEventDestroy(pe.e1);
     }
     c->pending.clear();
 }
@@ -5377,8 +5384,8 @@ void chiml_dev_destroy(chiml_dev_t* c) {
     for (hipGraphExec_t e : c->tile_exec)
         if (e) (void)hipGraphExecDestroy(e);
     for (auto& pe : c->pending) {
-        (void)hipEventDestroy(pe.second.first);
-        (void)hipEventDestroy(pe.second.second);
+        (void)hipEventDestroy(pe.e0);
+        (void)hipEventDestroy(pe.e1);
     }
     c->bufs.clear();
     c->qes.clear();

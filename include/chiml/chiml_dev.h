@@ -283,7 +283,8 @@ int chiml_dev_profile(chiml_dev_t* ctx, int enable);
 /* As chiml_dev_profile(ctx, 1) but timing only the launches of the named
  * kernels (one name, or several separated by commas), so that a timed run
  * carries few event records per step.  "field_step" names one event pair
- * around all field-update launches of each step. */
+ * around all field-update launches of each step; a launch that takes several
+ * steps (2D tiles, "update_tile") counts as that many. */
 int chiml_dev_profile_only(chiml_dev_t* ctx, const char* kernel);
 int chiml_dev_profile_read(chiml_dev_t* ctx, const char* kernel, double* total_ms, int* launches);
 /* Device memory the context holds (bytes). */

@@ -114,3 +114,20 @@ print(json.dumps([len(refused), k, kernels(log()), a.footprint(), b.footprint(),
     assert sweeps == ["k_h2v", "k_e2v"] * 3
     assert tiles == ["k_tile2"]
     assert one < two
+
+
+def test_field_step_timing_counts_the_steps(fake):
+    """profile_only("field_step") times the field update of every step, in
+    whatever number of launches the steps are taken."""
+    got = run(fake, """
+out = []
+for flux in (False, True):
+    sim = chiml_amd.FDTDField(deck2((68, 61), "fp32", flux=flux))
+    sim.profile_only("field_step")
+    sim.step(20)
+    sim.step(1)
+    ms, n = sim.profile_read("field_step")
+    out.append([ms > 0, n])
+print(json.dumps(out))
+""")
+    assert got == [[True, 21], [True, 21]]
