@@ -2349,7 +2349,8 @@ using TileM = TileShape<64, 2, 16>;
 using TileL = TileShape<64, 4, 16>;
 
 // ----------------------------------------------------- step counter ---------
-__global__ void k_set_step(int* step, int v) { *step = v; }
+// both slots: captured steps start on either
+__global__ void k_set_step(int* step, int v) { step[0] = step[1] = v; }
 
 // ----------------------------------------------- detectors and DFT ----------
 
@@ -3288,10 +3289,11 @@ struct chiml_dev {
     int nmat[3] = {1, 1, 1};
     int enq_step = 0;    // step counter value after the step being enqueued
     int graph_steps = 0;  // > 0: replay captured graphs of this many steps (even)
-    int graph_parity = 0;  // counter slot (steps_done & 1) the captured graph starts on
     bool capturing = false;  // do_steps is being captured into a graph
     bool device_flush = false;  // launch the DFT flush every step; it decides on the device
-    hipGraphExec_t gexec = nullptr;
+    hipGraphExec_t gexec[2] = {nullptr, nullptr};  // captured graphs, by the tile buffer set they start on (0: no tiles)
+    int graph_parity[2] = {0, 0};  // and the counter slot that a graph of sweeps starts on
+    bool graph_tiles = false;      // the graphs are of tile launches
     bool split = false;  // 3D interior + CPML-slab kernels
     bool rows = false;   // split: whole-row interior, one launch per field
     double step_bytes = 0;     // fields and emitter state
@@ -3314,7 +3316,6 @@ struct chiml_dev {
     const int* tile_det_ofs = nullptr;
     const TileDet* tile_det = nullptr;
     int tile_nset = 0;
-    hipGraphExec_t tile_exec[2] = {nullptr, nullptr};  // captured graphs, by the buffer set they start on
     bool fuse_sample = false;  // 2D: the E kernel takes the point detectors (no DFT, few single-cell points)
     bool det_single_field = true;  // every point detector reads one field (two cells) per point
     long long ade_groups = 0;  // largest pole-box group count over the E components (split path)
@@ -4294,7 +4295,7 @@ void do_steps(chiml_dev* c, StepArgs<T>& a, SampleArgs<T>& s, int n) {
     }
     if (host && n > 0) {
         const int end = c->steps_done + n;
-        hipLaunchKernelGGL(k_set_step, dim3(1), dim3(1), 0, c->stream, ctr + (end & 1), end);
+        hipLaunchKernelGGL(k_set_step, dim3(1), dim3(1), 0, c->stream, ctr, end);
     }
     a.stepv = -1;
     s.stepv = -1;
@@ -4323,8 +4324,10 @@ void set_tile_buffers(chiml_dev* c, StepArgs<T>& a, SampleArgs<T>& s, int k) {
     }
     T** psi[4] = {&a.pml[3].psi[1], &a.pml[4].psi[0], &a.pml[2].psi[0], &a.pml[2].psi[1]};
     for (int j = 0; j < 4; ++j) *psi[j] = static_cast<T*>(b[3 + j]);
-    a.P[2] = static_cast<T*>(b[7]);
-    a.J[2] = static_cast<T*>(b[8]);
+    if (c->tile_npole > 0) {
+        a.P[2] = static_cast<T*>(b[7]);
+        a.J[2] = static_cast<T*>(b[8]);
+    }
     c->tile_cur = k;
 }
 
@@ -4391,13 +4394,35 @@ TileArgs<T> tile_args(const chiml_dev* c, const StepArgs<T>& a, int cur) {
 
 // n steps in launches of up to kTileSteps.  Captured steps take an even
 // number of launches, so that a graph ends on the buffer set it starts on.
+int tile_launches(int n, bool captured) {
+    const int l = (n + kTileSteps - 1) / kTileSteps;
+    return captured ? l + l % 2 : l;
+}
+
+// Do tile launches beat the sweeps for n steps in one go?  A launch reads and
+// writes its whole state with the halo (1.8-4x the cells) however few steps it
+// takes, so one or two steps are faster swept, in place, on grids large enough
+// for that to outweigh the launches saved.  us a call of 1, 2 and 3 steps that
+// is waited for, sweeps / tiles: FP32 384^2 21.2/21.2, 30/22; 512^2 21.3/24.3,
+// 31/26; 1024^2 25.7/32.7, 39/35; without the wait 2048^2 35/62, 68/71, 102/80;
+// FP64 384^2 21.3/21.6, 31/23; 512^2 22.5/27.6, 33/29; 832^2 25.9/39.9, 40/44;
+// 2048^2 59/125, 116/144, 174/164.  Replayed from graphs the sweeps cost no host
+// launch and the second line lies lower (graphs of 4, us a step: FP32 896^2
+// 13.1/11.4, 1280^2 14.9/16.0; FP64 576^2 11.8/9.8, 768^2 12.9/13.6).
+bool tile_pays(const chiml_dev* c, int n) {
+    const int l = tile_launches(n, c->capturing), k = (n + l - 1) / l;
+    if (k > 2) return true;
+    const double cells = static_cast<double>(c->nx) * c->ny;
+    if (k == 1) return cells < 400.0 * 400;
+    const double side = c->prec == 32 ? (c->capturing ? 1000.0 : 2000.0) : (c->capturing ? 620.0 : 800.0);
+    return cells < side * side;
+}
+
 template <typename T>
 void do_tile_steps(chiml_dev* c, StepArgs<T>& a, SampleArgs<T>& s, int n) {
-    if (n == 0) return;
     const bool host = !c->capturing;
     int* ctr = c->step_ctr.as<int>();
-    int launches = (n + kTileSteps - 1) / kTileSteps;
-    if (!host && launches % 2) ++launches;
+    const int launches = tile_launches(n, !host);
     int cur = c->tile_cur;
     for (int l = 0, done = 0; l < launches; ++l) {
         const int k = (n - done + launches - l - 1) / (launches - l);
@@ -4421,7 +4446,7 @@ void do_tile_steps(chiml_dev* c, StepArgs<T>& a, SampleArgs<T>& s, int n) {
     }
     c->steps_done += n;
     c->enq_step = c->steps_done;
-    if (host) hipLaunchKernelGGL(k_set_step, dim3(1), dim3(1), 0, c->stream, ctr + cur, c->steps_done);
+    if (host) hipLaunchKernelGGL(k_set_step, dim3(1), dim3(1), 0, c->stream, ctr, c->steps_done);
     set_tile_buffers<T>(c, a, s, cur);
 }
 
@@ -5002,27 +5027,32 @@ int chiml_dev_create(const chiml_problem_t* p, chiml_dev_t** out) {
 }
 
 namespace {
-void enqueue_steps(chiml_dev* c, int n) {
-    if (c->tile) {
-        if (c->prec == 32) do_tile_steps<float>(c, c->a32, c->s32, n);
-        else do_tile_steps<double>(c, c->a64, c->s64, n);
-    } else if (c->prec == 32) do_steps<float>(c, c->a32, c->s32, n);
+void sweep_steps(chiml_dev* c, int n) {
+    if (c->prec == 32) do_steps<float>(c, c->a32, c->s32, n);
     else do_steps<double>(c, c->a64, c->s64, n);
+}
+
+void enqueue_steps(chiml_dev* c, int n) {
+    if (n == 0) return;
+    if (!c->tile || !tile_pays(c, n)) sweep_steps(c, n);
+    else if (c->prec == 32) do_tile_steps<float>(c, c->a32, c->s32, n);
+    else do_tile_steps<double>(c, c->a64, c->s64, n);
 }
 
 // Captures graph_steps steps of this context's launch sequence once; every
 // launch reads the step number from the device counter, so one graph serves
-// every chunk of the run.
+// every chunk of the run that starts on the same buffers.
 void ensure_graph(chiml_dev* c) {
-    hipGraphExec_t& exec = c->tile ? c->tile_exec[c->tile_cur] : c->gexec;
+    hipGraphExec_t& exec = c->gexec[c->tile_cur];
     if (exec) return;
     std::lock_guard<std::mutex> lk(g_capture_mu);
     hipGraph_t g = nullptr;
     const int saved = c->steps_done, saved_enq = c->enq_step;
-    c->graph_parity = c->steps_done & 1;
+    c->graph_parity[c->tile_cur] = c->steps_done & 1;
     HIP_TRY(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
     c->capturing = true;
     try {
+        c->graph_tiles = c->tile && tile_pays(c, c->graph_steps);
         enqueue_steps(c, c->graph_steps);
     } catch (...) {
         c->capturing = false;
@@ -5048,18 +5078,12 @@ int chiml_dev_step(chiml_dev_t* c, int n) {
         if (c->graph_steps > 0) {
             while (n >= c->graph_steps) {
                 ensure_graph(c);
-                if (c->tile) {
-                    HIP_TRY(hipGraphLaunch(c->tile_exec[c->tile_cur], c->stream));
-                    c->steps_done += c->graph_steps;
-                    n -= c->graph_steps;
-                    continue;
-                }
-                if ((c->steps_done & 1) != c->graph_parity) {  // realign the counter slot with one plain step
-                    enqueue_steps(c, 1);
+                if (!c->graph_tiles && (c->steps_done & 1) != c->graph_parity[c->tile_cur]) {
+                    sweep_steps(c, 1);  // realign the counter slot with one plain step
                     --n;
                     continue;
                 }
-                HIP_TRY(hipGraphLaunch(c->gexec, c->stream));
+                HIP_TRY(hipGraphLaunch(c->gexec[c->tile_cur], c->stream));
                 c->steps_done += c->graph_steps;
                 n -= c->graph_steps;
             }
@@ -5074,17 +5098,15 @@ int chiml_dev_step(chiml_dev_t* c, int n) {
 
 int chiml_dev_set_graph(chiml_dev_t* c, int steps_per_graph) {
     if (!c || steps_per_graph < 0) return fail(c, CHIML_E_INVALID, "invalid argument");
-    if (c->gexec) {
-        (void)hipGraphExecDestroy(c->gexec);
-        c->gexec = nullptr;
-    }
-    for (hipGraphExec_t& e : c->tile_exec) {
+    for (hipGraphExec_t& e : c->gexec) {
         if (e) (void)hipGraphExecDestroy(e);
         e = nullptr;
     }
     // even, so that every replay starts on the counter slot the graph was captured on
     c->graph_steps = steps_per_graph + (steps_per_graph & 1);
     c->device_flush = steps_per_graph > 0;
+    // graphs of tiles and of sweeps leave different slots current
+    if (c->tile) hipLaunchKernelGGL(k_set_step, dim3(1), dim3(1), 0, c->stream, c->step_ctr.as<int>(), c->steps_done);
     return CHIML_OK;
 }
 
@@ -5380,8 +5402,7 @@ void chiml_dev_destroy(chiml_dev_t* c) {
     if (!c) return;
     std::lock_guard<std::mutex> lk(g_capture_mu);
     (void)hipStreamSynchronize(c->stream);
-    if (c->gexec) (void)hipGraphExecDestroy(c->gexec);
-    for (hipGraphExec_t e : c->tile_exec)
+    for (hipGraphExec_t e : c->gexec)
         if (e) (void)hipGraphExecDestroy(e);
     for (auto& pe : c->pending) {
         (void)hipEventDestroy(pe.e0);

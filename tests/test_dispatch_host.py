@@ -131,3 +131,59 @@ for flux in (False, True):
 print(json.dumps(out))
 """)
     assert got == [[True, 21], [True, 21]]
+
+
+# n, steps of one call, tiles? -- both sides of each line of tile_pays
+SHORT = {"fp32": [(390, 1, True), (410, 1, False), (410, 2, True), (1990, 2, True), (2010, 2, False), (2010, 3, True)],
+         "fp64": [(390, 1, True), (410, 1, False), (410, 2, True), (790, 2, True), (810, 2, False), (810, 3, True)]}
+GRAPH = {"fp32": [(390, 2, True), (410, 2, False), (990, 4, True), (1010, 4, False), (1010, 6, True)],
+         "fp64": [(390, 2, True), (410, 2, False), (610, 4, True), (630, 4, False), (630, 6, True)]}
+
+
+@pytest.mark.parametrize("prec", ["fp32", "fp64"])
+def test_short_calls_on_large_2d_grids_take_the_sweeps(fake, prec):
+    """One or two steps (or a graph of 2 or 4) of a large 2D grid go through
+    the sweeps, in place; from three steps a launch on, tiles."""
+    got = run(fake, f"""
+out = []
+for n, k, _ in {SHORT[prec]}:
+    sim = chiml_amd.FDTDField(deck2((n, n), "{prec}"))
+    log()
+    sim.step(k)
+    out.append(kernels(log()))
+for n, k, _ in {GRAPH[prec]}:
+    sim = chiml_amd.FDTDField(deck2((n, n), "{prec}"))
+    sim.set_graph(k)
+    log()
+    sim.step(k)
+    sim.step(k)
+    lines = log()
+    assert [line[0] for line in lines].count("graph") == 2
+    out.append(kernels([line for line in lines if line[0] == "capture"]))
+print(json.dumps(out))
+""")
+    for (n, k, tiles), names in zip(SHORT[prec], got):
+        assert names == (["k_tile2"] if tiles else ["k_h2v", "k_e2v"] * k), (n, k)
+    for (n, k, tiles), names in zip(GRAPH[prec], got[len(SHORT[prec]):]):
+        assert names == (["k_tile2"] * 2 if tiles else ["k_h2v", "k_e2v"] * k), (n, k)
+
+
+def test_changing_graphs_of_a_tiled_deck(fake):
+    """Graphs of tiles and of sweeps in one run: each replay starts on the
+    buffers it was captured on, and a graph of sweeps on its counter slot."""
+    lines = run(fake, """
+sim = chiml_amd.FDTDField(deck2((430, 430), "fp32"))
+log()
+sim.set_graph(2)    # sweeps
+sim.step(5)         # two replays and a step
+sim.step(4)         # a step (the replays start on the other counter slot), a replay and a step
+sim.set_graph(16)   # tiles
+sim.step(19)        # a replay, then three steps to the other buffers
+sim.step(16)
+print(json.dumps([line[:2] for line in log() if "k_set_step" not in line[1]]))
+""")
+    seen = [(a, b.split("k_", 1)[1].split("I", 1)[0] if "k_" in b else b) for a, b in lines]
+    sweep, captured = [("launch", "h2v"), ("launch", "e2v")], [("capture", "h2v"), ("capture", "e2v")]
+    tile = [("capture", "tile2")] * 2
+    assert seen == (captured * 2 + [("graph", "1")] * 2 + sweep + sweep + [("graph", "1")] + sweep
+                    + tile + [("graph", "2"), ("launch", "tile2")] + tile + [("graph", "3")])

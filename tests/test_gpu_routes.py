@@ -59,3 +59,26 @@ def test_live_decks_of_different_pole_counts(prec):
         _same(_results(alone), _results(sim), p)
         alone.close()
         sim.close()
+
+
+@pytest.mark.parametrize("prec,n", [("fp32", (836, 828)), ("fp32", (831, 829)), ("fp64", (412, 404)), ("fp64", (407, 405))])
+def test_results_do_not_depend_on_the_calls(prec, n):
+    """Above the sizes at which one or two steps go through the sweeps: whole
+    runs, single steps between tiles, and graphs of either kind."""
+    deck = _deck2(n, prec, poles=2, pml=7, steps=60)
+    whole = chiml_amd.FDTDField(deck)
+    whole.step(53)
+    ref = _results(whole)
+    whole.close()
+    runs = {"pieces": [(0, (1, 1, 2, 1, 3, 1, 8, 1, 2, 9, 1, 1, 22))],
+            "graphs": [(2, (1, 2, 4, 3)), (4, (4, 1, 4, 2)), (8, (8, 1, 8)), (2, (2, 1, 2)), (0, (1, 7, 2))],
+            "graph4": [(4, (53,))]}
+    for label, plan in runs.items():
+        sim = chiml_amd.FDTDField(deck)
+        for graph, chunks in plan:
+            sim.set_graph(graph)
+            for k in chunks:
+                sim.step(k)
+        assert sum(sum(c) for _, c in plan) == 53
+        _same(ref, _results(sim), label)
+        sim.close()
