@@ -111,7 +111,6 @@ struct StepArgs {
     int px;  // cells per stored x row: nx, or nx rounded up to whole W-cell groups (the added cells stay zero)
     T inv_d[3];
     int Tp[3];
-    int fma_curl;  // 2D sweeps: curl_of's FMA form
     const uint8_t* mat_e[3];
     const T* ce[3];
     const T* inveps[3];
@@ -1881,7 +1880,7 @@ __global__ void __launch_bounds__(256) k_h2v(StepArgs<T> a) {
 // DET: the deck's point detectors (single-cell, Ez / Hx / Hy) are sampled
 // here, by the thread that owns each detector cell, at the advanced step:
 // no separate sample launch (2D decks without flux boxes and with few points).
-template <typename T, int W, bool SRC, bool DET>
+template <typename T, int W, bool SRC, bool DET, bool FMA>
 __device__ __forceinline__ void e2v_sweep(const StepArgs<T>& a, const SampleArgs<T>& sa, const MatLds<T> (*mt)[CHIML_MAX_MAT], int bx, int nb) {
     const int ny = a.ny, px = a.px, gx = px / W;
     const unsigned t = static_cast<unsigned>(xcd_block(bx, nb)) * blockDim.x + threadIdx.x;
@@ -1904,8 +1903,8 @@ __device__ __forceinline__ void e2v_sweep(const StepArgs<T>& a, const SampleArgs
     pml_group<T, W>(a.pml[2], 0, x0, x0, y, 0, px, ny, d1, a.inv_d[0], all, t1);
     pml_group<T, W>(a.pml[2], 1, y, x0, y, 0, px, ny, d2, a.inv_d[1], all, t2);
     T acc[W];
-    const unsigned plain = a.fma_curl && y >= a.Tp[1] && y < ny - a.Tp[1] ? cells_inside<W>(x0, a.nx, a.Tp[0]) : 0u;
-    curl_of<T, W, true>(t1, t2, d2, a.inv_d[1], plain, acc);
+    const unsigned plain = FMA && y >= a.Tp[1] && y < ny - a.Tp[1] ? cells_inside<W>(x0, a.nx, a.Tp[0]) : 0u;
+    curl_of<T, W, FMA>(t1, t2, d2, a.inv_d[1], plain, acc);
     const Pk<T, W> ez = e_finish_group<T, W>(a, mt, 2, i, x0, y, 0, all, acc, src, step);
     if (DET) {
         const int st = step_now(a.step, a.stepv) + 1;
@@ -1919,12 +1918,12 @@ __device__ __forceinline__ void e2v_sweep(const StepArgs<T>& a, const SampleArgs
     }
 }
 
-template <typename T, int W, bool SRC, bool DET>
+template <typename T, int W, bool SRC, bool DET, bool FMA>
 __global__ void __launch_bounds__(256) k_e2v(StepArgs<T> a, SampleArgs<T> sa, int nm2) {
     __shared__ MatLds<T> mt[3][CHIML_MAX_MAT];
     const int nm[3] = {0, 0, nm2};
     load_mat(a, mt, nm);
-    e2v_sweep<T, W, SRC, DET>(a, sa, mt, blockIdx.x, gridDim.x);
+    e2v_sweep<T, W, SRC, DET, FMA>(a, sa, mt, blockIdx.x, gridDim.x);
 }
 
 // --------------------------------------------- 2D: several steps a launch ----
@@ -3173,7 +3172,8 @@ __global__ void __launch_bounds__(256) k_be2v(const BatchSlot<T>* __restrict__ s
     if (bx >= q.nblk[kPhE]) return;
     const int nm[3] = {0, 0, q.nm[2]};
     load_mat(q.a, mt, nm);
-    e2v_sweep<T, W, true, false>(q.a, q.s, mt, bx, q.nblk[kPhE]);
+    if (q.fma) e2v_sweep<T, W, true, false, true>(q.a, q.s, mt, bx, q.nblk[kPhE]);
+    else e2v_sweep<T, W, true, false, false>(q.a, q.s, mt, bx, q.nblk[kPhE]);
 }
 
 template <typename T, int W, bool NT>
@@ -3612,7 +3612,6 @@ void build(chiml_dev* c, const chiml_problem_t* p, StepArgs<T>& a, SampleArgs<T>
         c->rows = gl.rows;
         c->cellwise = gl.cellwise;
         c->fma_curl = nx % gl.W != 0 || p->pml_T[0] % gl.W != 0;
-        a.fma_curl = c->fma_curl ? 1 : 0;
     }
     const int px = c->px, rw = c->vec ? static_cast<int>(16 / sizeof(T)) : 1;
     a.px = px;
@@ -4170,13 +4169,12 @@ void launch_fields(chiml_dev* c, StepArgs<T>& a) {
         {
             Timed t(c, "update_e");
             const SampleArgs<T>& sa = sample_args<T>(c);
-            if (c->fuse_sample) {
-                if (c->has_src) hipLaunchKernelGGL((k_e2v<T, W, true, true>), g, blk, 0, c->stream, a, sa, c->nmat[2]);
-                else hipLaunchKernelGGL((k_e2v<T, W, false, true>), g, blk, 0, c->stream, a, sa, c->nmat[2]);
-            } else {
-                if (c->has_src) hipLaunchKernelGGL((k_e2v<T, W, true, false>), g, blk, 0, c->stream, a, sa, c->nmat[2]);
-                else hipLaunchKernelGGL((k_e2v<T, W, false, false>), g, blk, 0, c->stream, a, sa, c->nmat[2]);
-            }
+            pick2(c->has_src, c->fuse_sample, [&](auto S, auto D) {
+                if (c->fma_curl)
+                    hipLaunchKernelGGL((k_e2v<T, W, decltype(S)::value, decltype(D)::value, true>), g, blk, 0, c->stream, a, sa, c->nmat[2]);
+                else
+                    hipLaunchKernelGGL((k_e2v<T, W, decltype(S)::value, decltype(D)::value, false>), g, blk, 0, c->stream, a, sa, c->nmat[2]);
+            });
         }
         return;
     }
@@ -4642,6 +4640,7 @@ BatchSlot<T> make_slot(chiml_dev* c, int p) {
     q.s.step = ctr + (1 - p);
     q.s.stepv = -1;
     for (int k = 0; k < 3; ++k) q.nm[k] = c->nmat[k];
+    q.fma = c->fma_curl ? 1 : 0;
     if (c->dim == 2) {
         const long long ng = static_cast<long long>(c->px / W) * c->ny;
         q.nblk[kPhH] = q.nblk[kPhE] = static_cast<int>((ng + 255) / 256);
@@ -4650,7 +4649,6 @@ BatchSlot<T> make_slot(chiml_dev* c, int p) {
         const int nyb = b.y1 - b.y0, by = b.by > 0 ? b.by : nyb;
         const long long ni = static_cast<long long>((b.x1 - b.x0) / W) * by * (b.z1 - b.z0) * ((nyb + by - 1) / by);
         const long long ns = static_cast<long long>(c->slab.nA) + c->slab.nB + c->slab.nC;
-        q.fma = c->fma_curl ? 1 : 0;
         q.b = b;
         q.m = c->slab;
         q.nib = static_cast<int>((ni + 255) / 256);

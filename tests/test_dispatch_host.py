@@ -187,3 +187,21 @@ print(json.dumps([line[:2] for line in log() if "k_set_step" not in line[1]]))
     tile = [("capture", "tile2")] * 2
     assert seen == (captured * 2 + [("graph", "1")] * 2 + sweep + sweep + [("graph", "1")] + sweep
                     + tile + [("graph", "2"), ("launch", "tile2")] + tile + [("graph", "3")])
+
+
+@pytest.mark.parametrize("prec,w", [("fp32", 4), ("fp64", 2)])
+def test_2d_sweeps_fuse_products_on_unaligned_grids_only(fake, prec, w):
+    """The E sweep's fused form (rows or x CPML of no whole groups) is an
+    instantiation of its own: on the others it cost registers and a wave."""
+    names = run(fake, f"""
+out = []
+for n, pml in (((1024, 900), 8), ((1025, 900), 8), ((1024, 900), 9)):
+    sim = chiml_amd.FDTDField(deck2(n, "{prec}", pml=pml, flux=True))
+    log()
+    sim.step(1)
+    out.append([line[1] for line in log() if "k_e2v" in line[1]])
+print(json.dumps(out))
+""")
+    kind = "d" if prec == "fp64" else "f"
+    want = [f"k_e2vI{kind}Li{w}ELb1ELb0ELb{fma}E" for fma in (0, 1, 1)]
+    assert all(len(n) == 1 and k in n[0] for n, k in zip(names, want)), names
