@@ -3298,7 +3298,7 @@ struct chiml_dev {
     bool rows = false;   // split: whole-row interior, one launch per field
     double step_bytes = 0;     // fields and emitter state
     bool stream_hint = false;  // split: once-touched words go past the caches (streams_past_caches)
-    bool cellwise = false;  // split, but stepped alone with one thread per cell (GridLayout::cellwise)
+    bool cellwise = false;  // stepped alone with one thread per cell (GridLayout::cellwise)
     bool fma_curl = false;  // rows or x CPML no whole groups: curls as the per-cell kernels round them (curl_of)
     bool fused = false;  // 3D: one fused H + E launch per step on ping-pong buffers
     FuseMap fmap{};
@@ -3610,7 +3610,7 @@ void build(chiml_dev* c, const chiml_problem_t* p, StepArgs<T>& a, SampleArgs<T>
         c->px = gl.px;
         c->split = gl.split;
         c->rows = gl.rows;
-        c->cellwise = gl.cellwise;
+        c->cellwise = gl.cellwise && (nz > 1 || p->nsrc > 0);  // 2D groups without a search for sources keep up
         c->fma_curl = nx % gl.W != 0 || p->pml_T[0] % gl.W != 0;
     }
     const int px = c->px, rw = c->vec ? static_cast<int>(16 / sizeof(T)) : 1;
@@ -4154,7 +4154,7 @@ void launch_fields(chiml_dev* c, StepArgs<T>& a) {
         }
         return;
     }
-    if (DIM == 2 && c->vec2d) {
+    if (DIM == 2 && c->vec2d && !c->cellwise) {
         constexpr int W = 16 / sizeof(T);
         const long long ng = static_cast<long long>(c->px / W) * c->ny;
         const dim3 g(static_cast<unsigned>((ng + 255) / 256)), blk(256);
@@ -4977,7 +4977,7 @@ int chiml_dev_create(const chiml_problem_t* p, chiml_dev_t** out) {
                 const int cu = p->det_comp[2 * t];
                 single = cu == p->det_comp[2 * t + 1] && p->det_cell[2 * t] == p->det_cell[2 * t + 1] && cu >= 2 && cu <= 4;
             }
-            c->fuse_sample = c->vec2d && single;
+            c->fuse_sample = c->vec2d && !c->cellwise && single;
             if (c->prec == 32) enable_tiles<float>(c.get(), p, c->a32, c->s32);
             else enable_tiles<double>(c.get(), p, c->a64, c->s64);
         }

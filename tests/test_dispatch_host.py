@@ -134,10 +134,10 @@ print(json.dumps(out))
 
 
 # n, steps of one call, tiles? -- both sides of each line of tile_pays
-SHORT = {"fp32": [(390, 1, True), (410, 1, False), (410, 2, True), (1990, 2, True), (2010, 2, False), (2010, 3, True)],
-         "fp64": [(390, 1, True), (410, 1, False), (410, 2, True), (790, 2, True), (810, 2, False), (810, 3, True)]}
-GRAPH = {"fp32": [(390, 2, True), (410, 2, False), (990, 4, True), (1010, 4, False), (1010, 6, True)],
-         "fp64": [(390, 2, True), (410, 2, False), (610, 4, True), (630, 4, False), (630, 6, True)]}
+SHORT = {"fp32": [(388, 1, True), (412, 1, False), (412, 2, True), (1988, 2, True), (2012, 2, False), (2012, 3, True)],
+         "fp64": [(388, 1, True), (412, 1, False), (412, 2, True), (788, 2, True), (812, 2, False), (812, 3, True)]}
+GRAPH = {"fp32": [(388, 2, True), (412, 2, False), (988, 4, True), (1012, 4, False), (1012, 6, True)],
+         "fp64": [(388, 2, True), (412, 2, False), (608, 4, True), (632, 4, False), (632, 6, True)]}
 
 
 @pytest.mark.parametrize("prec", ["fp32", "fp64"])
@@ -172,7 +172,7 @@ def test_changing_graphs_of_a_tiled_deck(fake):
     """Graphs of tiles and of sweeps in one run: each replay starts on the
     buffers it was captured on, and a graph of sweeps on its counter slot."""
     lines = run(fake, """
-sim = chiml_amd.FDTDField(deck2((430, 430), "fp32"))
+sim = chiml_amd.FDTDField(deck2((432, 432), "fp32"))
 log()
 sim.set_graph(2)    # sweeps
 sim.step(5)         # two replays and a step
@@ -205,3 +205,22 @@ print(json.dumps(out))
     kind = "d" if prec == "fp64" else "f"
     want = [f"k_e2vI{kind}Li{w}ELb1ELb0ELb{fma}E" for fma in (0, 1, 1)]
     assert all(len(n) == 1 and k in n[0] for n, k in zip(names, want)), names
+
+
+def test_small_unaligned_2d_grids_step_per_cell(fake):
+    """FP32, below the line of GridLayout::cellwise and with a source; a batch
+    takes the groups all the same."""
+    got = run(fake, """
+out = []
+for n, prec in (((257, 255), "fp32"), ((701, 699), "fp32"), ((260, 255), "fp32"), ((257, 255), "fp64")):
+    a, b = (chiml_amd.FDTDField(deck2(n, prec, flux=True)) for _ in range(2))
+    log()
+    a.step(1)
+    alone = kernels(log())
+    chiml_amd.step_batch([a, b], 1)
+    out.append([alone, kernels(log())])
+print(json.dumps(out))
+""")
+    cells, groups = ["k_update_h", "k_update_e", "k_sample"], ["k_h2v", "k_e2v", "k_sample"]
+    assert [g[0] for g in got] == [cells, groups, groups, groups]
+    assert all(g[1][:3] == ["k_bh2v", "k_be2v", "k_bsample"] for g in got)

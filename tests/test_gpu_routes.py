@@ -61,7 +61,7 @@ def test_live_decks_of_different_pole_counts(prec):
         sim.close()
 
 
-@pytest.mark.parametrize("prec,n", [("fp32", (836, 828)), ("fp32", (831, 829)), ("fp64", (412, 404)), ("fp64", (407, 405))])
+@pytest.mark.parametrize("prec,n", [("fp32", (836, 828)), ("fp32", (831, 829)), ("fp32", (431, 429)), ("fp64", (412, 404)), ("fp64", (407, 405))])
 def test_results_do_not_depend_on_the_calls(prec, n):
     """Above the sizes at which one or two steps go through the sweeps: whole
     runs, single steps between tiles, and graphs of either kind."""
@@ -81,4 +81,22 @@ def test_results_do_not_depend_on_the_calls(prec, n):
                 sim.step(k)
         assert sum(sum(c) for _, c in plan) == 53
         _same(ref, _results(sim), label)
+        sim.close()
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+@pytest.mark.parametrize("n", [(45, 41), (131, 70), (257, 255)])
+def test_batched_odd_flux_decks_equal_alone(n, prec):
+    """2D decks that no tile takes, of sizes that are no whole groups: alone in
+    one thread per cell (FP32) or in groups, batched in groups."""
+    mix = [_deck2(n, prec, poles=2, pml=7, flux=True), _deck2((n[0] + 1, n[1] + 2), prec, poles=1, flux=True),
+           _deck2((n[0] + 3, n[1]), prec, flux=True)]
+    sims = [chiml_amd.FDTDField(d) for d in mix]
+    for k in (1, 40, 7, 32):
+        chiml_amd.step_batch(sims, k)
+    for k, (deck, sim) in enumerate(zip(mix, sims)):
+        alone = chiml_amd.FDTDField(deck)
+        alone.step(80)
+        _same(_results(alone), _results(sim), k)
+        alone.close()
         sim.close()
