@@ -2592,8 +2592,11 @@ template <int N, int EB>
 __device__ __forceinline__ double2 den_deriv(double ih, const double2* H, const double2* X, int i, int j, const int* col, const double* val,
                                              int g0, int g1) {
     double2 s1 = make_double2(0.0, 0.0), s2 = s1;
-    // (three of the N terms in flight: all of them would cost half the waves)
-#pragma unroll 3
+    // Up to five terms are written out; of more, three are in flight at a time.
+    // 144,000 emitters, us a launch, in threes / written out: N = 4 packed
+    // 52.7/47.4, N = 5 full 134/124 (one lane per column: 123), N = 6 packed in
+    // fives 100 against 89, N = 8 packed 234 against 211.
+#pragma unroll (N <= 5 ? N : 3)
     for (int k = 0; k < N; ++k) {
         s1 = cadd(s1, cmul(H[(i + k * N) * EB], X[(k + j * N) * EB]));
         s2 = cadd(s2, cmul(X[(i + k * N) * EB], H[(k + j * N) * EB]));
