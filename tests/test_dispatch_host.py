@@ -224,3 +224,23 @@ print(json.dumps(out))
     cells, groups = ["k_update_h", "k_update_e", "k_sample"], ["k_h2v", "k_e2v", "k_sample"]
     assert [g[0] for g in got] == [cells, groups, groups, groups]
     assert all(g[1][:3] == ["k_bh2v", "k_be2v", "k_bsample"] for g in got)
+
+
+def test_padded_row_decks_take_the_kernels_they_are_for(fake):
+    """The decks that test_gpu_padded_rows.py compares with the oracle."""
+    sys.path.insert(0, ROOT)
+    from tests.route_decks import CASES
+    got = run(fake, """
+from tests.route_decks import CASES
+out = {}
+for name, (deck, _, _) in CASES.items():
+    sim = chiml_amd.FDTDField(deck)
+    log()
+    sim.step(1)
+    out[name] = [line[1] for line in log()]
+    sim.close()
+print(json.dumps(out))
+""")
+    for name, (_, _, kernels) in CASES.items():
+        for k in kernels:
+            assert any(k in line for line in got[name]), (name, k, got[name])
