@@ -2,7 +2,7 @@
 step them: rows or x CPML that are no whole groups (4 cells in FP32, 2 in
 FP64), above the sizes that step one thread per cell.  The kernels are checked
 on the CPU (test_dispatch_host.py), the results against the oracle
-(test_gpu_padded_rows.py)."""
+(test_gpu_padded_rows.py).  Also 2D decks that the tiles leave to the sweeps."""
 import json
 
 from chiml_amd import decks
@@ -98,6 +98,21 @@ def oblique(n, pml, prec, steps):
     return json.dumps(dk)
 
 
+def no_tiles(n, pml, prec, steps, points, sets):
+    """A 2D deck without a flux box that the tiles leave to the sweeps: points x
+    points detector cells in one tile, or so many metals of different poles."""
+    d = 0.05
+    dk = decks.empty_deck(n, d, steps, pml, precision=prec)
+    for k in range(sets):
+        pols = [dict(p, gamma=p["gamma"] * (1.0 + 0.1 * k)) for p in decks.gold_like_pols()[:1]]
+        dk["ObjectList"].append({"shape": "block", "material": "custom", "eps": 2.0, "pols": pols, "size": [1.6 * d, 9.6 * d, 0.0],
+                                 "loc": [(2 * k - sets) * d, 0.0, 0.0], "Basis_Set": []})
+    dk["SourceList"].append({"pol": "Ez", "size": [0.0] * 3, "loc": _point(n, d, (n[0] // 2 + 1, n[1] // 2 + 6, 0)), "PulseList": [_pulse()]})
+    dk["DetectorList"].append({"type": "Ez", "dtc_class": "cout", "fname": "d", "size": [(points - 1) * d, (points - 1) * d, 0.0],
+                               "loc": [decks._pos(17, n[0], d) + (points - 1) * d / 2.0, decks._pos(17, n[1], d) + (points - 1) * d / 2.0, 0.0]})
+    return json.dumps(dk)
+
+
 # name -> (deck, steps, kernels)
 CASES = {
     "metal_fp32": (metal((66, 60, 60), 7, "fp32", 40), 40, _h3("fp32")),
@@ -123,5 +138,9 @@ CASES = {
     "tfsf_2d_fp32": (tfsf((101, 94, 1), 7, "fp32", 90, (41, 39, 1), (0, 1, 0)), 90, _h2("fp32", src=0, det=1) + ["k_tfsf_stepIf"]),
     "tfsf_2d_fp64": (tfsf((101, 94, 1), 7, "fp64", 90, (41, 39, 1), (1, 2, 0)), 90, _h2("fp64", src=0, det=1) + ["k_tfsf_stepId"]),
     "oblique_2d_fp32": (oblique((101, 94, 1), 7, "fp32", 60), 60, _h2("fp32", src=0) + ["k_cell_srcIf"]),
+    "many_points_2d_fp64": (no_tiles((48, 44, 1), 4, "fp64", 60, 9, 1), 60, ["k_h2vIdLi2ELb1ELb0E", "k_e2vIdLi2ELb1ELb0ELb0E"]),
+    "many_points_2d_fp32": (no_tiles((48, 44, 1), 4, "fp32", 60, 9, 1), 60, ["k_h2vIfLi4ELb1ELb0E", "k_e2vIfLi4ELb1ELb0ELb0E"]),
+    "many_poles_2d_fp64": (no_tiles((48, 44, 1), 4, "fp64", 60, 1, 9), 60, ["k_h2vIdLi2ELb1ELb0E", "k_e2vIdLi2ELb1ELb1ELb0E"]),
+    "many_poles_2d_fp32": (no_tiles((48, 44, 1), 4, "fp32", 60, 1, 9), 60, ["k_h2vIfLi4ELb1ELb0E", "k_e2vIfLi4ELb1ELb1ELb0E"]),
     "oblique_2d_fp64": (oblique((101, 94, 1), 7, "fp64", 60), 60, _h2("fp64", src=0) + ["k_cell_srcId"]),
 }

@@ -8,6 +8,7 @@ import pytest
 
 import chiml_amd
 from chiml_amd import decks
+from tests.route_decks import emitters, metal
 
 pytestmark = pytest.mark.gpu
 
@@ -98,5 +99,28 @@ def test_batched_odd_flux_decks_equal_alone(n, prec):
         alone = chiml_amd.FDTDField(deck)
         alone.step(80)
         _same(_results(alone), _results(sim), k)
+        alone.close()
+        sim.close()
+
+
+def test_batched_unaligned_3d_decks_equal_alone():
+    """3D metals whose rows are no whole groups: FP32 ones in groups when
+    batched, alone in one thread per cell below the line and in groups above
+    it; FP64 ones step alone inside the call.  One aligned deck of each
+    precision and one with emitters share the launches."""
+    mix = [metal((33, 30, 31), 5, "fp32", 60), metal((66, 60, 60), 7, "fp32", 60), metal((33, 30, 31), 5, "fp64", 60),
+           metal((65, 62, 61), 5, "fp64", 60), metal((64, 60, 60), 8, "fp32", 60), metal((64, 60, 60), 8, "fp64", 60),
+           emitters((66, 60, 60), 7, "fp32", 60, (5, 7, 3), 4), emitters((613, 615, 1), 7, "fp32", 60, (9, 5, 1), 2),
+           emitters((91, 93, 1), 7, "fp64", 60, (9, 5, 1), 3)]
+    sims = [chiml_amd.FDTDField(d) for d in mix]
+    for k in (7, 13, 1, 20, 19):
+        chiml_amd.step_batch(sims, k)
+    for k, (deck, sim) in enumerate(zip(mix, sims)):
+        alone = chiml_amd.FDTDField(deck)
+        alone.step(60)
+        a, b = _results(alone), _results(sim)
+        _same(a, b, k)
+        for q, p in zip(alone.qeArr(), sim.qeArr()):
+            assert np.array_equal(q.population(0), p.population(0)), k
         alone.close()
         sim.close()
