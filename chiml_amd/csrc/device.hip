@@ -5230,12 +5230,13 @@ int chiml_dev_flux_plan(chiml_dev_t* c, int nface, const int* npt, const int* co
     if (nface < 1 || nface > kFluxFaces || !npt || !ids || !cw || !sw || !plan) return fail(c, CHIML_E_INVALID, "invalid argument");
     if (c->dgs.empty() || c->dgs[0].n == 0) return fail(c, CHIML_E_INVALID, "no flux samples");
     std::lock_guard<std::mutex> lk(g_capture_mu);
+    const size_t held = c->bufs.size(), footprint = c->footprint;
     try {
         chiml_dev::FluxPlan pl;
         FluxPlanDev& d = pl.dev;
         d.nface = nface;
         for (int f = 0; f < nface; ++f) {
-            if (npt[f] < 0) throw std::runtime_error("flux plan: point count");
+            if (npt[f] < 0) throw std::invalid_argument("flux plan: point count");
             d.npt[f] = npt[f];
             d.start[f + 1] = d.start[f] + (npt[f] + 255) / 256 * 256;
             for (int k = 0; k < 4; ++k) d.cw[f][k] = cw[4 * f + k];
@@ -5248,7 +5249,7 @@ int chiml_dev_flux_plan(chiml_dev_t* c, int nface, const int* npt, const int* co
                 hw[d.start[f] + p] = sw[f][p];
                 for (int k = 0; k < 16; ++k) {
                     const int id = ids[f][static_cast<size_t>(k) * npt[f] + p];
-                    if (id >= c->dgs[0].n) throw std::runtime_error("flux plan: sample index out of range");
+                    if (id >= c->dgs[0].n) throw std::invalid_argument("flux plan: sample index out of range");
                     hi[k * total + d.start[f] + p] = id;
                 }
             }
@@ -5258,7 +5259,12 @@ int chiml_dev_flux_plan(chiml_dev_t* c, int nface, const int* npt, const int* co
         pl.partial = reinterpret_cast<double2*>(c->zeros<double>(2 * static_cast<size_t>(std::max(pl.blocks, 1)) * c->dgs[0].nfreq));
         *plan = static_cast<int>(c->flux_plans.size());
         c->flux_plans.push_back(pl);
+    } catch (std::invalid_argument& e) {
+        return fail(c, CHIML_E_INVALID, e.what());
     } catch (std::exception& e) {
+        (void)hipGetLastError();
+        c->bufs.resize(held);
+        c->footprint = footprint;
         return fail(c, CHIML_E_HIP, e.what());
     }
     return CHIML_OK;

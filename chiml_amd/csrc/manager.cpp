@@ -2015,7 +2015,8 @@ static std::vector<double> simpson_weights(int n, double d) {
 }
 
 // The faces of box fi as tables for the device (fluxFields' averaging and
-// fluxFaces' integration), uploaded at the first read of its flux.
+// fluxFaces' integration), uploaded at the first read of its flux; -1 where
+// the device has no room for them.
 int FDTDField::fluxPlan(int fi) {
     FluxBox& fb = fluxes.at(fi);
     if (fb.plan >= 0) return fb.plan;
@@ -2071,9 +2072,9 @@ int FDTDField::fluxPlan(int fi) {
         pi[v] = ids[v].data();
         pw[v] = sw[v].data();
     }
-    if (chiml_dev_flux_plan(dev_, nface, npt.data(), pi.data(), cw.data(), pw.data(), &fb.plan) != CHIML_OK)
-        throw std::runtime_error(chiml_dev_last_error(dev_));
-    return fb.plan;
+    const int rc = chiml_dev_flux_plan(dev_, nface, npt.data(), pi.data(), cw.data(), pw.data(), &fb.plan);
+    if (rc == CHIML_E_INVALID) throw std::runtime_error(chiml_dev_last_error(dev_));
+    return rc == CHIML_OK ? fb.plan : -1;
 }
 
 // Per face and frequency: tempFlux = fluxConv_ * weight_ * simps2D(...).
@@ -2083,9 +2084,10 @@ std::vector<std::vector<cplx>> FDTDField::fluxFaces(int fi) {
     chiml_dev_steps_done(dev_, &steps);
     const double nt = steps / fb.timeInt + 1;
     std::vector<std::vector<cplx>> out;
-    if (fb.loaded.empty() && ndft > 0) {  // combined, multiplied and integrated on the device
+    const int plan = fb.loaded.empty() && ndft > 0 ? fluxPlan(fi) : -1;
+    if (plan >= 0) {  // combined, multiplied and integrated on the device
         std::vector<double> reim(2 * fb.faces.size() * nfreq);
-        if (chiml_dev_flux(dev_, fluxPlan(fi), nt, reim.data()) != CHIML_OK) throw std::runtime_error(chiml_dev_last_error(dev_));
+        if (chiml_dev_flux(dev_, plan, nt, reim.data()) != CHIML_OK) throw std::runtime_error(chiml_dev_last_error(dev_));
         for (size_t v = 0; v < fb.faces.size(); ++v) {
             std::vector<cplx>& fv = out.emplace_back(nfreq, 0.0);
             for (int k = 0; k < nfreq; ++k)

@@ -6,7 +6,9 @@
  *
  * What a test reads and sets: fake_hip_log() (one line per call of interest),
  * fake_hip_clear(), fake_hip_fail_size(bytes): hipMalloc of exactly that many
- * bytes fails from its second call on.
+ * bytes fails from its second call on; fake_hip_refuse(n): the first n - 1
+ * calls of hipMalloc from here on succeed, the others fail (0: none fails).
+ * fake_hip_held(): bytes allocated and not freed.
  */
 #include <hip/hip_runtime_api.h>
 
@@ -23,7 +25,12 @@ std::map<const void*, std::string>& names() {
     return *m;
 }
 size_t g_fail_size = 0;
-int g_fail_seen = 0;
+int g_fail_seen = 0, g_refuse = 0;
+size_t g_held = 0;
+std::map<void*, size_t>& blocks() {
+    static auto* m = new std::map<void*, size_t>;
+    return *m;
+}
 bool g_capturing = false;
 struct Call {
     dim3 g, b;
@@ -40,6 +47,8 @@ void fake_hip_fail_size(size_t bytes) {
     g_fail_size = bytes;
     g_fail_seen = 0;
 }
+void fake_hip_refuse(int n) { g_refuse = n; }
+size_t fake_hip_held() { return g_held; }
 
 void** __hipRegisterFatBinary(const void*) {
     static void* h = nullptr;
@@ -84,11 +93,21 @@ hipError_t hipMalloc(void** p, size_t n) {
         put("refused " + std::to_string(n));
         return hipErrorOutOfMemory;
     }
+    if (g_refuse == 1) return hipErrorOutOfMemory;
+    if (g_refuse > 1) --g_refuse;
     *p = std::calloc(n ? n : 1, 1);
-    return *p ? hipSuccess : hipErrorOutOfMemory;
+    if (!*p) return hipErrorOutOfMemory;
+    blocks()[*p] = n;
+    g_held += n;
+    return hipSuccess;
 }
 hipError_t hipMallocAsync(void** p, size_t n, hipStream_t) { return hipMalloc(p, n); }
 hipError_t hipFree(void* p) {
+    auto it = blocks().find(p);
+    if (it != blocks().end()) {
+        g_held -= it->second;
+        blocks().erase(it);
+    }
     std::free(p);
     return hipSuccess;
 }

@@ -14,10 +14,11 @@ import pytest
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 PRELUDE = """
-import ctypes, json, sys
+import ctypes, json, re, sys
 fake = ctypes.CDLL({fake!r}, mode=ctypes.RTLD_GLOBAL)
 fake.fake_hip_log.restype = ctypes.c_char_p
 fake.fake_hip_fail_size.argtypes = [ctypes.c_size_t]
+fake.fake_hip_held.restype = ctypes.c_size_t
 import chiml_amd
 from chiml_amd import decks
 
@@ -39,7 +40,7 @@ def log():
 
 def kernels(lines):
     # the launched kernels by their short names, the step counter's left out
-    names = ["k_" + line[1].split("k_", 1)[1].split("I", 1)[0] for line in lines if line[0] in ("launch", "capture")]
+    names = [re.search("k_[a-z0-9_]+", line[1]).group() for line in lines if line[0] in ("launch", "capture")]
     return [k for k in names if not k.startswith("k_set_step")]
 """
 
@@ -244,3 +245,23 @@ print(json.dumps(out))
     for name, (_, _, kernels) in CASES.items():
         for k in kernels:
             assert any(k in line for line in got[name]), (name, k, got[name])
+
+
+def test_no_memory_for_the_flux_tables(fake):
+    """A flux spectrum is read on the host where the card has no room for the
+    faces' tables; what was taken of them is given back."""
+    got = run(fake, """
+import numpy as np
+sim = chiml_amd.FDTDField(deck2((68, 61), "fp64", flux=True))
+sim.step(4)
+held, out = fake.fake_hip_held(), []
+for n in (1, 2, 3):
+    fake.fake_hip_refuse(n)
+    f = sim.fluxArr()[0].getFlux()
+    fake.fake_hip_refuse(0)
+    out.append([f.size, fake.fake_hip_held() == held, [k for k in kernels(log()) if "flux" in k]])
+f = sim.fluxArr()[0].getFlux()
+out.append([f.size, fake.fake_hip_held() > held, [k for k in kernels(log()) if "flux" in k]])
+print(json.dumps(out))
+""")
+    assert got == [[3, True, []]] * 3 + [[3, True, ["k_flux_faces"]]]
