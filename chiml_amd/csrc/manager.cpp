@@ -1982,16 +1982,8 @@ std::vector<std::array<std::vector<cplx>, 4>> FDTDField::fluxFields(int fi) {
 
 // simpson() as weights: the result for f is sum_i w[i] f[i].
 static std::vector<double> simpson_weights(int n, double d) {
+    if (n == 1) return {d};
     std::vector<double> w(n, 0.0);
-    std::vector<cplx> unit(n, cplx(0.0, 0.0));
-    if (n < 8) {
-        for (int i = 0; i < n; ++i) {
-            unit[i] = 1.0;
-            w[i] = simpson(unit.data(), n, d).real();
-            unit[i] = 0.0;
-        }
-        return w;
-    }
     if (n % 2 == 0) {
         for (int i = 0; i < (n - 2) / 2; i++) {
             w[2 * i] += d / 6.0;
