@@ -452,8 +452,8 @@ __global__ void __launch_bounds__(256) k_update_e(StepArgs<T> a) {
 // ~6.3 TB/s with 16-byte lanes.  Rows are stored in whole groups and the psi
 // regions widened to whole groups (grid_layout.hpp; identity coefficients on
 // the added positions), so that the W cells of a group share their CPML
-// membership on every axis.  101x93x87 FP32 with a 10-cell CPML: one thread
-// per cell 65 us a step, groups 49.
+// membership on every axis.  101x93x87 FP32 with a 10-cell CPML and a
+// three-pole metal: one thread per cell 48.6 us a step, groups 27.1.
 // The interior walk leaves out the y and z CPML terms at compile time, and
 // blocks and groups are numbered in 32 bits: 256^3 FP32 with a 16-cell CPML
 // 0.302 -> 0.284 ms a step (the 64-bit divisions of the numbering and the
@@ -2634,7 +2634,7 @@ __device__ __forceinline__ double2 den_deriv(double ih, const double2* H, const 
 // to cover its phases (load, two derivatives, store), so a lane holds one entry
 // (78 VGPRs, 6 waves per SIMD).  With one lane per column (236 VGPRs, 2 waves)
 // the same launch took 407 us, now 231 (3.4 TB/s); the copy rate would allow
-// 155.  4 waves per SIMD measured 275, blocks of 16 emitters 330.  32,768
+// 124.  4 waves per SIMD measured 275, blocks of 16 emitters 330.  32,768
 // two-level emitters: 10.1 -> 6.8 us.
 constexpr int kMlGamLds = 256;  // Lindblad entries staged in LDS (more are read from global memory)
 
@@ -2849,7 +2849,7 @@ __global__ void __launch_bounds__(kPopThreads) k_finish_sample(QeDev q, const do
     else sample_at<T>(s, (blockIdx.x - q.npop) * blockDim.x + threadIdx.x);
 }
 
-// Population detectors past the four the density kernel sums in registers:
+// Population detectors past the four the density kernel sums in LDS:
 // on recording steps, block (b, jj - j0) sums entry (ri, cj) of the stored
 // density matrices (the conjugate of (cj, ri) below the diagonal when
 // packed) over a strided subset of the member/emitter columns, then a tree in

@@ -212,7 +212,7 @@ typedef struct {
     const chiml_qe_t* qe;
     const double* eps_node;  /* (nx*ny*nz) eps at the nodes, used by the emitter back-coupling */
 
-    /* DFT groups 1..ndftg (group 0 is ndft / dft_* above), at most 7. */
+    /* DFT groups 1..ndftg (group 0 is ndft / dft_* above), at most 15. */
     int ndftg;
     const chiml_dft_group_t* dftg;
 
@@ -299,7 +299,8 @@ void chiml_dev_destroy(chiml_dev_t* ctx);
  * them, through a device-side table of per-simulation parameter blocks that
  * the call allocates (stream-ordered) and frees.  Emitter and DFT launches
  * stay per simulation, on the batch's stream; contexts of other classes step
- * alone on their own streams.  The batch runs on the stream of its first
+ * alone on their own streams (TFSF surfaces, per-cell sources, unaligned FP64
+ * 3D grids, and 2D decks that take several steps per launch).  The batch runs on the stream of its first
  * context, joined by events with the others' streams before and after, so the
  * call is asynchronous like chiml_dev_step.  Every simulation's arithmetic
  * is that of chiml_dev_step, so results are identical bit for bit.  A context
