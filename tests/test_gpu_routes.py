@@ -73,7 +73,9 @@ def test_results_do_not_depend_on_the_calls(prec, n):
     whole.close()
     runs = {"pieces": [(0, (1, 1, 2, 1, 3, 1, 8, 1, 2, 9, 1, 1, 22))],
             "graphs": [(2, (1, 2, 4, 3)), (4, (4, 1, 4, 2)), (8, (8, 1, 8)), (2, (2, 1, 2)), (0, (1, 7, 2))],
-            "graph4": [(4, (53,))]}
+            "graph4": [(4, (53,))],
+            # graphs of sweeps captured and replayed on either buffer set
+            "flipped": [(0, (3,)), (2, (4, 3)), (0, (7,)), (2, (6, 1)), (8, (8, 8)), (2, (2,)), (0, (3, 8))]}
     for label, plan in runs.items():
         sim = chiml_amd.FDTDField(deck)
         for graph, chunks in plan:
