@@ -1945,9 +1945,11 @@ __global__ void __launch_bounds__(256) k_e2v(StepArgs<T> a, SampleArgs<T> sa, in
 // in halos), large ones large tiles (1.8x).  A block has 8-16 waves of few
 // rows: the same 32 x 32 tile with 4 rows a thread (1 wave per SIMD) measured
 // 2.6 us a step, with 2 rows 1.85, with 1 row 1.7 but slower with poles;
-// 16-step launches (64 x 48 tiles) 2.9.  Measured with a read of the fields
-// per pass: 256^2 FP64 8.1 -> 1.9 us a step, 301x243 FP32 with a metal
-// cylinder 12.5 -> 2.0, 512^2 FP32 11.9 -> 4.2, 1024^2 FP32 19.9 -> 10.7.
+// 16-step launches (64 x 48 tiles) 2.9.  us a step in long runs, two sweeps /
+// tiles: 256^2 FP64 8.1/1.75, 301x243 FP32 with a metal cylinder 12.9/1.9, FP32
+// 512^2 9.8/2.5, 1024^2 16.6/4.9, 2048^2 33.5/15.8, 6144^2 253/120; FP64 2048^2
+// 58.7/32.4, 6144^2 485/279: no size was found from which the sweeps are faster
+// (one or two steps at a time they are: tile_pays).
 constexpr int kTileSteps = 8;
 constexpr int kTileDet = 64;  // detector points of one tile at most
 constexpr int kTileSets = 8;  // pole sets at most
